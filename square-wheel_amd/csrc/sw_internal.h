@@ -317,11 +317,25 @@ struct WaterTexLaunch
 };
 void launch_water_texture(hipStream_t st, const float* field, uint32_t log2w, uint32_t log2h, const WaterTexLaunch& w, sw_texel* texels);
 // fire (generative_texture_effect_fire.rs): one step (update into heat_old, then the points) and the
-// palette texture + lite mips (dst levels given by texel offsets)
+// palette texture + lite mips (dst levels given by texel offsets). Up to FIRE_ARG_POINTS points travel
+// in the kernel's arguments, packed as address (area below 2^22) and heat; points_dev is their device
+// copy when there are more.
+const uint32_t FIRE_ARG_POINTS_SMALL = 64u, FIRE_ARG_POINTS = 512u;
+const uint32_t FIRE_POINT_ADDRESS = (1u << 22) - 1u, FIRE_POINT_HEAT_SHIFT = 22u;
+template <uint32_t N>
+struct FirePoints
+{
+	uint32_t n;
+	uint32_t p[N];
+};
+struct FirePalette
+{
+	uint32_t color[256];
+};
 void launch_fire_step(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h, uint32_t attenuation_i,
-	bool slow, const sw_heat_point* points_dev, uint32_t num_points);
+	bool slow, const sw_heat_point* points, uint32_t num_points, const sw_heat_point* points_dev);
 void launch_fire_texture(hipStream_t st, const uint8_t* heat, uint32_t log2w, uint32_t log2h, const uint64_t dst_offset[5],
-	const uint32_t* palette_dev, uint32_t* lite);
+	const uint32_t palette[256], uint32_t* lite);
 void launch_skybox_side(hipStream_t st, uint32_t color_bits, const void* image, uint32_t image_w, uint32_t size, int32_t brightness,
 	void* dst);
 

@@ -1681,7 +1681,7 @@ int sw_fire_step(sw_ctx* ctx, uint8_t* heat_device, uint8_t* heat_old_device, ui
 	(void)hipSetDevice(ctx->device);
 	int r;
 	const sw_heat_point* pts_dev = nullptr;
-	if(num_points)
+	if(num_points > swk::FIRE_ARG_POINTS) // else the points travel in the kernel's arguments
 	{
 		const size_t bytes = sizeof(sw_heat_point) * num_points;
 		char* staging = nullptr;
@@ -1694,7 +1694,7 @@ int sw_fire_step(sw_ctx* ctx, uint8_t* heat_device, uint8_t* heat_old_device, ui
 	}
 	{
 		StageTimer t(ctx, STAGE_TEXTURES);
-		swk::launch_fire_step(ctx->stream, heat_device, heat_old_device, log2_width, log2_height, attenuation_i, slow != 0, pts_dev, num_points);
+		swk::launch_fire_step(ctx->stream, heat_device, heat_old_device, log2_width, log2_height, attenuation_i, slow != 0, points, num_points, pts_dev);
 	}
 	return hip_check(ctx, hipGetLastError(), "fire step launch");
 }
@@ -1720,17 +1720,9 @@ int sw_fire_make_texture(sw_ctx* ctx, sw_map* map, const uint8_t* heat_device, u
 		off[mip] = l.offset;
 	}
 	(void)hipSetDevice(ctx->device);
-	int r;
-	char* staging = nullptr;
-	if((r = ensure(ctx, ctx->fire_args, 1024)) || (r = stage_begin(ctx, 1024, &staging)))
-		return r;
-	std::memcpy(staging, palette, 1024);
-	if((r = stage_copy(ctx, ctx->fire_args.p, 1024)))
-		return r;
 	{
 		StageTimer t(ctx, STAGE_TEXTURES);
-		swk::launch_fire_texture(ctx->stream, heat_device, log2_width, log2_height, off, static_cast<const uint32_t*>(ctx->fire_args.p),
-			static_cast<uint32_t*>(map->lite.p));
+		swk::launch_fire_texture(ctx->stream, heat_device, log2_width, log2_height, off, palette, static_cast<uint32_t*>(map->lite.p));
 	}
 	return hip_check(ctx, hipGetLastError(), "fire texture launch");
 }

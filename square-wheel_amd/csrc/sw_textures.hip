@@ -540,95 +540,194 @@ __global__ __launch_bounds__(256) void k_water_texture_tiles(const float* field,
 	}
 }
 
-// The palette texture (generate_emissive_texture_based_on_heat_map, :470-486) of one 16 x 16 tile and
-// the tile's texels of lite mips 1 .. 4 (build_texture_lite_mip, textures.rs:385-415).
-__global__ __launch_bounds__(256) void k_fire_texture_tiles(const uint8_t* heat, uint32_t log2w, const uint32_t* palette, uint32_t* lite,
-	uint64_t o0, uint64_t o1, uint64_t o2, uint64_t o3, uint64_t o4)
+// The average of the lane's 2 x 2 square of texels, the square's lanes step apart in Morton order:
+// its first lane, then x + 1 (step), y + 1 (2 * step) and both.
+SW_DEV uint32_t quad_average(uint32_t v, uint32_t lane, uint32_t step)
 {
-	__shared__ uint32_t tile[16 * 16];
-	const uint64_t off[5] = {o0, o1, o2, o3, o4};
-	const uint32_t tx = blockIdx.x & ((1u << (log2w - 4)) - 1u), ty = blockIdx.x >> (log2w - 4);
-	const uint32_t lx = threadIdx.x & 15u, ly = threadIdx.x >> 4;
-	const uint32_t x = tx * 16u + lx, y = ty * 16u + ly;
-	const uint32_t c = palette[heat[x + (y << log2w)]];
-	tile[threadIdx.x] = c;
-	lite[off[0] + x + (y << log2w)] = c;
+	const uint32_t first = lane & ~(4u * step - 1u); // the square's (0, 0) lane
+	return average_4(uint32_t(__shfl(int(v), int(first))), uint32_t(__shfl(int(v), int(first + 2u * step))),
+		uint32_t(__shfl(int(v), int(first + step))), uint32_t(__shfl(int(v), int(first + 3u * step))));
+}
+
+// The palette texture (generate_emissive_texture_based_on_heat_map, :470-486) and its lite mips 1 .. 4
+// (build_texture_lite_mip, textures.rs:385-415), a 16 x 16 tile per wave: a lane takes a 2 x 2 square of
+// mip 0 and its mip 1 texel, the lanes lie in Morton order, so mips 2 .. 4 come from lane exchanges
+// (no barriers). Bound by launch and memory latency: the palette travels in the kernel's arguments
+// (no copy ahead of the launch), is staged in LDS once per block.
+__global__ __launch_bounds__(256) void k_fire_texture(const uint8_t* heat, uint32_t log2w, uint32_t tiles, swk::FirePalette palette,
+	uint32_t* lite, uint64_t o0, uint64_t o1, uint64_t o2, uint64_t o3, uint64_t o4)
+{
+	__shared__ uint32_t pal[256];
+	pal[threadIdx.x] = palette.color[threadIdx.x];
 	__syncthreads();
-	for(uint32_t mip = 1, n = 8; mip <= 4; ++mip, n >>= 1)
-	{
-		uint32_t v = 0;
-		const bool active = lx < n && ly < n;
-		if(active)
-			v = average_4(tile[(2u * ly) * 16u + 2u * lx], tile[(2u * ly + 1u) * 16u + 2u * lx], tile[(2u * ly) * 16u + 2u * lx + 1u],
-				tile[(2u * ly + 1u) * 16u + 2u * lx + 1u]);
-		__syncthreads();
-		if(active)
-		{
-			tile[ly * 16u + lx] = v;
-			lite[off[mip] + (tx * n + lx) + ((ty * n + ly) << (log2w - mip))] = v;
-		}
-		__syncthreads();
-	}
+	const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+	if(tile >= tiles)
+		return; // uniform over the wave
+	const uint32_t tx = tile & ((1u << (log2w - 4)) - 1u), ty = tile >> (log2w - 4);
+	const uint32_t qx = (lane & 1u) | ((lane >> 1) & 2u) | ((lane >> 2) & 4u), qy = ((lane >> 1) & 1u) | ((lane >> 2) & 2u) | ((lane >> 3) & 4u);
+	const uint32_t x = tx * 16u + qx * 2u, y = ty * 16u + qy * 2u;
+	const uint32_t i0 = x + (y << log2w), i1 = i0 + (1u << log2w);
+	const uint32_t c00 = pal[heat[i0]], c10 = pal[heat[i0 + 1]], c01 = pal[heat[i1]], c11 = pal[heat[i1 + 1]];
+	lite[o0 + i0] = c00;
+	lite[o0 + i0 + 1] = c10;
+	lite[o0 + i1] = c01;
+	lite[o0 + i1 + 1] = c11;
+	uint32_t v = average_4(c00, c01, c10, c11);
+	lite[o1 + (tx * 8u + qx) + ((ty * 8u + qy) << (log2w - 1))] = v;
+	v = quad_average(v, lane, 1);
+	if((lane & 3u) == 0)
+		lite[o2 + (tx * 4u + (qx >> 1)) + ((ty * 4u + (qy >> 1)) << (log2w - 2))] = v;
+	v = quad_average(v, lane, 4);
+	if((lane & 15u) == 0)
+		lite[o3 + (tx * 2u + (qx >> 2)) + ((ty * 2u + (qy >> 2)) << (log2w - 3))] = v;
+	v = quad_average(v, lane, 16);
+	if(lane == 0)
+		lite[o4 + tx + (ty << (log2w - 4))] = v;
 }
 
 } // namespace
 
 namespace
 {
-// update_heat_map (:357-468), fast variant: row y < h - 2 from rows y + 1 (x - 1, x, x + 1, wrapped)
-// and y + 2; row h - 2 takes row h - 1 twice; the last row is cleared. All reads see the old map
-// (the reference walks rows downwards and reads only rows below), so one lane per element.
-__global__ __launch_bounds__(256) void k_fire_update_fast(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w, uint32_t log2h, uint32_t att)
+// update_heat_map (:357-468), fast variant, and the step's set_heat points: row y < h - 2 from rows
+// y + 1 (x - 1, x, x + 1, wrapped) and y + 2; row h - 2 takes row h - 1 twice; the last row is cleared.
+// All reads see the old map (the reference walks rows downwards and reads only rows below). A block
+// takes 1024 consecutive texels, four per thread; the points (packed as address and heat in the
+// kernel's arguments) then raise the block's texels in LDS by atomic maxima, so a step is one launch
+// with no copy ahead of it: bound by launch latency (a 64 x 64 map's step: 2.2 us of update, 9.4 us of
+// points and 2.7 us of copy as three operations, 3 us as one). WORDS: both buffers are 4-byte
+// aligned, texels move as words.
+template <uint32_t N, bool WORDS>
+__global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
 {
-	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	if(i >> (log2w + log2h))
-		return;
+	__shared__ __align__(16) uint32_t cells[1024];
 	const uint32_t w = 1u << log2w, h = 1u << log2h, mx = w - 1u;
+	const uint32_t b0 = blockIdx.x * 1024u, i = b0 + threadIdx.x * 4u;
+	const bool in = (i >> (log2w + log2h)) == 0;
+	uint32_t v[4] = {0, 0, 0, 0};
 	const uint32_t x = i & mx, y = i >> log2w;
-	if(y == h - 1u)
+	if(in && y != h - 1u)
 	{
-		dst[i] = 0;
-		return;
+		const uint32_t r1 = (y + 1u) << log2w, r2 = (y + 2u < h ? y + 2u : y + 1u) << log2w;
+		uint32_t a[6], c[4];
+		a[0] = src[r1 + ((x - 1u) & mx)];
+		a[5] = src[r1 + ((x + 4u) & mx)];
+		if(WORDS)
+		{
+			const uint32_t wa = *reinterpret_cast<const uint32_t*>(src + r1 + x), wc = *reinterpret_cast<const uint32_t*>(src + r2 + x);
+			for(uint32_t k = 0; k < 4; ++k)
+			{
+				a[k + 1] = (wa >> (8 * k)) & 0xFFu;
+				c[k] = (wc >> (8 * k)) & 0xFFu;
+			}
+		}
+		else
+			for(uint32_t k = 0; k < 4; ++k)
+			{
+				a[k + 1] = src[r1 + x + k];
+				c[k] = src[r2 + x + k];
+			}
+		for(uint32_t k = 0; k < 4; ++k)
+			v[k] = ((a[k] + a[k + 1] + a[k + 2] + c[k]) * att) >> 20;
 	}
-	const uint32_t r1 = (y + 1u) << log2w, r2 = (y + 2u < h ? y + 2u : y + 1u) << log2w;
-	const uint32_t sum = uint32_t(src[r1 + ((x - 1u) & mx)]) + src[r1 + x] + src[r1 + ((x + 1u) & mx)] + src[r2 + x];
-	dst[i] = uint8_t((sum * att) >> 20);
+	if(pts.n)
+	{
+		*reinterpret_cast<uint4*>(cells + threadIdx.x * 4u) = make_uint4(v[0], v[1], v[2], v[3]);
+		__syncthreads();
+		for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+		{
+			const uint32_t p = pts.p[k], a = (p & swk::FIRE_POINT_ADDRESS) - b0;
+			if(a < 1024u)
+				atomicMax(&cells[a], p >> swk::FIRE_POINT_HEAT_SHIFT);
+		}
+		__syncthreads();
+		const uint4 r = *reinterpret_cast<const uint4*>(cells + threadIdx.x * 4u);
+		v[0] = r.x;
+		v[1] = r.y;
+		v[2] = r.z;
+		v[3] = r.w;
+	}
+	if(!in)
+		return;
+	if(WORDS)
+		*reinterpret_cast<uint32_t*>(dst + i) = v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24);
+	else
+		for(uint32_t k = 0; k < 4; ++k)
+			dst[i + k] = uint8_t(v[k]);
 }
 
-// the slow variant: each row is a chain (the left neighbour is the value just written; the last
-// texel's right neighbour is the row's new first texel), from the row and the row below; one lane
-// per row
-__global__ __launch_bounds__(64) void k_fire_update_slow(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w, uint32_t log2h, uint32_t att)
+// The slow variant: each row is a chain (the left neighbour is the value just written; the last
+// texel's right neighbour is the row's new first texel), from the row and the row below. A block
+// takes 16 rows, 256 columns at a time: all threads sum what a texel reads besides its left neighbour
+// (the loads do not depend on the chain, src and dst are distinct buffers) into LDS, one lane per row
+// runs the chain there, and all threads store the texels, after the step's points raised them.
+// Bound by the chain (an add, a multiply and a shift per texel); with each lane loading its own row's
+// bytes the 64 x 64 step took 5.3 us of update beside the points' 9.4 us.
+#define FIRE_SLOW_ROWS 16u
+#define FIRE_SLOW_COLS 256u
+template <uint32_t N>
+__global__ __launch_bounds__(256) void k_fire_step_slow(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
 {
-	const uint32_t y = blockIdx.x * 64u + threadIdx.x;
+	// a row's cells: the sums, then the chain's values (a word between rows: the chain's lanes read 16
+	// rows at one column, which then lie in 16 banks)
+	__shared__ uint32_t cells[FIRE_SLOW_ROWS][FIRE_SLOW_COLS + 1];
 	const uint32_t w = 1u << log2w, h = 1u << log2h;
-	if(y >= h)
-		return;
-	const uint32_t row = y << log2w;
-	if(y == h - 1u)
+	const uint32_t y0 = blockIdx.x * FIRE_SLOW_ROWS; // h is a multiple of 16
+	const uint32_t cols = w < FIRE_SLOW_COLS ? w : FIRE_SLOW_COLS, log2c = log2w < 8 ? log2w : 8u;
+	uint32_t prev = 0, first = 0;
+	if(threadIdx.x < FIRE_SLOW_ROWS)
+		prev = src[((y0 + threadIdx.x) << log2w) + w - 1u]; // the first texel's left neighbour
+	for(uint32_t x0 = 0; x0 < w; x0 += cols)
 	{
-		for(uint32_t x = 0; x < w; ++x)
-			dst[row + x] = 0;
-		return;
-	}
-	const uint32_t below = row + w;
-	const uint32_t first = ((uint32_t(src[row + w - 1u]) + src[row] + src[row + 1u] + src[below]) * att) >> 20;
-	dst[row] = uint8_t(first);
-	uint32_t prev = first & 0xFFu;
-	// the loads do not depend on the chain (src and dst are distinct buffers): unrolled, they overlap
+		for(uint32_t k = threadIdx.x; k < FIRE_SLOW_ROWS << log2c; k += 256u)
+		{
+			const uint32_t r = k >> log2c, x = x0 + (k & (cols - 1u)), row = (y0 + r) << log2w;
+			uint32_t s = 0;
+			if(y0 + r != h - 1u)
+				s = uint32_t(src[row + x]) + (x + 1u < w ? src[row + x + 1u] : 0u) + src[row + w + x];
+			cells[r][k & (cols - 1u)] = s;
+		}
+		__syncthreads();
+		if(threadIdx.x < FIRE_SLOW_ROWS && y0 + threadIdx.x != h - 1u)
+		{
+			uint32_t* c = cells[threadIdx.x];
 #pragma unroll 8
-	for(uint32_t x = 1; x < w - 1u; ++x)
-	{
-		const uint32_t v = ((prev + src[row + x] + src[row + x + 1u] + src[below + x]) * att) >> 20;
-		dst[row + x] = uint8_t(v);
-		prev = v & 0xFFu;
+			for(uint32_t k = 0; k < cols; ++k)
+			{
+				uint32_t s = c[k];
+				if(x0 + k == w - 1u)
+					s += first;
+				prev = ((prev + s) * att) >> 20;
+				if(x0 + k == 0)
+					first = prev;
+				c[k] = prev;
+			}
+		}
+		__syncthreads();
+		if(pts.n)
+		{
+			for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+			{
+				const uint32_t p = pts.p[k], a = p & swk::FIRE_POINT_ADDRESS;
+				const uint32_t px = (a & (w - 1u)) - x0, py = (a >> log2w) - y0;
+				if(px < cols && py < FIRE_SLOW_ROWS)
+					atomicMax(&cells[py][px], p >> swk::FIRE_POINT_HEAT_SHIFT);
+			}
+			__syncthreads();
+		}
+		for(uint32_t k = threadIdx.x; k < FIRE_SLOW_ROWS << log2c; k += 256u)
+		{
+			const uint32_t r = k >> log2c, c = k & (cols - 1u);
+			dst[((y0 + r) << log2w) + x0 + c] = uint8_t(cells[r][c]);
+		}
+		__syncthreads(); // the next columns rewrite the cells
 	}
-	const uint32_t last = ((prev + src[row + w - 1u] + (first & 0xFFu) + src[below + w - 1u]) * att) >> 20;
-	dst[row + w - 1u] = uint8_t(last);
 }
 
-// set_heat (:80-86) for the step's points, 64 at a time: the first point of each address takes the
-// maximum of the batch's heats for it (max is order-free)
+// set_heat (:80-86) for more points than a step's kernel arguments hold, 64 at a time: the first point
+// of each address takes the maximum of the batch's heats for it (max is order-free)
 __global__ __launch_bounds__(64) void k_fire_points(uint8_t* heat, const sw_heat_point* pts, uint32_t n, uint32_t log2w, uint32_t log2h)
 {
 	__shared__ uint32_t sa[64], sh[64];
@@ -682,22 +781,47 @@ void launch_water_texture(hipStream_t st, const float* field, uint32_t log2w, ui
 {
 	hipLaunchKernelGGL(k_water_texture_tiles, dim3(1u << (log2w + log2h - 8)), dim3(256), 0, st, field, log2w, log2h, w, texels);
 }
-void launch_fire_step(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h, uint32_t attenuation_i,
-	bool slow, const sw_heat_point* points_dev, uint32_t num_points)
+template <uint32_t N>
+static void launch_fire_step_n(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h,
+	uint32_t attenuation_i, bool slow, const sw_heat_point* points, uint32_t num_points)
 {
-	const uint32_t area = 1u << (log2w + log2h), h = 1u << log2h;
+	FirePoints<N> p;
+	p.n = num_points;
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	for(uint32_t k = 0; k < num_points; ++k)
+		p.p[k] = ((points[k].x & mx) + ((points[k].y & my) << log2w)) | ((points[k].heat & 0xFFu) << FIRE_POINT_HEAT_SHIFT);
+	const uint32_t blocks = ((1u << (log2w + log2h)) + 1023u) / 1024u;
 	if(slow)
-		hipLaunchKernelGGL(k_fire_update_slow, dim3((h + 63u) / 64u), dim3(64), 0, st, heat, heat_old, log2w, log2h, attenuation_i);
+		hipLaunchKernelGGL(k_fire_step_slow<N>, dim3((1u << log2h) / FIRE_SLOW_ROWS), dim3(256), 0, st, heat, heat_old, log2w, log2h,
+			attenuation_i, p);
+	else if((reinterpret_cast<uintptr_t>(heat) | reinterpret_cast<uintptr_t>(heat_old)) % 4 == 0)
+		hipLaunchKernelGGL((k_fire_step_fast<N, true>), dim3(blocks), dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
 	else
-		hipLaunchKernelGGL(k_fire_update_fast, dim3((area + 255u) / 256u), dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i);
-	if(num_points)
+		hipLaunchKernelGGL((k_fire_step_fast<N, false>), dim3(blocks), dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
+}
+
+void launch_fire_step(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h, uint32_t attenuation_i,
+	bool slow, const sw_heat_point* points, uint32_t num_points, const sw_heat_point* points_dev)
+{
+	// the smaller argument block where it holds the points: the runtime copies the whole block per launch
+	if(num_points <= FIRE_ARG_POINTS_SMALL)
+		launch_fire_step_n<FIRE_ARG_POINTS_SMALL>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, points, num_points);
+	else if(num_points <= FIRE_ARG_POINTS)
+		launch_fire_step_n<FIRE_ARG_POINTS>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, points, num_points);
+	else
+	{
+		launch_fire_step_n<FIRE_ARG_POINTS_SMALL>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, nullptr, 0);
 		hipLaunchKernelGGL(k_fire_points, dim3(1), dim3(64), 0, st, heat_old, points_dev, num_points, log2w, log2h);
+	}
 }
 
 void launch_fire_texture(hipStream_t st, const uint8_t* heat, uint32_t log2w, uint32_t log2h, const uint64_t dst_offset[5],
-	const uint32_t* palette_dev, uint32_t* lite)
+	const uint32_t palette[256], uint32_t* lite)
 {
-	hipLaunchKernelGGL(k_fire_texture_tiles, dim3(1u << (log2w + log2h - 8)), dim3(256), 0, st, heat, log2w, palette_dev, lite, dst_offset[0],
+	FirePalette p;
+	std::memcpy(p.color, palette, sizeof(p.color));
+	const uint32_t tiles = 1u << (log2w + log2h - 8);
+	hipLaunchKernelGGL(k_fire_texture, dim3((tiles + 3u) / 4u), dim3(256), 0, st, heat, log2w, tiles, p, lite, dst_offset[0],
 		dst_offset[1], dst_offset[2], dst_offset[3], dst_offset[4]);
 }
 
