@@ -33,7 +33,8 @@ enum
 	COUNTER_ERROR = 9,
 	COUNTER_COUNT = 16, // size of one block
 	COUNTER_RESULT = 16, // result block [16, 32)
-	COUNTER_TOTAL = 32,
+	COUNTER_WATER_TICKET = 32, // k_water_step's readers that are done (its last reader clears it)
+	COUNTER_TOTAL = 36,
 };
 
 enum
@@ -304,9 +305,27 @@ void launch_depth(hipStream_t st, const char* args_dev, const DepthPlan& plan, c
 	float* texels);
 // A skybox side (mip 0 from the image, then up to four halvings) back to back at dst.
 // water (generative_texture_effect_water.rs): one step (points, then the stencil into field_old) and
-// the wavy texture + mips (dst levels given by texel offsets)
+// the wavy texture + mips (dst levels given by texel offsets). Up to WATER_ARG_POINTS points travel in
+// the kernel's arguments, sorted by address; points_dev is their device copy when there are more.
+// ticket: a cleared device word, left cleared.
+const uint32_t WATER_ARG_POINTS_SMALL = 64u, WATER_ARG_POINTS = 256u;
+const uint32_t WATER_BLOCK = 1024u; // elements of a k_water_step block
+const uint32_t WATER_MAX_BLOCKS = (1u << 21) / WATER_BLOCK; // field areas are below 2^22: at most 2^21
+template <uint32_t N>
+struct WavePoints
+{
+	uint32_t n;
+	uint32_t address[N];
+	float value[N];
+};
+// neighbour n (left, right, up, down) of element a on the torus
+__host__ __device__ inline uint32_t water_neighbour(uint32_t a, uint32_t n, uint32_t log2w, uint32_t log2h)
+{
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u, x = a & mx, y = a >> log2w;
+	return n < 2u ? (y << log2w) + ((n ? x + 1u : x - 1u) & mx) : (((n == 2u ? y - 1u : y + 1u) & my) << log2w) + x;
+}
 void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
-	const sw_wave_point* points_dev, uint32_t num_points);
+	const sw_wave_point* points, uint32_t num_points, const sw_wave_point* points_dev, uint32_t* ticket);
 struct WaterTexLaunch
 {
 	uint64_t dst_offset[5]; // mip 0 .. 4

@@ -1647,7 +1647,7 @@ int sw_water_step(sw_ctx* ctx, float* field_device, float* field_old_device, uin
 	(void)hipSetDevice(ctx->device);
 	int r;
 	const sw_wave_point* pts_dev = nullptr;
-	if(num_points)
+	if(num_points > swk::WATER_ARG_POINTS) // else the points travel in the kernel's arguments
 	{
 		const size_t bytes = sizeof(sw_wave_point) * num_points;
 		char* staging = nullptr;
@@ -1660,7 +1660,8 @@ int sw_water_step(sw_ctx* ctx, float* field_device, float* field_old_device, uin
 	}
 	{
 		StageTimer t(ctx, STAGE_TEXTURES);
-		swk::launch_water_step(ctx->stream, field_device, field_old_device, log2_width, log2_height, attenuation, pts_dev, num_points);
+		swk::launch_water_step(ctx->stream, field_device, field_old_device, log2_width, log2_height, attenuation, points, num_points, pts_dev,
+			static_cast<uint32_t*>(ctx->counters.p) + COUNTER_WATER_TICKET);
 	}
 	return hip_check(ctx, hipGetLastError(), "water step launch");
 }

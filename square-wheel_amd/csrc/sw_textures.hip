@@ -8,6 +8,7 @@
 // them in order (each operation reads only its source and the same destination texel, so doing
 // them texel by texel gives the reference's level-by-level result).
 #include <algorithm>
+#include <bitset>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -355,8 +356,8 @@ namespace
 // ---------------------------------------------------------------------------------------------
 // Water (generative_texture_effect_water.rs)
 // ---------------------------------------------------------------------------------------------
-// add_point_value (:68-76) for the step's points, 64 at a time: the first point of each address in
-// a batch adds the batch's values for that address in order (points at one address add up in the
+// add_point_value (:68-76) for more points than a step's kernel arguments hold, 64 at a time: the first
+// point of each address in a batch adds the batch's values for that address in order (points at one address add up in the
 // reference's order; distinct addresses go in parallel); batches follow each other.
 __global__ __launch_bounds__(64) void k_water_points(float* field, float* field_old, const sw_wave_point* pts, uint32_t n,
 	uint32_t log2w, uint32_t log2h)
@@ -399,44 +400,157 @@ __global__ __launch_bounds__(64) void k_water_points(float* field, float* field_
 	}
 }
 
-// update_wave_field (:307-418): the field is a torus (rows and columns wrap); one lane per element
-__global__ __launch_bounds__(256) void k_water_stencil(float* __restrict__ dst, const float* __restrict__ src, uint32_t log2w, uint32_t log2h, float attenuation)
+// update_wave_field (:307-418), with the step's points (add_point_value, :68-76) where they travel in the
+// kernel's arguments: the field is a torus (rows and columns wrap); a block takes WATER_BLOCK consecutive
+// elements, four per thread. The stencil reads the field with the points added: the threads whose
+// neighbours hold points add them to the values they loaded, in the points' order (an address's additions
+// in the reference's order), and the owners subtract them from the old field. The field itself is updated
+// by the last of the blocks that read any point's element (they take tickets; nobody waits), when all of
+// them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 7 us
+// (2.9 us of copy, 4.3 us of points and 5.3 us of stencil as three operations); its 12.6 MB take 2.6 us at
+// the rate of a large copy. VEC: both buffers are 16-byte aligned.
+template <uint32_t N, bool VEC>
+__global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, float* __restrict__ src, uint32_t log2w, uint32_t log2h,
+	float attenuation, swk::WavePoints<N> pts, uint32_t readers, uint32_t* __restrict__ ticket)
 {
-	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	if(i >> (log2w + log2h))
-		return;
+	__shared__ uint64_t near_mask[N / 64 + 1]; // points whose element, or a neighbour of it, lies in this block
+	__shared__ uint32_t reads, last;
 	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	const uint32_t i = blockIdx.x * swk::WATER_BLOCK + threadIdx.x * 4u;
+	const bool in = (i >> (log2w + log2h)) == 0;
 	const uint32_t x = i & mx, y = i >> log2w;
-	const uint32_t row = y << log2w, up = ((y - 1u) & my) << log2w, down = ((y + 1u) & my) << log2w;
-	const float sum = ((src[row + ((x - 1u) & mx)] + src[row + ((x + 1u) & mx)]) + src[up + x]) + src[down + x];
-	dst[i] = (sum * 0.5f - dst[i]) * attenuation;
+	const uint32_t row = y << log2w, up = (((y - 1u) & my) << log2w) + x, down = (((y + 1u) & my) << log2w) + x;
+	const uint32_t il = row + ((x - 1u) & mx), ir = row + ((x + 4u) & mx);
+	float c[6], u[4], d[4], o[4];
+	if(in)
+	{
+		c[0] = src[il];
+		c[5] = src[ir];
+		if(VEC)
+		{
+			const float4 c4 = *reinterpret_cast<const float4*>(src + i), u4 = *reinterpret_cast<const float4*>(src + up),
+						 d4 = *reinterpret_cast<const float4*>(src + down), o4 = *reinterpret_cast<const float4*>(dst + i);
+			c[1] = c4.x, c[2] = c4.y, c[3] = c4.z, c[4] = c4.w;
+			u[0] = u4.x, u[1] = u4.y, u[2] = u4.z, u[3] = u4.w;
+			d[0] = d4.x, d[1] = d4.y, d[2] = d4.z, d[3] = d4.w;
+			o[0] = o4.x, o[1] = o4.y, o[2] = o4.z, o[3] = o4.w;
+		}
+		else
+#pragma unroll
+			for(uint32_t k = 0; k < 4; ++k)
+			{
+				c[k + 1] = src[i + k];
+				u[k] = src[up + k];
+				d[k] = src[down + k];
+				o[k] = dst[i + k];
+			}
+	}
+	if(pts.n)
+	{
+		if(threadIdx.x == 0)
+			reads = 0;
+		__syncthreads();
+		for(uint32_t base = threadIdx.x & ~63u; base < pts.n; base += 256u)
+		{
+			const uint32_t k = base + (threadIdx.x & 63u);
+			bool near = false, read = false;
+			if(k < pts.n)
+			{
+				const uint32_t a = pts.address[k];
+				for(uint32_t n = 0; n < 4; ++n)
+					read = read || swk::water_neighbour(a, n, log2w, log2h) / swk::WATER_BLOCK == blockIdx.x;
+				near = read || a / swk::WATER_BLOCK == blockIdx.x;
+			}
+			const uint64_t m = __ballot(near), r = __ballot(read);
+			if((threadIdx.x & 63u) == 0)
+			{
+				near_mask[base / 64u] = m;
+				if(r)
+					reads = 1; // every writer writes 1
+			}
+		}
+		__syncthreads();
+		for(uint32_t q = 0; q * 64u < pts.n; ++q)
+			for(uint64_t m = near_mask[q]; m; m &= m - 1u)
+			{
+				const uint32_t k = q * 64u + uint32_t(__builtin_ctzll(m)), a = pts.address[k];
+				const float v = pts.value[k];
+				// c[1 .. 4] are the thread's own elements: neighbours of each other
+				c[0] = a == il ? c[0] + v : c[0];
+				c[5] = a == ir ? c[5] + v : c[5];
+#pragma unroll
+				for(uint32_t e = 0; e < 4; ++e)
+				{
+					c[e + 1] = a == i + e ? c[e + 1] + v : c[e + 1];
+					o[e] = a == i + e ? o[e] - v : o[e];
+					u[e] = a == up + e ? u[e] + v : u[e];
+					d[e] = a == down + e ? d[e] + v : d[e];
+				}
+			}
+	}
+	if(in)
+	{
+		float r[4];
+#pragma unroll
+		for(uint32_t k = 0; k < 4; ++k)
+		{
+			const float sum = ((c[k] + c[k + 2]) + u[k]) + d[k];
+			r[k] = (sum * 0.5f - o[k]) * attenuation;
+		}
+		if(VEC)
+			*reinterpret_cast<float4*>(dst + i) = make_float4(r[0], r[1], r[2], r[3]);
+		else
+#pragma unroll
+			for(uint32_t k = 0; k < 4; ++k)
+				dst[i + k] = r[k];
+	}
+	if(pts.n == 0 || !reads)
+		return; // uniform over the block
+	// Every element of the field that this block reads has been read: the sums made of them were stored
+	// before the barrier. Nothing else has to be ordered (the field is only read until the last reader
+	// writes it), so the ticket is relaxed: a fence here would write back the L2's dirty lines, most of
+	// the new field, once per reading block (the step took 10.7 us with fences).
+	__syncthreads();
+	if(threadIdx.x == 0)
+		last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
+	__syncthreads();
+	if(!last)
+		return;
+	// the last reader: an address's points lie together, its first point's thread adds them up in order
+	for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+	{
+		const uint32_t a = pts.address[k];
+		if(k > 0 && pts.address[k - 1u] == a)
+			continue;
+		float f = src[a];
+		for(uint32_t j = k; j < pts.n && pts.address[j] == a; ++j)
+			f += pts.value[j];
+		src[a] = f;
+	}
+	if(threadIdx.x == 0)
+		*ticket = 0;
 }
 
 // PackedNormalRoughness::pack (textures.rs:33-39, fast_math.rs:64-78): x 127 per lane, cvtps2dq,
-// signed saturation to bytes
+// signed saturation to bytes. A value here is at most 127 in magnitude up to rounding, or NaN (a normal's
+// lane, a roughness), never above 2^31, so the saturation can go first: NaN becomes -128, as cvtps2dq's
+// "integer indefinite" does, and adding 1.5 * 2^23 rounds to the nearest even integer in the low bits.
+SW_DEV uint32_t pack_lane(float v)
+{
+	return __float_as_uint(__builtin_fminf(__builtin_fmaxf(v * 127.0f, -128.0f), 127.0f) + 12582912.0f) & 0xFFu;
+}
 SW_DEV int32_t pack_normal_roughness_dev(float x, float y, float z, float r)
 {
-	const float v[4] = {x * 127.0f, y * 127.0f, z * 127.0f, r * 127.0f};
-	uint32_t out = 0;
-	for(int k = 0; k < 4; ++k)
-	{
-		const int32_t q0 = f32_to_i32_rne_x86(v[k]);
-		const int32_t q = q0 < -128 ? -128 : q0 > 127 ? 127 : q0;
-		out |= (uint32_t(q) & 0xFFu) << (8 * k);
-	}
-	return int32_t(out);
+	return int32_t(pack_lane(x) | (pack_lane(y) << 8) | (pack_lane(z) << 16) | (pack_lane(r) << 24));
 }
 
-// make_wavy_texture_impl (:497-682) per texel: the normal from the field's central differences,
+// make_wavy_texture_impl (:497-682) per texel: the normal from the field's central differences dx, dy,
 // normalised as cgmath's normalize (v * (1 / |v|)), colours by mode
-SW_DEV sw_texel water_texel(const float* field, uint32_t log2w, uint32_t log2h, const swk::WaterTexLaunch& w, const sw_texel* texels,
+SW_DEV sw_texel water_texel(float dx, float dy, uint32_t log2w, uint32_t log2h, const swk::WaterTexLaunch& w, const sw_texel* texels,
 	uint32_t x, uint32_t y)
 {
 	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
-	const uint32_t i = x + (y << log2w);
-	const uint32_t row = y << log2w, up = ((y - 1u) & my) << log2w, down = ((y + 1u) & my) << log2w;
-	const float dx = field[row + ((x + 1u) & mx)] - field[row + ((x - 1u) & mx)];
-	const float dy = field[down + x] - field[up + x];
+	const uint32_t row = y << log2w, i = x + row;
 	const float m2 = (dx * dx + dy * dy) + 1.0f;
 	const float s = 1.0f / __builtin_sqrtf(m2);
 	const float nx = dx * s, ny = dy * s, nz = s;
@@ -510,34 +624,107 @@ SW_DEV sw_texel texel_mip(sw_texel p00, sw_texel p01, sw_texel p10, sw_texel p11
 	return t;
 }
 
-// The wavy texture of one 16 x 16 tile of mip 0 and the tile's texels of mips 1 .. 4, built in LDS
-// (a mip texel depends only on the square of mip 0 under it): one launch for the texture and its mips.
-__global__ __launch_bounds__(256) void k_water_texture_tiles(const float* field, uint32_t log2w, uint32_t log2h, swk::WaterTexLaunch w,
-	sw_texel* texels)
+// The lane's 2 x 2 square of texels at Morton distance step (the square's first lane, then x + 1 at step,
+// y + 1 at 2 * step) as one texel of the next mip.
+SW_DEV sw_texel quad_mip(sw_texel t, uint32_t lane, uint32_t step)
 {
-	__shared__ sw_texel tile[16 * 16];
-	const uint32_t tx = blockIdx.x & ((1u << (log2w - 4)) - 1u), ty = blockIdx.x >> (log2w - 4);
-	const uint32_t lx = threadIdx.x & 15u, ly = threadIdx.x >> 4;
-	const uint32_t x = tx * 16u + lx, y = ty * 16u + ly;
-	const sw_texel t = water_texel(field, log2w, log2h, w, texels, x, y);
-	tile[threadIdx.x] = t;
-	texels[w.dst_offset[0] + x + (y << log2w)] = t; // each lane reads only its own old texel
-	__syncthreads();
-	for(uint32_t mip = 1, n = 8; mip <= 4; ++mip, n >>= 1)
+	const uint32_t first = lane & ~(4u * step - 1u);
+	auto from = [&](uint32_t l) {
+		sw_texel r;
+		r.diffuse = uint32_t(__shfl(int(t.diffuse), int(l)));
+		r.packed_normal_roughness = __shfl(t.packed_normal_roughness, int(l));
+		return r;
+	};
+	return texel_mip(from(first), from(first + 2u * step), from(first + step), from(first + 3u * step));
+}
+
+// The wavy texture and its mips 1 .. 4 in one launch, a 16 x 16 tile of mip 0 per wave (a mip texel
+// depends only on the square of mip 0 under it): a lane takes a 2 x 2 square of mip 0 and its mip 1 texel;
+// the lanes lie in Morton order, so the block's first wave takes mip 2 of its four tiles from LDS (a
+// texel's four parts follow each other), then mips 3 and 4 by lane exchanges. A square shares its field
+// loads (12 values for four texels' 16). Bound by the correctly rounded roots and divisions of the normals:
+// that is why the upper mips are gathered into one wave instead of costing every wave a pass each
+// (1024 x 1024: 15.5 us with a texel per thread and the mips through LDS with barriers, 12.6 us with a pass
+// per wave and mip, 9.9 us so; its 27 MB take 5.7 us at the rate of a large copy).
+// PAIRS: the field is 8-byte aligned and the level starts on 16 bytes, so field values and texels move in
+// pairs.
+template <bool PAIRS>
+__global__ __launch_bounds__(256) void k_water_texture(const float* __restrict__ field, uint32_t log2w, uint32_t log2h, uint32_t tiles,
+	swk::WaterTexLaunch w, sw_texel* texels)
+{
+	__shared__ sw_texel mip1[256];
+	const uint32_t lane = threadIdx.x & 63u;
+	// past the last tile a wave redoes it (the same texels) for the barrier below
+	const uint32_t tile = std::min(blockIdx.x * 4u + (threadIdx.x >> 6), tiles - 1u);
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	const uint32_t tx = tile & ((1u << (log2w - 4)) - 1u), ty = tile >> (log2w - 4);
+	const uint32_t qx = (lane & 1u) | ((lane >> 1) & 2u) | ((lane >> 2) & 4u), qy = ((lane >> 1) & 1u) | ((lane >> 2) & 2u) | ((lane >> 3) & 4u);
+	const uint32_t x = tx * 16u + qx * 2u, y = ty * 16u + qy * 2u;
+	// rows y - 1 .. y + 2 at columns x, x + 1; rows y, y + 1 also at x - 1 and x + 2
+	float f[4][4];
+#pragma unroll
+	for(uint32_t r = 0; r < 4; ++r)
 	{
-		sw_texel v{};
-		const bool active = lx < n && ly < n;
-		if(active)
-			v = texel_mip(tile[(2u * ly) * 16u + 2u * lx], tile[(2u * ly + 1u) * 16u + 2u * lx], tile[(2u * ly) * 16u + 2u * lx + 1u],
-				tile[(2u * ly + 1u) * 16u + 2u * lx + 1u]);
-		__syncthreads();
-		if(active)
+		const float* row = field + (((y + r - 1u) & my) << log2w);
+		if(PAIRS)
 		{
-			tile[ly * 16u + lx] = v;
-			texels[w.dst_offset[mip] + (tx * n + lx) + ((ty * n + ly) << (log2w - mip))] = v;
+			const float2 p = *reinterpret_cast<const float2*>(row + x);
+			f[r][1] = p.x;
+			f[r][2] = p.y;
 		}
-		__syncthreads();
+		else
+		{
+			f[r][1] = row[x];
+			f[r][2] = row[x + 1u];
+		}
+		if(r == 1 || r == 2)
+		{
+			f[r][0] = row[(x - 1u) & mx];
+			f[r][3] = row[(x + 2u) & mx];
+		}
 	}
+	const uint32_t i0 = x + (y << log2w), i1 = i0 + (1u << log2w);
+	sw_texel* out = texels + w.dst_offset[0];
+	sw_texel t[2][2]; // [y][x]
+#pragma unroll
+	for(uint32_t r = 0; r < 2; ++r)
+#pragma unroll
+		for(uint32_t c = 0; c < 2; ++c)
+			t[r][c] = water_texel(f[r + 1][c + 2] - f[r + 1][c], f[r + 2][c + 1] - f[r][c + 1], log2w, log2h, w, texels, x + c, y + r);
+	if(PAIRS)
+	{
+		*reinterpret_cast<uint4*>(out + i0) = make_uint4(t[0][0].diffuse, uint32_t(t[0][0].packed_normal_roughness), t[0][1].diffuse,
+			uint32_t(t[0][1].packed_normal_roughness));
+		*reinterpret_cast<uint4*>(out + i1) = make_uint4(t[1][0].diffuse, uint32_t(t[1][0].packed_normal_roughness), t[1][1].diffuse,
+			uint32_t(t[1][1].packed_normal_roughness));
+	}
+	else
+	{
+		out[i0] = t[0][0];
+		out[i0 + 1] = t[0][1];
+		out[i1] = t[1][0];
+		out[i1 + 1] = t[1][1];
+	}
+	sw_texel v = texel_mip(t[0][0], t[1][0], t[0][1], t[1][1]);
+	texels[w.dst_offset[1] + (tx * 8u + qx) + ((ty * 8u + qy) << (log2w - 1))] = v;
+	mip1[threadIdx.x] = v;
+	__syncthreads();
+	if(threadIdx.x >= 64u)
+		return;
+	// the first wave: lane 16 q + j takes mip 2 texel j (Morton order) of the block's tile q
+	const uint32_t mt = blockIdx.x * 4u + (lane >> 4);
+	const bool ok = mt < tiles;
+	const uint32_t mtx = mt & ((1u << (log2w - 4)) - 1u), mty = mt >> (log2w - 4);
+	const uint32_t jx = (lane & 1u) | ((lane >> 1) & 2u), jy = ((lane >> 1) & 1u) | ((lane >> 2) & 2u);
+	v = texel_mip(mip1[lane * 4u], mip1[lane * 4u + 2u], mip1[lane * 4u + 1u], mip1[lane * 4u + 3u]);
+	if(ok)
+		texels[w.dst_offset[2] + (mtx * 4u + jx) + ((mty * 4u + jy) << (log2w - 2))] = v;
+	v = quad_mip(v, lane, 1);
+	if(ok && (lane & 3u) == 0)
+		texels[w.dst_offset[3] + (mtx * 2u + (jx >> 1)) + ((mty * 2u + (jy >> 1)) << (log2w - 3))] = v;
+	v = quad_mip(v, lane, 4);
+	if(ok && (lane & 15u) == 0)
+		texels[w.dst_offset[4] + mtx + (mty << (log2w - 4))] = v;
 }
 
 // The average of the lane's 2 x 2 square of texels, the square's lanes step apart in Morton order:
@@ -767,19 +954,60 @@ __global__ __launch_bounds__(64) void k_fire_points(uint8_t* heat, const sw_heat
 
 namespace swk
 {
-void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
-	const sw_wave_point* points_dev, uint32_t num_points)
+template <uint32_t N>
+static void launch_water_step_n(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
+	const sw_wave_point* points, uint32_t num_points, uint32_t* ticket)
 {
-	if(num_points)
+	WavePoints<N> p;
+	p.n = num_points;
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	// sorted by address, an address's points in their order: only their own order matters to it
+	uint64_t order[N];
+	for(uint32_t k = 0; k < num_points; ++k)
+		order[k] = (uint64_t((points[k].x & mx) + ((points[k].y & my) << log2w)) << 32) | k;
+	std::sort(order, order + num_points);
+	// the blocks that read a point's element: those of its four neighbours
+	std::bitset<WATER_MAX_BLOCKS> readers;
+	for(uint32_t k = 0; k < num_points; ++k)
+	{
+		p.address[k] = uint32_t(order[k] >> 32);
+		p.value[k] = points[uint32_t(order[k])].value;
+		for(uint32_t n = 0; n < 4; ++n)
+			readers.set(water_neighbour(p.address[k], n, log2w, log2h) / WATER_BLOCK);
+	}
+	const uint32_t blocks = ((1u << (log2w + log2h)) + WATER_BLOCK - 1u) / WATER_BLOCK;
+	const bool vec = (reinterpret_cast<uintptr_t>(field) | reinterpret_cast<uintptr_t>(field_old)) % 16 == 0;
+	if(vec)
+		hipLaunchKernelGGL((k_water_step<N, true>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
+			uint32_t(readers.count()), ticket);
+	else
+		hipLaunchKernelGGL((k_water_step<N, false>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
+			uint32_t(readers.count()), ticket);
+}
+
+void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
+	const sw_wave_point* points, uint32_t num_points, const sw_wave_point* points_dev, uint32_t* ticket)
+{
+	// the smaller argument block where it holds the points: the runtime copies the whole block per launch
+	if(num_points <= WATER_ARG_POINTS_SMALL)
+		launch_water_step_n<WATER_ARG_POINTS_SMALL>(st, field, field_old, log2w, log2h, attenuation, points, num_points, ticket);
+	else if(num_points <= WATER_ARG_POINTS)
+		launch_water_step_n<WATER_ARG_POINTS>(st, field, field_old, log2w, log2h, attenuation, points, num_points, ticket);
+	else
+	{
 		hipLaunchKernelGGL(k_water_points, dim3(1), dim3(64), 0, st, field, field_old, points_dev, num_points, log2w, log2h);
-	const uint32_t area = 1u << (log2w + log2h);
-	hipLaunchKernelGGL(k_water_stencil, dim3((area + 255u) / 256u), dim3(256), 0, st, field_old, static_cast<const float*>(field), log2w,
-		log2h, attenuation);
+		launch_water_step_n<WATER_ARG_POINTS_SMALL>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
+	}
 }
 
 void launch_water_texture(hipStream_t st, const float* field, uint32_t log2w, uint32_t log2h, const WaterTexLaunch& w, sw_texel* texels)
 {
-	hipLaunchKernelGGL(k_water_texture_tiles, dim3(1u << (log2w + log2h - 8)), dim3(256), 0, st, field, log2w, log2h, w, texels);
+	const uint32_t tiles = 1u << (log2w + log2h - 8);
+	const dim3 grid((tiles + 3u) / 4u);
+	if(reinterpret_cast<uintptr_t>(field) % 8 == 0 && reinterpret_cast<uintptr_t>(texels + w.dst_offset[0]) % 16 == 0)
+		hipLaunchKernelGGL(k_water_texture<true>, grid, dim3(256), 0, st, field, log2w, log2h, tiles, w, texels);
+	else
+		hipLaunchKernelGGL(k_water_texture<false>, grid, dim3(256), 0, st, field, log2w, log2h, tiles, w, texels);
 }
 template <uint32_t N>
 static void launch_fire_step_n(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h,
