@@ -4,20 +4,24 @@
 //
 // The reference steps 1 / z by additions along a span (inv_z += d_inv_z_dx) and along the rows of a
 // polygon part (line_inv_z += d_inv_z_dy); float addition rounds at every step, so each value is the
-// end of a chain of additions. The kernels keep those chains: a wave computes 64 consecutive values
-// of a chain by a lane-serial scan (lane j adds to lane j - 1's value), chunk after chunk.
+// end of a chain of additions, which sw_chain.h gives without walking it: every row's and every
+// pixel's value on its own.
 //
-//   k_depth_setup   one wave per draw: the edge walk (lane 0) into parts, then per row of each part
-//                   the span's x range and its first pixel's 1 / z (the rows' chain by the scan)
-//   k_depth_raster  one wave per four depth-buffer rows, a 16-lane row of the wave per buffer row:
-//                   the target's draws in order, each covering span filled 16 pixels at a time
-//                   (the pixels' chain by a 16-lane scan, the four rows' chains side by side)
+//   k_depth_setup   one wave per draw: the edge walk into parts (identical on all lanes, comparisons
+//                   only), the parts' slopes one part per lane, then one row per lane: the span's x
+//                   range and its first pixel's 1 / z. Reads the packed draws and vertices straight
+//                   from pinned host memory (each byte once, so no copy goes ahead of the launch) and
+//                   leaves in device memory what the raster reads many times.
+//   k_depth_raster  one wave per depth-buffer row: the row's spans of the target's draws from the last
+//                   to the first, each taking the pixels no later overwriting draw has taken (64-pixel
+//                   masks, scalar arithmetic), until all are taken; then each pixel's 1 / z once.
 #include <cstring>
 #include <string>
 #include <vector>
 
 #include "sw_internal.h"
 #include "sw_device.h"
+#include "sw_chain.h"
 
 using namespace swd;
 
@@ -40,16 +44,24 @@ struct DepthDrawDev
 	uint32_t depth_test;
 	uint32_t target;
 	uint32_t pad;
-	uint64_t rec_base; // the draw's row records: rec_base + y, y < the target's height
 };
 
 struct DepthTargetDev
 {
 	uint64_t offset; // of the depth buffer in the texels
+	uint64_t rec_base; // row records: rec_base + y * num_draws + (draw - first_draw)
 	uint32_t w, h;
 	uint32_t first_draw, num_draws;
-	uint32_t first_row_block; // raster blocks: first_row_block + y / DEPTH_ROWS_PER_BLOCK
+	uint32_t first_row; // raster rows: first_row + y
 	uint32_t flags; // SW_DEPTH_*
+};
+
+// What the raster reads of a draw, beside its row records.
+struct DepthDrawInfo
+{
+	int32_t first, end; // rows [first, end) have records
+	float dx;
+	uint32_t depth_test;
 };
 
 // make_shadow_map_circle (light.rs:130-154): texels [0, dx) and [size - dx, size) of row y are
@@ -64,267 +76,320 @@ SW_DEV uint32_t circle_margin(int32_t size, int32_t y)
 
 struct DepthLaunch
 {
-	const DepthDrawDev* draws;
-	const DepthTargetDev* targets;
-	uint32_t num_targets;
-	uint32_t pad;
+	const DepthDrawDev* draws; // pinned host memory: draws, targets and vertices
+	const DepthTargetDev* host_targets;
 	const int32_t* vdata;
+	DepthTargetDev* targets; // device memory, written by the setup
+	DepthDrawInfo* infos;
 	DepthRow* rows;
-	int32_t* draw_rows; // per draw: [first, end) rows with records
 	float* texels;
-};
-
-// value of lane j = value of lane j - 1 + d, lane 0 = start (a chain of j float additions). Each
-// round moves every lane's value one lane up (the DPP wavefront shift wave_shr:1) and adds d; after
-// round s lanes 0 .. s hold their final values. Called with all 64 lanes active.
-SW_DEV float lane_shr1(float v)
-{
-	return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xF, 0xF, false));
-}
-// within each 16-lane row of the wave: sublane j gets sublane j - 1's value (DPP row_shr:1), and
-// the chain of four independent 16-value pieces (sublane 0 of each row takes its own start)
-SW_DEV float row_shr1(float v)
-{
-	return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x111, 0xF, 0xF, false));
-}
-SW_DEV float serial_chain16(float start, float d)
-{
-	const bool first = (threadIdx.x & 15u) == 0;
-	float v = start;
-	for(uint32_t s = 1; s < 16; ++s)
-	{
-		const float p = row_shr1(v) + d;
-		v = first ? start : p;
-	}
-	return v;
-}
-SW_DEV float serial_chain(float start, float d)
-{
-	const bool first = (threadIdx.x & 63u) == 0;
-	float v = start;
-	for(uint32_t s = 1; s < 64; ++s)
-	{
-		const float p = lane_shr1(v) + d;
-		v = first ? start : p;
-	}
-	return v;
-}
-
-struct Part
-{
-	int32_t y0, y1; // rows [y0, y1), clamped to the buffer
-	int32_t xl, xr; // x_left / x_right of row y0 (with + 0.5)
-	int32_t dxl, dxr;
-	float line_inv_z; // of row y0
+	uint32_t num_draws, num_targets, num_rows;
 };
 
 #define MAX_DEPTH_PARTS SW_MAX_POLYGON_VERTICES
 
-__global__ __launch_bounds__(64) void k_depth_setup(DepthLaunch L)
+SW_DEV int32_t lane_pull(int32_t v, uint32_t src) { return __builtin_amdgcn_ds_bpermute(int32_t(src << 2), v); }
+SW_DEV float lane_pull_f(float v, uint32_t src) { return __builtin_bit_cast(float, lane_pull(__builtin_bit_cast(int, v), src)); }
+SW_DEV int32_t rl(int32_t v, uint32_t lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// Four draws per block, a wave each; blocks past the draws copy the targets to device memory.
+__global__ __launch_bounds__(256) void k_depth_setup(DepthLaunch L, uint32_t draw_blocks)
 {
-	__shared__ Part parts[MAX_DEPTH_PARTS];
-	__shared__ uint32_t num_parts;
-	const DepthDrawDev d = L.draws[blockIdx.x];
-	const DepthTargetDev t = L.targets[d.target];
-	const uint32_t lane = threadIdx.x;
-	DepthRow* rows = L.rows + d.rec_base;
-	for(uint32_t y = lane; y < t.h; y += 64)
-		rows[y] = DepthRow{0, 0, 0.0f};
-	if(lane == 0)
+	const uint32_t lane = threadIdx.x & 63u;
+	if(blockIdx.x >= draw_blocks)
 	{
-		// fill_polygon (rasterizer.rs:1315-1412): from the lowest vertex up both chains
-		const int32_t* v = L.vdata + d.first_vertex_int;
-		const uint32_t n = d.num_vertices;
-		uint32_t lower = 0;
-		int32_t min_y = v[1];
-		for(uint32_t i = 0; i < n; ++i)
-			if(v[i * 2 + 1] < min_y)
-			{
-				min_y = v[i * 2 + 1];
-				lower = i;
-			}
-		uint32_t left = lower, right = lower, np = 0;
-		int32_t cur_y = min_y;
-		const int32_t H = int32_t(t.h);
-		for(uint32_t guard = 0; guard < 2 * n + 2; ++guard)
-		{
-			const uint32_t next_left = left + n - 1 >= n ? left + n - 1 - n : left + n - 1;
-			const uint32_t next_right = right + 1 >= n ? right + 1 - n : right + 1;
-			const int32_t lx = v[left * 2], ly = v[left * 2 + 1], nlx = v[next_left * 2], nly = v[next_left * 2 + 1];
-			const int32_t rx = v[right * 2], ry = v[right * 2 + 1], nrx = v[next_right * 2], nry = v[next_right * 2 + 1];
-			const int32_t dy_left = nly - ly, dy_right = nry - ry;
-			const int32_t next_y = nly < nry ? nly : nry;
-			bool fill = false;
-			int32_t xs_l = 0, xs_r = 0, dl = 0, dr = 0;
-			if(dy_left > FIXED16_HALF && dy_right > FIXED16_HALF)
-			{
-				dl = fixed16_div(nlx - lx, dy_left);
-				dr = fixed16_div(nrx - rx, dy_right);
-				xs_l = lx + fixed16_mul(dl, cur_y - ly);
-				xs_r = rx + fixed16_mul(dr, cur_y - ry);
-				fill = true;
-			}
-			else if(dy_left > 0 && dy_right > 0)
-			{
-				const int32_t cur_y_int = fixed16_round_to_int(cur_y), next_y_int = fixed16_round_to_int(next_y);
-				if(cur_y_int < next_y_int)
-				{
-					const int32_t thin_line_y = int_to_fixed16(cur_y_int) + FIXED16_HALF;
-					xs_l = lx + fixed16_mul_div(thin_line_y - ly, nlx - lx, dy_left);
-					xs_r = rx + fixed16_mul_div(thin_line_y - ry, nrx - rx, dy_right);
-					fill = true;
-				}
-			}
-			if(fill && np < MAX_DEPTH_PARTS)
-			{
-				// fill_polygon_part (:1414-1465): the part's first row
-				const int32_t y0 = imax32(fixed16_round_to_int(cur_y), 0);
-				const int32_t y1 = imin32(fixed16_round_to_int(next_y), H);
-				const int32_t y_start_delta = int_to_fixed16(y0) + FIXED16_HALF - cur_y;
-				Part& p = parts[np++];
-				p.y0 = y0;
-				p.y1 = y1;
-				p.xl = xs_l + fixed16_mul(y_start_delta, dl) + FIXED16_HALF;
-				p.xr = xs_r + fixed16_mul(y_start_delta, dr) + FIXED16_HALF;
-				p.dxl = dl;
-				p.dxr = dr;
-				p.line_inv_z = float(y0) * d.dy + 0.5f * (d.dx + d.dy) + d.k;
-			}
-			if(next_left == next_right)
-				break;
-			if(nry < nly)
-				right = next_right;
-			else
-				left = next_left;
-			cur_y = next_y;
-		}
-		num_parts = np;
+		const uint32_t words = L.num_targets * uint32_t(sizeof(DepthTargetDev) / 4u);
+		const uint32_t i = (blockIdx.x - draw_blocks) * 256u + threadIdx.x;
+		if(i < words)
+			reinterpret_cast<uint32_t*>(L.targets)[i] = reinterpret_cast<const uint32_t*>(L.host_targets)[i];
+		return;
 	}
-	__syncthreads();
-	int32_t first = int32_t(t.h), end = 0;
-	for(uint32_t pi = 0; pi < num_parts; ++pi)
+	const uint32_t di = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+	if(di >= L.num_draws)
+		return; // uniform over the wave; no barriers below
+	const DepthDrawDev d = L.draws[di];
+	const DepthTargetDev t = L.host_targets[d.target];
+	const uint32_t n = d.num_vertices;
+	int32_t vx = 0, vy = 0; // lane i: vertex i
+	if(lane < n)
 	{
-		const Part p = parts[pi];
-		if(p.y0 >= p.y1)
-			continue;
-		first = imin32(first, p.y0);
-		end = imax32(end, p.y1);
-		float carry = p.line_inv_z;
-		for(int32_t yb = p.y0; yb < p.y1; yb += 64)
+		vx = L.vdata[d.first_vertex_int + lane * 2u];
+		vy = L.vdata[d.first_vertex_int + lane * 2u + 1u];
+	}
+	// fill_polygon (rasterizer.rs:1315-1412): from the lowest vertex up both chains; lane p keeps part p
+	uint32_t lower = 0, np = 0;
+	int32_t min_y = rl(vy, 0);
+	for(uint32_t i = 0; i < n; ++i)
+		if(rl(vy, i) < min_y)
 		{
-			const float line_inv_z = serial_chain(carry, d.dy);
-			const int32_t y = yb + int32_t(lane);
-			if(y < p.y1)
+			min_y = rl(vy, i);
+			lower = i;
+		}
+	uint32_t left = lower, right = lower;
+	int32_t cur_y = min_y;
+	const int32_t H = int32_t(t.h);
+	uint32_t pl = 0, pnl = 0, pr = 0, pnr = 0;
+	int32_t p_cur = 0, p_y0 = 0, p_y1 = 0;
+	bool p_wide = false;
+	for(uint32_t guard = 0; guard < 2 * n + 2; ++guard)
+	{
+		const uint32_t next_left = left + n - 1 >= n ? left + n - 1 - n : left + n - 1;
+		const uint32_t next_right = right + 1 >= n ? right + 1 - n : right + 1;
+		const int32_t ly = rl(vy, left), nly = rl(vy, next_left), ry = rl(vy, right), nry = rl(vy, next_right);
+		const int32_t dy_left = nly - ly, dy_right = nry - ry;
+		const int32_t next_y = nly < nry ? nly : nry;
+		const bool wide = dy_left > FIXED16_HALF && dy_right > FIXED16_HALF;
+		const bool thin = !wide && dy_left > 0 && dy_right > 0 && fixed16_round_to_int(cur_y) < fixed16_round_to_int(next_y);
+		if((wide || thin) && np < MAX_DEPTH_PARTS)
+		{
+			if(lane == np)
 			{
-				const uint32_t r = uint32_t(y - p.y0);
-				const int32_t xl = int32_t(uint32_t(p.xl) + r * uint32_t(p.dxl)), xr = int32_t(uint32_t(p.xr) + r * uint32_t(p.dxr));
-				const int32_t x0 = imax32(fixed16_floor_to_int(xl), 0), x1 = imin32(fixed16_floor_to_int(xr), int32_t(t.w));
-				DepthRow row{0, 0, 0.0f};
+				pl = left;
+				pnl = next_left;
+				pr = right;
+				pnr = next_right;
+				p_cur = cur_y;
+				p_wide = wide;
+				p_y0 = imax32(fixed16_round_to_int(cur_y), 0);
+				p_y1 = imin32(fixed16_round_to_int(next_y), H);
+			}
+			np++;
+		}
+		if(next_left == next_right)
+			break;
+		if(nry < nly)
+			right = next_right;
+		else
+			left = next_left;
+		cur_y = next_y;
+	}
+	// the parts' sides and first rows (fill_polygon, fill_polygon_part :1414-1465), lane p for part p;
+	// every lane takes part in the exchanges
+	const int32_t lx = lane_pull(vx, pl), ly = lane_pull(vy, pl), nlx = lane_pull(vx, pnl), nly = lane_pull(vy, pnl);
+	const int32_t rx = lane_pull(vx, pr), ry = lane_pull(vy, pr), nrx = lane_pull(vx, pnr), nry = lane_pull(vy, pnr);
+	int32_t xl = 0, xr = 0, dl = 0, dr = 0;
+	float line_inv_z = 0.0f;
+	if(lane < np)
+	{
+		int32_t xs_l, xs_r;
+		if(p_wide)
+		{
+			dl = fixed16_div(nlx - lx, nly - ly);
+			dr = fixed16_div(nrx - rx, nry - ry);
+			xs_l = lx + fixed16_mul(dl, p_cur - ly);
+			xs_r = rx + fixed16_mul(dr, p_cur - ry);
+		}
+		else
+		{
+			const int32_t thin_line_y = int_to_fixed16(fixed16_round_to_int(p_cur)) + FIXED16_HALF;
+			xs_l = lx + fixed16_mul_div(thin_line_y - ly, nlx - lx, nly - ly);
+			xs_r = rx + fixed16_mul_div(thin_line_y - ry, nrx - rx, nry - ry);
+		}
+		const int32_t y_start_delta = int_to_fixed16(p_y0) + FIXED16_HALF - p_cur;
+		xl = xs_l + fixed16_mul(y_start_delta, dl) + FIXED16_HALF;
+		xr = xs_r + fixed16_mul(y_start_delta, dr) + FIXED16_HALF;
+		line_inv_z = float(p_y0) * d.dy + 0.5f * (d.dx + d.dy) + d.k;
+	}
+	int32_t first = H, end = 0;
+	for(uint32_t q = 0; q < np; ++q)
+	{
+		const int32_t y0 = rl(p_y0, q), y1 = rl(p_y1, q);
+		if(y0 < y1)
+		{
+			first = imin32(first, y0);
+			end = imax32(end, y1);
+		}
+	}
+	// a row per lane: its part is the last one that holds it
+	for(int32_t yb = first; yb < end; yb += 64)
+	{
+		const int32_t y = yb + int32_t(lane);
+		uint32_t part = MAX_DEPTH_PARTS;
+		for(uint32_t q = 0; q < np; ++q)
+		{
+			const int32_t y0 = rl(p_y0, q), y1 = rl(p_y1, q);
+			part = y >= y0 && y < y1 ? q : part;
+		}
+		const uint32_t src = part < MAX_DEPTH_PARTS ? part : 0u;
+		const int32_t y0 = lane_pull(p_y0, src);
+		const int32_t r_xl = lane_pull(xl, src), r_xr = lane_pull(xr, src), r_dl = lane_pull(dl, src), r_dr = lane_pull(dr, src);
+		const float r_z = lane_pull_f(line_inv_z, src);
+		if(y < end)
+		{
+			DepthRow row{0, 0, 0.0f};
+			if(part < MAX_DEPTH_PARTS)
+			{
+				const uint32_t r = uint32_t(y - y0);
+				const int32_t x_left = wadd(r_xl, wmul(int32_t(r), r_dl)), x_right = wadd(r_xr, wmul(int32_t(r), r_dr));
+				const int32_t x0 = imax32(fixed16_floor_to_int(x_left), 0), x1 = imin32(fixed16_floor_to_int(x_right), int32_t(t.w));
 				if(x0 < x1)
-					row = DepthRow{uint16_t(x0), uint16_t(x1), line_inv_z + float(x0) * d.dx};
-				rows[y] = row;
+					row = DepthRow{uint16_t(x0), uint16_t(x1), swchain::chain_add(r_z, d.dy, r) + float(x0) * d.dx};
 			}
-			carry = __shfl(line_inv_z, 63) + d.dy;
+			L.rows[t.rec_base + uint64_t(uint32_t(y)) * t.num_draws + (di - t.first_draw)] = row;
 		}
 	}
 	if(lane == 0)
-	{
-		L.draw_rows[blockIdx.x * 2] = first < end ? first : 0;
-		L.draw_rows[blockIdx.x * 2 + 1] = first < end ? end : 0;
-	}
+		L.infos[di] = DepthDrawInfo{first < end ? first : 0, first < end ? end : 0, d.dx, d.depth_test};
 }
 
-#define DEPTH_ROWS_PER_BLOCK 4u // one 16-lane row of the wave per depth-buffer row
-#define DEPTH_LDS_WIDTH 1024u // rows up to this width are drawn in LDS, written back once
-
-__global__ __launch_bounds__(64) void k_depth_raster(DepthLaunch L)
+// bits [0, n) of 64, n clamped to [0, 64]
+SW_DEV uint64_t low_bits(int32_t n) { return n <= 0 ? 0ull : n >= 64 ? ~0ull : (1ull << n) - 1ull; }
+// the bits of [x0, x1) that lie in the 32 columns from base on
+SW_DEV uint32_t span_bits(int32_t x0, int32_t x1, int32_t base)
 {
-	uint32_t lo = 0, hi = L.num_targets;
-	while(hi - lo > 1)
+	const int32_t a = imax32(x0 - base, 0), b = imin32(x1 - base, 32);
+	return a < b ? (~0u << a) & (~0u >> (32 - b)) : 0u;
+}
+
+#define DEPTH_SEGMENTS 4u // 64-pixel segments a wave holds at once
+
+// The rows of a 256 x 256 cube side take one pass of 256 columns each. A back-to-front list overwrites
+// most pixels several times: walked backwards, a row is finished after its nearest spans, and each pixel's
+// chain is evaluated once instead of once per draw that covers it. Eight lights' 256 x 256 cube maps (3.1
+// Mtexels, 1,633 draws): 33.6 us with every span filled in draw order by 16-lane chains.
+__global__ __launch_bounds__(256) void k_depth_raster(DepthLaunch L)
+{
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+	if(wave >= L.num_rows)
+		return; // uniform over the wave; no barriers below
+	// the row's target: the last one whose rows start at or before this one, 64 targets a step
+	uint32_t ti = 0;
+	for(uint32_t base = 0; base < L.num_targets; base += 64u)
 	{
-		const uint32_t mid = (lo + hi) >> 1;
-		if(L.targets[mid].first_row_block <= blockIdx.x)
-			lo = mid;
-		else
-			hi = mid;
+		const bool le = base + lane < L.num_targets && L.targets[base + lane].first_row <= wave;
+		const uint32_t count = uint32_t(__popcll(__ballot(le)));
+		if(count)
+			ti = base + count - 1u;
+		if(count < 64u)
+			break;
 	}
-	const DepthTargetDev t = L.targets[lo];
-	const uint32_t lane = threadIdx.x, g = lane >> 4, sub = lane & 15u;
-	const int32_t y = int32_t((blockIdx.x - t.first_row_block) * DEPTH_ROWS_PER_BLOCK + g);
-	const bool row_ok = y < int32_t(t.h);
-	__shared__ float srow[DEPTH_ROWS_PER_BLOCK * DEPTH_LDS_WIDTH];
-	const bool in_lds = t.w <= DEPTH_LDS_WIDTH;
-	float* grow = L.texels + t.offset + uint64_t(row_ok ? y : 0) * t.w;
-	float* row = in_lds ? srow + g * DEPTH_LDS_WIDTH : grow;
-	if(in_lds)
-	{
-		if(row_ok)
-			for(uint32_t x = sub; x < t.w; x += 16)
-				row[x] = grow[x];
-		__syncthreads();
-	}
+	const DepthTargetDev t = L.targets[ti];
+	const int32_t y = int32_t(wave - t.first_row);
 	const uint32_t draws_end = t.first_draw + t.num_draws;
-	for(uint32_t base = t.first_draw; base < draws_end; base += 16)
+	const DepthRow* rows = L.rows + t.rec_base + uint64_t(uint32_t(y)) * t.num_draws;
+	float* out = L.texels + t.offset + uint64_t(uint32_t(y)) * t.w;
+	// lane's draw di: its span of this row, packed x0 | x1 << 16 (0: none), 1 / z at x0
+	auto load_span = [&](bool ok, uint32_t di, DepthDrawInfo& info, float& inv_z) -> uint32_t {
+		inv_z = 0.0f;
+		info = DepthDrawInfo{0, 0, 0.0f, 0};
+		if(!ok)
+			return 0u;
+		const DepthRow r = rows[di - t.first_draw]; // not written outside the draw's rows: dropped below
+		info = L.infos[di];
+		inv_z = r.inv_z;
+		return y >= info.first && y < info.end && r.x0 < r.x1 ? uint32_t(r.x0) | (uint32_t(r.x1) << 16) : 0u;
+	};
+	for(uint32_t cx = 0; cx < t.w; cx += 64u * DEPTH_SEGMENTS)
 	{
-		// lane (g, j) fetches draw base + j and its record of row y
-		const uint32_t di = base + sub;
-		uint32_t span = 0;
-		float inv_z = 0.0f, dx = 0.0f;
-		int32_t test = 0;
-		if(di < draws_end)
+		uint64_t open[DEPTH_SEGMENTS]; // pixels no overwriting draw has taken yet
+		float z[DEPTH_SEGMENTS];
+		uint32_t from[DEPTH_SEGMENTS]; // the draw that took the pixel, + 1
+		uint64_t any_open = 0;
+		bool tests = false;
+#pragma unroll
+		for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 		{
-			const DepthDrawDev d = L.draws[di];
-			dx = d.dx;
-			test = int32_t(d.depth_test);
-			const int32_t y_first = L.draw_rows[di * 2], y_end = L.draw_rows[di * 2 + 1];
-			if(row_ok && y >= y_first && y < y_end)
+			open[s] = low_bits(int32_t(t.w) - int32_t(cx + 64u * s));
+			any_open |= open[s];
+			z[s] = 0.0f;
+			from[s] = 0;
+		}
+		// backwards, 64 draws at a time: lane k holds draw chunk_end - 1 - k
+		for(uint32_t chunk_end = draws_end; chunk_end > t.first_draw && any_open; chunk_end = chunk_end - t.first_draw > 64u ? chunk_end - 64u : t.first_draw)
+		{
+			const uint32_t left = chunk_end - t.first_draw;
+			DepthDrawInfo info;
+			float inv_z;
+			const uint32_t span = load_span(lane < left, chunk_end - 1u - lane, info, inv_z);
+			const bool meets = (span >> 16) > cx && (span & 0xFFFFu) < cx + 64u * DEPTH_SEGMENTS && span != 0u;
+			tests = tests || __ballot(meets && info.depth_test != 0u) != 0;
+			uint64_t hits = __ballot(meets && info.depth_test == 0u);
+			// every lane's span as bits of the segments, so that a hit costs two readlanes, three scalar
+			// operations and a select per segment
+			uint32_t src[DEPTH_SEGMENTS], bits[DEPTH_SEGMENTS][2];
+#pragma unroll
+			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 			{
-				const DepthRow r = L.rows[d.rec_base + uint32_t(y)];
-				if(r.x0 < r.x1)
+				src[s] = 64u;
+#pragma unroll
+				for(uint32_t h = 0; h < 2; ++h)
+					bits[s][h] = span_bits(int32_t(span & 0xFFFFu), int32_t(span >> 16), int32_t(cx + 64u * s + 32u * h));
+			}
+			while(hits && any_open)
+			{
+				const uint32_t k = uint32_t(__builtin_ctzll(hits));
+				hits &= hits - 1u;
+				any_open = 0;
+#pragma unroll
+				for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 				{
-					span = uint32_t(r.x0) | (uint32_t(r.x1) << 16);
-					inv_z = r.inv_z;
+					const uint64_t take = open[s] & (uint64_t(uint32_t(rl(int32_t(bits[s][0]), k))) | (uint64_t(uint32_t(rl(int32_t(bits[s][1]), k))) << 32));
+					open[s] ^= take;
+					any_open |= open[s];
+					src[s] = __builtin_amdgcn_inverse_ballot_w64(take) ? k : src[s];
+				}
+			}
+			// the pixels taken in this chunk: their chain's end
+#pragma unroll
+			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+			{
+				if(__ballot(src[s] < 64u) == 0)
+					continue;
+				const uint32_t k = src[s] & 63u;
+				const float start = lane_pull_f(inv_z, k), step = lane_pull_f(info.dx, k);
+				const uint32_t x0 = uint32_t(lane_pull(int32_t(span), k)) & 0xFFFFu;
+				if(src[s] < 64u)
+				{
+					z[s] = swchain::chain_add(start, step, cx + 64u * s + lane - x0);
+					from[s] = chunk_end - k;
 				}
 			}
 		}
-		const uint64_t any = __ballot(span != 0u);
-		uint32_t draw_mask = uint32_t((any | (any >> 16) | (any >> 32) | (any >> 48)) & 0xFFFFu);
-		while(draw_mask)
+		if(tests)
 		{
-			// the draws in order; each group draws its own row's span
-			const int j = __builtin_ctz(draw_mask);
-			draw_mask &= draw_mask - 1u;
-			const float ddx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dx), j));
-			const bool dtest = __builtin_amdgcn_readlane(test, j) != 0;
-			const int src = int((g << 4) | uint32_t(j));
-			const uint32_t sp = uint32_t(__shfl(int(span), src));
-			float carry = __shfl(inv_z, src);
-			const uint32_t x0 = sp & 0xFFFFu, len = (sp >> 16) - x0; // 0 where the row is not covered (sp = 0)
-			const uint32_t len_all = max(max(uint32_t(__shfl(int(len), 0)), uint32_t(__shfl(int(len), 16))),
-				max(uint32_t(__shfl(int(len), 32)), uint32_t(__shfl(int(len), 48))));
-			for(uint32_t c = 0; c < len_all; c += 16)
+			// depth-tested draws over the pixels' overwriting draw (or the buffer's value), in order
+#pragma unroll
+			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 			{
-				const float v = serial_chain16(carry, ddx);
-				if(c + sub < len)
+				const uint32_t x = cx + 64u * s + lane;
+				if(from[s] == 0 && x < t.w)
+					z[s] = out[x];
+			}
+			for(uint32_t base = t.first_draw; base < draws_end; base += 64u)
+			{
+				DepthDrawInfo info;
+				float inv_z;
+				const uint32_t span = load_span(base + lane < draws_end, base + lane, info, inv_z);
+				uint64_t hits = __ballot((span >> 16) > cx && (span & 0xFFFFu) < cx + 64u * DEPTH_SEGMENTS && span != 0u && info.depth_test != 0u);
+				while(hits)
 				{
-					const uint32_t x = x0 + c + sub;
-					row[x] = dtest ? fmax_r(v, row[x]) : v;
+					const uint32_t k = uint32_t(__builtin_ctzll(hits));
+					hits &= hits - 1u;
+					const uint32_t sp = uint32_t(rl(int32_t(span), k)), x0 = sp & 0xFFFFu, x1 = sp >> 16;
+					const float start = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, inv_z), k));
+					const float step = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, info.dx), k));
+#pragma unroll
+					for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+					{
+						const uint32_t x = cx + 64u * s + lane;
+						if(x >= x0 && x < x1 && base + k + 1u > from[s])
+							z[s] = fmax_r(swchain::chain_add(start, step, x - x0), z[s]);
+					}
 				}
-				carry = __shfl(v, int((g << 4) | 15u)) + ddx;
 			}
 		}
+		const uint32_t margin = t.flags & SW_DEPTH_CIRCLE ? circle_margin(int32_t(t.w), y) : 0u;
+#pragma unroll
+		for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+		{
+			const uint32_t x = cx + 64u * s + lane;
+			const bool outside = (t.flags & SW_DEPTH_CIRCLE) && (x < margin || x >= t.w - margin);
+			// with depth tests every pixel is stored (one that no draw touched as it was)
+			if(x < t.w && (outside || tests || !__builtin_amdgcn_inverse_ballot_w64(open[s])))
+				out[x] = outside ? 1.0e24f : z[s];
+		}
 	}
-	__syncthreads();
-	if((t.flags & SW_DEPTH_CIRCLE) && row_ok)
-	{
-		const uint32_t dx = circle_margin(int32_t(t.w), y);
-		for(uint32_t x = sub; x < t.w; x += 16)
-			if(x < dx || x >= t.w - dx)
-				row[x] = 1.0e24f;
-	}
-	if(in_lds && row_ok)
-		for(uint32_t x = sub; x < t.w; x += 16)
-			grow[x] = row[x];
 }
 
 } // namespace
@@ -337,7 +402,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 	std::vector<DepthTargetDev> tg(num_targets);
 	std::vector<DepthDrawDev> dd(num_draws);
 	uint64_t rec = 0;
-	uint32_t row_blocks = 0, next_draw = 0;
+	uint32_t rows = 0, next_draw = 0;
 	for(uint32_t i = 0; i < num_targets; ++i)
 	{
 		const sw_depth_target& t = targets[i];
@@ -353,10 +418,11 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 			return (error = which + "unknown flags"), -1;
 		if((t.flags & SW_DEPTH_CIRCLE) && t.width != t.height)
 			return (error = which + "the circle needs a square target"), -1;
-		if(uint64_t(row_blocks) + t.height > 0x7FFFFFFFu)
+		if(uint64_t(rows) + t.height > 0x7FFFFFFFu)
 			return (error = "depth targets: too many rows"), -1;
-		tg[i] = DepthTargetDev{t.offset, t.width, t.height, t.first_draw, t.num_draws, row_blocks, t.flags};
-		row_blocks += (t.height + DEPTH_ROWS_PER_BLOCK - 1) / DEPTH_ROWS_PER_BLOCK;
+		tg[i] = DepthTargetDev{t.offset, rec, t.width, t.height, t.first_draw, t.num_draws, rows, t.flags};
+		rows += t.height;
+		rec += uint64_t(t.height) * t.num_draws;
 		for(uint32_t k = t.first_draw; k < t.first_draw + t.num_draws; ++k)
 		{
 			const sw_depth_draw& s = draws[k];
@@ -364,8 +430,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 				uint64_t(s.first_vertex_int) + 2ull * s.num_vertices > num_vertex_ints)
 				return (error = "depth draw " + std::to_string(k) + ": vertices out of range"), -1;
 			dd[k] = DepthDrawDev{s.first_vertex_int, s.num_vertices, s.depth_equation[0], s.depth_equation[1], s.depth_equation[2],
-				s.depth_test ? 1u : 0u, i, 0, rec};
-			rec += t.height;
+				s.depth_test ? 1u : 0u, i, 0};
 		}
 	}
 	if(next_draw != num_draws)
@@ -373,7 +438,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 	plan.targets_at = (sizeof(DepthDrawDev) * dd.size() + 255) & ~size_t(255);
 	plan.bytes = plan.targets_at + sizeof(DepthTargetDev) * tg.size();
 	plan.row_records = rec;
-	plan.row_blocks = row_blocks;
+	plan.rows = rows;
 	plan.num_draws = num_draws;
 	plan.num_targets = num_targets;
 	packed.assign(plan.bytes, 0);
@@ -383,14 +448,25 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 }
 
 size_t depth_row_record_bytes() { return sizeof(DepthRow); }
-
-void launch_depth(hipStream_t st, const char* args_dev, const DepthPlan& plan, const int32_t* vdata, void* rows, int32_t* draw_rows, float* texels)
+size_t depth_work_bytes(const DepthPlan& plan)
 {
-	if(plan.num_draws == 0 || plan.row_blocks == 0)
+	return ((sizeof(DepthTargetDev) * plan.num_targets + 255) & ~size_t(255)) + sizeof(DepthDrawInfo) * plan.num_draws;
+}
+
+void launch_depth(hipStream_t st, const char* args, const int32_t* vdata, const DepthPlan& plan, char* work, void* rows, float* texels,
+	bool raster)
+{
+	DepthLaunch L{reinterpret_cast<const DepthDrawDev*>(args), reinterpret_cast<const DepthTargetDev*>(args + plan.targets_at), vdata,
+		reinterpret_cast<DepthTargetDev*>(work),
+		reinterpret_cast<DepthDrawInfo*>(work + ((sizeof(DepthTargetDev) * plan.num_targets + 255) & ~size_t(255))),
+		static_cast<DepthRow*>(rows), texels, plan.num_draws, plan.num_targets, plan.rows};
+	if(plan.num_draws == 0 || plan.rows == 0)
 		return;
-	DepthLaunch L{reinterpret_cast<const DepthDrawDev*>(args_dev), reinterpret_cast<const DepthTargetDev*>(args_dev + plan.targets_at),
-		plan.num_targets, 0, vdata, static_cast<DepthRow*>(rows), draw_rows, texels};
-	hipLaunchKernelGGL(k_depth_setup, dim3(plan.num_draws), dim3(64), 0, st, L);
-	hipLaunchKernelGGL(k_depth_raster, dim3(plan.row_blocks), dim3(64), 0, st, L);
+	const uint32_t draw_blocks = (plan.num_draws + 3u) / 4u;
+	const uint32_t copy_blocks = (plan.num_targets * uint32_t(sizeof(DepthTargetDev) / 4u) + 255u) / 256u;
+	if(!raster)
+		hipLaunchKernelGGL(k_depth_setup, dim3(draw_blocks + copy_blocks), dim3(256), 0, st, L, draw_blocks);
+	else
+		hipLaunchKernelGGL(k_depth_raster, dim3((plan.rows + 3u) / 4u), dim3(256), 0, st, L);
 }
 } // namespace swk

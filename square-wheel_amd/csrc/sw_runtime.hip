@@ -76,8 +76,8 @@ struct sw_ctx
 
 	// command buffers / work buffers
 	DevBuf views, surfaces, lights, light_indices, draws, vdata, surf_ext, blk_surf, parts, spans, drec, dbounds, counters, arena, fb,
-		tonemap_out, tonemap_sums, bloom0, bloom1, bloom_lines, model_args, model_scratch, texop_args, shadows, depth_args, depth_vdata,
-		depth_rows, depth_draw_rows, water_points, fire_args, portal_mix, mesh_args, mesh_fans;
+		tonemap_out, tonemap_sums, bloom0, bloom1, bloom_lines, model_args, model_scratch, texop_args, shadows, depth_args,
+		depth_rows, water_points, fire_args, portal_mix, mesh_args, mesh_fans;
 	uint32_t num_shadows = 0; // sw_set_light_shadows: entries in `shadows`
 	const float* shadow_texels = nullptr;
 	uint32_t tile_rows = 8; // raster tile height (SW_TILE_ROWS_*), set by sw_set_tile_rows / the autotuner
@@ -137,6 +137,7 @@ struct sw_ctx
 	// pinned: packed launch arguments (model preparation, texture ops, depth draws, shadows), a ring
 	// of slots so that the host fills the next slot while earlier copies wait in the stream
 	char* arg_staging[ARG_STAGING_SLOTS] = {};
+	void* arg_staging_dev[ARG_STAGING_SLOTS] = {}; // their device addresses
 	size_t arg_staging_cap[ARG_STAGING_SLOTS] = {};
 	hipEvent_t arg_staging_event[ARG_STAGING_SLOTS] = {}; // recorded after the last copy out of the slot
 	uint32_t arg_staging_slot = 0; // the slot of the current stage_begin
@@ -870,8 +871,8 @@ void sw_ctx_destroy(sw_ctx* ctx)
 		(void)hipGraphDestroy(ctx->graph);
 	DevBuf* bufs[] = {&ctx->views, &ctx->surfaces, &ctx->lights, &ctx->light_indices, &ctx->draws, &ctx->vdata, &ctx->surf_ext, &ctx->blk_surf,
 		&ctx->parts, &ctx->spans, &ctx->drec, &ctx->dbounds, &ctx->counters, &ctx->arena, &ctx->fb, &ctx->tonemap_out, &ctx->tonemap_sums,
-		&ctx->bloom0, &ctx->bloom1, &ctx->bloom_lines, &ctx->model_args, &ctx->model_scratch, &ctx->texop_args, &ctx->shadows, &ctx->depth_args, &ctx->depth_vdata,
-		&ctx->depth_rows, &ctx->depth_draw_rows, &ctx->water_points, &ctx->fire_args};
+		&ctx->bloom0, &ctx->bloom1, &ctx->bloom_lines, &ctx->model_args, &ctx->model_scratch, &ctx->texop_args, &ctx->shadows, &ctx->depth_args,
+		&ctx->depth_rows, &ctx->water_points, &ctx->fire_args};
 	for(DevBuf* b : bufs)
 		release(ctx, *b);
 	if(ctx->counters_host)
@@ -1336,9 +1337,15 @@ int sw_postprocess_device(sw_ctx* ctx, const void* hdr_device, uint32_t width, u
 
 // Small launch arguments travel from pinned staging memory. stage_begin takes the next slot of the
 // ring, waits until the copies out of it (ARG_STAGING_SLOTS calls ago) have completed (its event),
-// grows it if needed and returns it; stage_copy queues a copy out of the slot (at src_offset) and
-// records the slot's event after it.
-static int stage_begin(sw_ctx* ctx, size_t bytes, char** out)
+// grows it if needed and returns it (and its device address); stage_copy queues a copy out of the slot
+// (at src_offset) and records the slot's event after it; a launch that reads the slot itself is followed by
+// stage_used.
+static int stage_used(sw_ctx* ctx)
+{
+	return hip_check(ctx, hipEventRecord(ctx->arg_staging_event[ctx->arg_staging_slot], ctx->stream), "argument staging event");
+}
+
+static int stage_begin(sw_ctx* ctx, size_t bytes, char** out, const char** out_device = nullptr)
 {
 	int r;
 	const uint32_t k = (ctx->arg_staging_slot + 1) % ARG_STAGING_SLOTS;
@@ -1352,8 +1359,9 @@ static int stage_begin(sw_ctx* ctx, size_t bytes, char** out)
 		ctx->arg_staging[k] = nullptr;
 		ctx->arg_staging_cap[k] = 0;
 		const size_t cap = std::max<size_t>(bytes * 2, 64 << 10);
-		if((r = hip_check(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->arg_staging[k]), cap, hipHostMallocDefault),
-				"argument staging allocation")))
+		if((r = hip_check(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->arg_staging[k]), cap, hipHostMallocMapped),
+				"argument staging allocation")) ||
+			(r = hip_check(ctx, hipHostGetDevicePointer(&ctx->arg_staging_dev[k], ctx->arg_staging[k], 0), "argument staging address")))
 			return r;
 		ctx->arg_staging_cap[k] = cap;
 	}
@@ -1361,6 +1369,8 @@ static int stage_begin(sw_ctx* ctx, size_t bytes, char** out)
 		(r = hip_check(ctx, hipEventCreateWithFlags(&ctx->arg_staging_event[k], hipEventDisableTiming), "argument staging event")))
 		return r;
 	*out = ctx->arg_staging[k];
+	if(out_device)
+		*out_device = static_cast<const char*>(ctx->arg_staging_dev[k]);
 	return SW_OK;
 }
 
@@ -1371,7 +1381,7 @@ static int stage_copy(sw_ctx* ctx, void* dst_device, size_t bytes, size_t src_of
 	if((r = hip_check(ctx, hipMemcpyAsync(dst_device, ctx->arg_staging[k] + src_offset, bytes, hipMemcpyHostToDevice, ctx->stream),
 			"argument copy")))
 		return r;
-	return hip_check(ctx, hipEventRecord(ctx->arg_staging_event[k], ctx->stream), "argument staging event");
+	return stage_used(ctx);
 }
 
 int sw_mix_portal_textures(sw_ctx* ctx, sw_map* map, uint32_t color_bits, const sw_portal_mix* mixes, uint32_t num_mixes,
@@ -1795,24 +1805,27 @@ int sw_render_depth(sw_ctx* ctx, const sw_depth_target* targets, uint32_t num_ta
 	(void)hipSetDevice(ctx->device);
 	int r;
 	const size_t vbytes = sizeof(int32_t) * num_vertex_ints;
-	if((r = ensure(ctx, ctx->depth_args, plan.bytes)) || (r = ensure(ctx, ctx->depth_vdata, std::max<size_t>(vbytes, 4))) ||
-		(r = ensure(ctx, ctx->depth_rows, std::max<uint64_t>(plan.row_records, 1) * swk::depth_row_record_bytes())) ||
-		(r = ensure(ctx, ctx->depth_draw_rows, sizeof(int32_t) * 2 * std::max<uint32_t>(num_draws, 1))))
+	if((r = ensure(ctx, ctx->depth_args, swk::depth_work_bytes(plan))) ||
+		(r = ensure(ctx, ctx->depth_rows, std::max<uint64_t>(plan.row_records, 1) * swk::depth_row_record_bytes())))
 		return r;
-	// the packed draws and the vertex data through one staging slot (no copy from pageable memory)
+	// the packed draws and the vertex data in one staging slot, which the setup reads itself
 	char* staging = nullptr;
+	const char* staging_dev = nullptr;
 	const size_t vat = (plan.bytes + 255) & ~size_t(255);
-	if((r = stage_begin(ctx, vat + vbytes, &staging)))
+	if((r = stage_begin(ctx, vat + vbytes, &staging, &staging_dev)))
 		return r;
 	std::memcpy(staging, ctx->depth_packed.data(), plan.bytes);
 	if(vbytes)
 		std::memcpy(staging + vat, vertex_data, vbytes);
-	if((r = stage_copy(ctx, ctx->depth_args.p, plan.bytes)) || (vbytes && (r = stage_copy(ctx, ctx->depth_vdata.p, vbytes, vat))))
-		return r;
 	{
 		StageTimer t(ctx, STAGE_DEPTH);
-		swk::launch_depth(ctx->stream, static_cast<const char*>(ctx->depth_args.p), plan, static_cast<const int32_t*>(ctx->depth_vdata.p),
-			ctx->depth_rows.p, static_cast<int32_t*>(ctx->depth_draw_rows.p), depth_texels_device);
+		for(const bool raster : {false, true})
+		{
+			swk::launch_depth(ctx->stream, staging_dev, reinterpret_cast<const int32_t*>(staging_dev + vat), plan,
+				static_cast<char*>(ctx->depth_args.p), ctx->depth_rows.p, depth_texels_device, raster);
+			if(!raster && (r = stage_used(ctx)))
+				return r;
+		}
 	}
 	return hip_check(ctx, hipGetLastError(), "depth launch");
 }
