@@ -820,7 +820,7 @@ def main():
     launches = max(prof[dominant][1], 1)
     avg_s = prof[dominant][0] / 1e3 / launches
     achieved = bytes_sum[dominant] / launches / avg_s / 1e9
-    raster_key = f"k_raster_tiles_rows{plain_rows}" + ("_sspan" if ctx.scalar_spans() else "")
+    raster_key = f"k_raster_tiles_rows{plain_rows}"
     traffic_key = {"raster_tiles": raster_key, "setup_and_surfaces": "k_setup_and_surfaces_256",
                    "build_surfaces": "k_build_surfaces"}.get(dominant)
     traffic = read_traffic("plain1080p", traffic_key) if traffic_key else None

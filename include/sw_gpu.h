@@ -360,23 +360,21 @@ int sw_batch_wait(sw_ctx* ctx);
  * HIP graph and replays it; inputs must be device-resident and unchanged in size. */
 int sw_render_batch_graph(sw_ctx* ctx, sw_map* map, const sw_batch* batch, void* out_framebuffer_device);
 
-/* Raster tile height. The raster kernel gives each 64-pixel-wide screen tile of 4, 8 or 16 rows
- * to one wave (default 8). Small tiles give more waves (latency hiding on small frames), tall tiles
- * amortise the per-tile draw binning (large batches). No counterpart in the reference (its
- * rasteriser walks the rows of one screen rect per thread, rect_splitting.rs:23-78). */
+/* Raster tile height. The raster kernel gives each screen tile of 4, 8 or 16 rows (default 8) and 16, 32
+ * or 64 pixels of width, chosen from the views' sizes, to one wave. Small tiles give more waves (latency
+ * hiding on small frames), large ones amortise the per-tile draw binning (large batches). No counterpart
+ * in the reference (its rasteriser walks the rows of one screen rect per thread, rect_splitting.rs:23-78). */
 #define SW_TILE_ROWS_COUNT 3 /* candidates: 4, 8, 16 */
 int sw_set_tile_rows(sw_ctx* ctx, uint32_t rows);
 uint32_t sw_get_tile_rows(const sw_ctx* ctx);
 
-/* How the raster kernel loads the span records of its (draw, row) items: 1 = one scalar load per
- * item into SGPRs, 0 = one vector load per 16 items shared with readlane. Both give identical
- * output; which is faster depends on the workload (the autotuner picks). */
+/* How the raster kernel loaded span records when it had two ways: kept for callers that set it, the value
+ * is stored and returned and changes nothing else (there is one way now, as fast as either was or faster). */
 int sw_set_scalar_spans(sw_ctx* ctx, uint32_t enable);
 uint32_t sw_get_scalar_spans(const sw_ctx* ctx);
 
-/* Autotuner: renders `batch` with every tile height and both span load modes, keeps the fastest
- * for this context and reports the milliseconds per batch of each tile height (4, 8, 16 rows; the
- * better mode) in out_ms (may be NULL). */
+/* Autotuner: renders `batch` with every tile height, keeps the fastest for this context and reports the
+ * milliseconds per batch of each (4, 8, 16 rows) in out_ms (may be NULL). */
 int sw_autotune_batch(
 	sw_ctx* ctx, sw_map* map, const sw_batch* batch, void* out_framebuffer_device, uint32_t* out_rows,
 	double out_ms[SW_TILE_ROWS_COUNT]);

@@ -101,4 +101,15 @@ SW_HD uint32_t z_from_inv_z(uint32_t div)
 	return uint32_t(double(1u << 31) / double(div));
 }
 
+// The same quotient for the divisors of a perspective span's pixels, with one correction step: for
+// 2048 <= div < 2^22 the quotient x is at most 2^20, so 2^31 * rcp is within x * 2^-21 <= 0.5 of x for an rcp
+// within 4 ulp; less 0.5 (exact: the value is below 2^21, a multiple of 2^-4) it lies in (x - 1, x], its
+// truncation q is floor(x) or one less, and the remainder decides. Both factors of q * div are below
+// 2^24 (a full-rate 24-bit multiplication).
+SW_HD uint32_t z_from_rcp_near(uint32_t div, float rcp)
+{
+	const uint32_t q = uint32_t(__builtin_fmaf(rcp, 2147483648.0f, -0.5f));
+	return q + (0x80000000u - (q & 0xFFFFFFu) * (div & 0xFFFFFFu) >= div ? 1u : 0u);
+}
+
 } // namespace swdiv

@@ -12,6 +12,7 @@
 // Raster tiles are 64 pixels wide (one pixel column per lane) and TILE_ROWS rows high, chosen per
 // context among SW_TILE_ROWS_* (the autotuner times each).
 #define MAX_TILE_ROWS 16
+#define NUM_SIMDS 1024u // 256 CUs of four
 // rasterizer.rs:137-271 walks at most n - 1 vertex pairs of an n <= 24 polygon.
 #define MAX_PARTS_PER_DRAW 24
 
@@ -81,7 +82,7 @@ struct ViewExt
 {
 	sw_view v;
 	uint32_t num_bands; // tile rows of the view
-	uint32_t cols; // 64-pixel columns
+	uint32_t cols; // tile columns
 	uint32_t first_tile; // global tile (wave) index of tile 0
 	uint32_t pad;
 	uint64_t arena_end; // end of the view's arena region: the next view's offset, or the arena's end
@@ -250,9 +251,8 @@ void launch_build_surfaces(hipStream_t st, uint32_t color_bits, const MapPtrs& m
 // Kernels 1 + 2 in one launch when the host prepared the surfaces.
 void launch_setup_and_surfaces(hipStream_t st, uint32_t lanes, uint32_t color_bits, SetupArgs a, const ViewsArg& views,
 	const SurfaceArgs& sa, const MapPtrs& m);
-// Kernel 3: one wave per 64 x tile_rows tile (binning fused); scalar_spans: span records through
-// the scalar unit (else vector loads shared with readlane).
-void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, bool scalar_spans, const MapPtrs& m,
+// Kernel 3: one wave per tile_width x tile_rows tile (binning fused); widths 16, 32, 64, rows 4, 8, 16 (at most 512 pixels).
+void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
 	const DrawBounds* bounds, const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views, const void* arena,
 	const void* skybox, void* fb, uint32_t total_tiles, const uint32_t* counters);
 // Kernel 4 (one block): per-draw statistics -> result block (host-mapped), live block cleared.

@@ -10,15 +10,16 @@
 //                     block -> first surface table of the next kernel.
 //   k_build_surfaces  one thread per surface-arena texel, flattened over all surfaces of all views:
 //                     surfaces.rs:433-852 + :854-971 for that texel
-//   k_raster_tiles    one wave per 64 x ROWS screen tile (ROWS = 4, 8 or 16): ballots over the
+//   k_raster_tiles    one wave per screen tile of 16, 32 or 64 x 4, 8 or 16 pixels: ballots over the
 //                     view's draws pick the ones overlapping the tile, in draw order; the tile's
-//                     colour lives in LDS; a part's span records for the tile rows are loaded
-//                     across lanes at once and broadcast with readlane; the texel addresses of all
-//                     rows are computed and fetched together, then blended in row order with
-//                     write_into_framebuffer (:424-445, :558-572, :705-719, :1223-1279)
+//                     colours live in registers, 16 x 4 pixels to one; a draw's span records for
+//                     the tile rows are loaded at once and broadcast over each row's 16 lanes; its
+//                     texels are fetched together, then blended with write_into_framebuffer
+//                     (:424-445, :558-572, :705-719, :1223-1279)
 //   k_finish          one block: per-draw statistics -> result counters, live counters cleared
 //   k_tonemap         one thread per pixel: postprocessor.rs:237-253
 #include <algorithm>
+#include <utility>
 
 #include "sw_device.h"
 #include <hip/hip_ext.h>
@@ -2133,102 +2134,155 @@ __global__ __launch_bounds__(1024) void k_finish(const DrawRec* __restrict__ dre
 }
 
 // =============================================================================================
-// Tiled raster: one wave per 64 x ROWS tile, one pixel column per lane, colour in registers
+// Tiled raster: one wave per 16 NK x ROWS tile, a lane per pixel of its 16 x 4 units, colour in registers
 // =============================================================================================
 
-// Texel address of one pixel of a polygon span: perspective (rasterizer.rs:425-452) or linear tc
-// (line-z :559-579, affine :705-727); -1 if the texel lies outside the texture (skipped; the
-// reference's clamps keep its unchecked fetches inside).
-template <int KIND>
-SW_DEV int32_t polygon_texel_index(const int32_t* sv, int32_t j, uint32_t tw, uint32_t th)
+// Global memory by bytes: keeps a load whose address travels as an integer (a readlane result) a global_load
+// (a generic pointer would make it a flat load, which also waits on, and occupies, the LDS counter).
+typedef __attribute__((address_space(1))) const char* GlobalBytes;
+
+// Lane N of each 16-lane row of the wave, in all of the row's lanes (DPP row_newbcast).
+template <int N>
+SW_DEV int32_t row_lane(int32_t v)
 {
-	uint32_t u, v;
-	if(KIND == 0)
-	{
-		const int32_t inv_z = wadd(sv[0], wmul(j, sv[1]));
-		uint32_t div = uint32_t(inv_z) >> INV_Z_PRE_SHIFT;
-		div = div ? div : 1u;
-		// (1 << Z_CALC_SHIFT) / div, exact through the double quotient
-		const uint32_t z = swdiv::z_from_inv_z(div);
-		const int32_t t0 = wadd(sv[2], wmul(j, sv[3]));
-		const int32_t t1 = wadd(sv[4], wmul(j, sv[5]));
-		u = uint32_t((uint64_t(z) * uint64_t(int64_t(t0))) >> TC_FINAL_SHIFT);
-		v = uint32_t((uint64_t(z) * uint64_t(int64_t(t1))) >> TC_FINAL_SHIFT);
-	}
-	else
-	{
-		u = uint32_t(wadd(sv[0], wmul(j, sv[1])) >> 16);
-		v = uint32_t(wadd(sv[2], wmul(j, sv[3])) >> 16);
-	}
-	return (u < tw && v < th) ? int32_t(u + v * tw) : -1;
+	return __builtin_amdgcn_update_dpp(0, v, 0x150 + N, 0xF, 0xF, false);
 }
 
-// Element i of a global-memory array whose address travels as an integer (a readlane result): the
-// global address space keeps the load a global_load (a generic pointer would make it a flat load,
-// which also waits on, and occupies, the LDS counter).
+// The lanes where p holds (one scalar compare; __ballot goes through an integer per lane) and back.
+SW_DEV uint64_t lanes_of(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+SW_DEV bool lane_in(uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes); }
+
+// x as whatever its register holds (so that a loop carries nothing into it), and x as a value the compiler
+// knows nothing about (neither the conditions it was made of, nor anything to compute ahead of a branch).
 template <class T>
-SW_DEV T global_at(uint64_t addr, int32_t i)
+SW_DEV void any_value(T& x)
 {
-	typedef __attribute__((address_space(1))) const T* GlobalPtr;
-	typedef __attribute__((address_space(1))) const char* GlobalBytes;
-	// i * sizeof(T) < 2^32: textures hold at most 2^29 texels (the draw validation)
-	return *(GlobalPtr)((GlobalBytes)addr + uint32_t(i) * uint32_t(sizeof(T)));
+	asm("" : "=v"(x));
+}
+template <class T>
+SW_DEV void one_value(T& x)
+{
+	asm volatile("" : "+v"(x));
 }
 
-
-// Texel indices of a draw's active rows in the tile (bit rr of gmask: row rr's span meets the
-// tile), the span values read from lane g * ROWS + rr: -1 outside the span or the texture. KIND 0:
-// perspective, 1: linear tc, 3: triangle (upper0 = y0 - first row - rows of the lower part: row rr
-// is in the upper part when upper0 + rr >= 0; its u / v steps d0 / d1 per part).
-template <int KIND, int ROWS>
-SW_DEV void span_texel_indices(int32_t (&tix)[ROWS], uint32_t gmask, int g, const SpanRec& mine, int32_t x, uint32_t tw,
-	uint32_t th, int32_t upper0, int32_t d0u, int32_t d0l, int32_t d1u, int32_t d1l)
+// f(0) .. f(N - 1) with the index a constant in each call, so that the arrays it indexes are registers from
+// the start (indexed by an unrolled loop they were moved as whole register tuples).
+template <int... I, class F>
+SW_DEV void for_each_constant(std::integer_sequence<int, I...>, F&& f)
 {
-#pragma unroll
-	for(int rr = 0; rr < ROWS; ++rr)
-	{
-		if(!(gmask & (1u << rr)))
-			continue;
-		const int sl = g * ROWS + rr;
-		const int32_t sx0 = __builtin_amdgcn_readlane(mine.x0, sl), sx1 = __builtin_amdgcn_readlane(mine.x1, sl);
-		const int32_t j = x - sx0;
-		const bool in = x >= sx0 && x < sx1;
-		int32_t t;
-		if constexpr(KIND == 3)
-		{
-			const bool upper = upper0 + rr >= 0;
-			const int32_t s0 = __builtin_amdgcn_readlane(mine.v[0], sl), s1 = __builtin_amdgcn_readlane(mine.v[1], sl);
-			const uint32_t u = uint32_t(fixed16_floor_to_int(wadd(s0, wmul(j, upper ? d0u : d0l))));
-			const uint32_t v = uint32_t(fixed16_floor_to_int(wadd(s1, wmul(j, upper ? d1u : d1l))));
-			t = u < tw && v < th ? int32_t(u + v * tw) : -1;
-		}
-		else
-		{
-			int32_t sv[6];
-#pragma unroll
-			for(int i = 0; i < (KIND == 0 ? 6 : 4); ++i)
-				sv[i] = __builtin_amdgcn_readlane(mine.v[i], sl);
-			t = polygon_texel_index<KIND>(sv, j, tw, th);
-		}
-		tix[rr] = in ? t : -1;
-	}
+	(f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+SW_DEV void for_each_constant(F&& f)
+{
+	for_each_constant(std::make_integer_sequence<int, N>{}, f);
 }
 
-// The tile's draws are taken 64 at a time in draw order: a ballot bins them, the hits are
-// compacted into the low lanes, which load their draw's parameters at once. Then GD draws at a
-// time (GD * ROWS = 16 (draw, row) items): one lane per item loads its span record, every lane
-// computes the texel address of its pixel for all 16 items, issues the 16 fetches together and
-// blends them in painter's order into its ROWS colours.
-template <class CT, int ROWS, bool SSPAN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(typename CT::T) == 4 && ROWS <= 8 ? 5 : 1)))
+// Span record ITEM of a group in the lanes of its row: 8 dwords of a half of the row's 16 lanes, two records
+// to a register (a row without a record holds zeros: an empty span).
+template <int ITEM, int DWORDS>
+SW_DEV SpanRec row_span(const int32_t (&dwords)[DWORDS])
+{
+	constexpr int first = ITEM % 2 * 8;
+	const int32_t v = dwords[ITEM / 2];
+	return SpanRec{row_lane<first>(v), row_lane<first + 1>(v),
+		{row_lane<first + 2>(v), row_lane<first + 3>(v), row_lane<first + 4>(v), row_lane<first + 5>(v), row_lane<first + 6>(v),
+			row_lane<first + 7>(v)}};
+}
+
+// One draw's texels of a tile: unit (rs, k) is the 16 x 4 pixels at columns 16 k, rows 4 rs of the tile, and
+// the lane its pixel of every unit. The draw's span records are items FIRST + rs of dwords. Sets ok[unit] to
+// the lanes whose pixel lies in the span and its texel in the texture (0 for a unit that no span meets), and
+// tix[unit] to those texels' indices (0 in the unit's other lanes, unset where ok is 0).
+// KIND 0: perspective (rasterizer.rs:425-452), 1: linear texture coordinates (line-z :559-579, affine
+// :705-727), 3: triangle (:1223-1240; d0, d1: the row's u and v steps). The interpolants step by 16 pixels
+// from unit to unit with additions (integers that wrap, so the sums equal the products).
+// Inside a span the record's clamps keep inv_z in [2^8, 2^29] and tc at 0 or above, so z's divisor is in
+// [1, 2^21] and the products below are unsigned; outside it the values are dropped.
+template <int KIND, int RS, int NK, int FIRST, int DWORDS>
+SW_DEV void unit_texel_indices(const int32_t (&dwords)[DWORDS], int32_t x, uint32_t tw, uint32_t th,
+	const int32_t (&d0)[RS], const int32_t (&d1)[RS], uint32_t (&tix)[RS * NK], uint64_t (&ok)[RS * NK])
+{
+	for_each_constant<RS>([&](auto rs_c) __attribute__((always_inline)) {
+		constexpr int rs = rs_c;
+		const SpanRec rec = row_span<FIRST + rs>(dwords);
+		const uint32_t len = uint32_t(rec.x1 - rec.x0);
+		int32_t j = wadd(x, -rec.x0);
+		const int32_t s0 = KIND == 3 ? d0[rs] : KIND == 0 ? rec.v[3] : rec.v[1];
+		const int32_t s1 = KIND == 3 ? d1[rs] : KIND == 0 ? rec.v[5] : rec.v[3];
+		int32_t t0 = wadd(KIND == 0 ? rec.v[2] : rec.v[0], wmul(j, s0));
+		int32_t t1 = wadd(KIND == 0 ? rec.v[4] : KIND == 3 ? rec.v[1] : rec.v[2], wmul(j, s1));
+		int32_t iz = KIND == 0 ? wadd(rec.v[0], wmul(j, rec.v[1])) : 0;
+		for_each_constant<NK>([&](auto k_c) __attribute__((always_inline)) {
+			constexpr int k = k_c, unit = rs * NK + k;
+			const uint64_t in = lanes_of(uint32_t(j) < len);
+			uint64_t unit_ok = 0;
+			if(in != 0)
+			{
+				uint32_t u, v;
+				if(KIND == 0)
+				{
+					// (1 << Z_CALC_SHIFT) / div (lanes outside the span take a divisor of the fast quotient),
+					// then (z * tc) >> TC_FINAL_SHIFT (34) from the product's upper half
+					uint32_t div = lane_in(in) ? uint32_t(iz) >> INV_Z_PRE_SHIFT : 2048u;
+					uint32_t z = swdiv::z_from_rcp_near(div, SWDIV_RCP(float(div)));
+					if(lanes_of(div < 2048u) != 0)
+					{
+						// far spans only; the empty asm keeps the compiler from computing this ahead of the branch
+						one_value(div);
+						z = div < 2048u ? swdiv::z_from_inv_z(div ? div : 1u) : z;
+					}
+					u = __umulhi(z, uint32_t(t0)) >> (TC_FINAL_SHIFT - 32);
+					v = __umulhi(z, uint32_t(t1)) >> (TC_FINAL_SHIFT - 32);
+				}
+				else
+				{
+					u = uint32_t(t0 >> 16);
+					v = uint32_t(t1 >> 16);
+				}
+				unit_ok = in & lanes_of(u < tw) & lanes_of(v < th);
+				tix[unit] = lane_in(unit_ok) ? u + (v & 0xFFFFFFu) * (tw & 0xFFFFFFu) : 0u; // tw, th <= 65536
+			}
+			ok[unit] = unit_ok;
+			if(k + 1 < NK)
+			{
+				j = wadd(j, 16);
+				t0 = wadd(t0, wmul(s0, 16));
+				t1 = wadd(t1, wmul(s1, 16));
+				if(KIND == 0)
+					iz = wadd(iz, wmul(rec.v[1], 16));
+			}
+		});
+	});
+}
+
+// The tile's draws are taken 64 at a time in draw order: a ballot bins them, the hits are compacted into the
+// low lanes, which load their draw's parameters at once. Then GD draws at a time (four units of 16 x 4 pixels
+// together in narrow tiles): the span records of the tile's rows, requested one group ahead (from the bounds,
+// so without waiting for the draws' parameters), give the texel addresses of the units that the spans meet;
+// their fetches are issued together and blended in painter's order into the pixels' colours.
+//
+// A wave works on 16 x 4 pixels per instruction: a span record is broadcast to its row's lanes by DPP (a
+// 64 x 1 strip per instruction took eight readlanes per strip), the interpolants step with additions, the
+// draw's kind and blend are tested once per draw instead of once per row, and a unit that no span meets
+// costs one compare, where polygons' edges leave most of a 64-pixel strip empty. Against those strips
+// (best span load mode of each): 1920 x 1080 11.1 us from 13.6, 2560 x 1440 Color64 with 64 models and 256
+// decals 37.4 from 48.4, 256 views of 1.08e8 pixels 273 from 384, 13 views in Color64 24.1 from 32.6. Bound
+// by instruction issue (82% of the cycles issue VALU on the 256 views); tiles with hundreds of small
+// triangles wait for one texel fetch per draw. Worse: eight or sixteen units together (registers), all
+// bounds' ballots before the first draw, the next draw's texel addresses during a fetch (registers, moves).
+template <class CT, int ROWS, int NK>
+__global__ __launch_bounds__(256)
 void k_raster_tiles(MapPtrs m, const DrawBounds* __restrict__ bounds,
 	const DrawRec* __restrict__ drec, const PartRec* __restrict__ parts, const SpanRec* __restrict__ spans,
 	const ViewsArg views, const typename CT::T* __restrict__ arena, const typename CT::T* __restrict__ skybox,
 	typename CT::T* __restrict__ fb, uint32_t total_tiles, const uint32_t* __restrict__ counters)
 {
 	typedef typename CT::T C;
-	constexpr int GD = ROWS >= 16 ? 1 : 16 / ROWS;
-	// wave-uniform (readfirstlane): the tile, its view and every per-item value derived from them
+	constexpr int RS = ROWS / 4, UNITS = RS * NK, WIDTH = 16 * NK;
+	constexpr int GD = UNITS < 4 ? 4 / UNITS : 1;
+	constexpr int DWORDS = (GD * RS + 1) / 2;
+	// wave-uniform (readfirstlane): the tile, its view and every per-draw value derived from them
 	// stay scalar, so the uniform tests below are scalar branches
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
 	const uint32_t t = blockIdx.x * 4 + wave;
@@ -2237,469 +2291,222 @@ void k_raster_tiles(MapPtrs m, const DrawBounds* __restrict__ bounds,
 	// the error flag is read now and tested before the first span record is read (span records may
 	// be incomplete after an overflow), so its latency overlaps the tile's first loads
 	const uint32_t err = counters[COUNTER_ERROR];
-	uint32_t lo = 0, hi = views.count;
-	while(hi - lo > 1)
+	// the tile's view: the last one starting at or before it, a probe per lane and level
+	uint32_t lo = 0;
+	for(uint32_t n = views.count; n > 1;)
 	{
-		const uint32_t mid = (lo + hi) >> 1;
-		if(views[mid].first_tile <= t)
-			lo = mid;
-		else
-			hi = mid;
+		const uint32_t step = (n + 63u) / 64u, probe = lo + lane * step;
+		const uint64_t le = lanes_of(lane * step < n && views[probe].first_tile <= t);
+		const uint32_t last = le ? 63u - uint32_t(__builtin_clzll(le)) : 0u;
+		lo += last * step;
+		n = std::min(step, n - last * step);
 	}
 	const ViewExt& ve = views[lo];
 	const uint32_t local = t - ve.first_tile;
 	const uint32_t band = local / ve.cols;
 	const uint32_t col = local - band * ve.cols;
-	const int32_t x0 = int32_t(col * 64);
+	const int32_t x0 = int32_t(col * WIDTH);
 	const int32_t y0 = int32_t(band * ROWS);
 	const int32_t W = int32_t(ve.v.width), H = int32_t(ve.v.height);
-	const int32_t x = x0 + int32_t(lane);
+	const int32_t x = x0 + int32_t(lane & 15u), y = y0 + int32_t(lane >> 4); // the lane's pixel of unit (0, 0)
 	C* vfb = fb + ve.v.fb_offset;
 	const C bg = C(ve.v.background_color);
 
-	C acc[ROWS];
-#pragma unroll
-	for(int r = 0; r < ROWS; ++r)
-	{
-		const int32_t y = y0 + r;
+	C acc[UNITS];
+	for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+		const int32_t px = x + 16 * (u % NK), py = y + 4 * (u / NK);
 		C c = bg;
-		if(!ve.v.clear_background && x < W && y < H)
-			c = vfb[uint64_t(y) * uint32_t(W) + uint32_t(x)];
-		acc[r] = c;
-	}
+		if(!ve.v.clear_background && px < W && py < H)
+			c = vfb[uint64_t(uint32_t(py)) * uint32_t(W) + uint32_t(px)];
+		acc[u] = c;
+	});
 
 	const uint32_t first_draw = ve.v.first_draw, num_draws = ve.v.num_draws;
 	const uint64_t lanes_below = (1ull << lane) - 1ull;
+	// the bounds of the next 64 draws, loaded ahead of the test of the current ones
+	auto load_bounds = [&](uint32_t base) __attribute__((always_inline)) {
+		return base + lane < num_draws ? bounds[first_draw + base + lane] : DrawBounds{1, 0, 1, 0, 0, 0};
+	};
+	DrawBounds next_b = load_bounds(0);
 	for(uint32_t base = 0; base < num_draws; base += 64)
 	{
 		// ordered binning: lane i tests draw base + i against this tile
 		const uint32_t di = first_draw + base + lane;
-		bool hit = false;
-		DrawBounds b = DrawBounds{1, 0, 1, 0, 0, 0};
-		if(base + lane < num_draws)
-		{
-			b = bounds[di];
-			hit = b.row_min < y0 + ROWS && b.row_max > y0 && b.x_min < x0 + 64 && b.x_max > x0;
-		}
+		const DrawBounds b = next_b;
+		if(base + 64 < num_draws)
+			next_b = load_bounds(base + 64);
+		const bool hit = b.row_min < y0 + ROWS && b.row_max > y0 && b.x_min < x0 + WIDTH && b.x_max > x0;
 		const uint64_t mask = __ballot(hit);
 		if(!mask)
 			continue;
+		if(err & ERROR_SPAN_OVERFLOW)
+			return; // the host runs the batch again with room for every span record
 		const uint32_t nh = uint32_t(__popcll(mask));
 		// compact the hits into lanes 0 .. nh - 1, in draw order (a permutation of the lanes); the
 		// hits' full records are loaded by those lanes
 		const uint32_t dst = hit ? uint32_t(__popcll(mask & lanes_below)) : nh + uint32_t(__popcll(~mask & lanes_below));
 		const uint32_t h_di = uint32_t(lane_push(int32_t(di), dst));
-		// With 4-row tiles in the vector span mode, the span records of the first 16 / ROWS hits are
-		// loaded now, from the bounds, while the hits' full records are loaded below: lane L takes
-		// draw L / ROWS at tile row L % ROWS, for a row whose span is not empty (inside the records).
-		constexpr bool PREFETCH = !SSPAN && ROWS == 4;
-		SpanRec next_span = SpanRec{0, 0, {0, 0, 0, 0, 0, 0}};
-		bool next_ok = false;
-		int32_t b_span_base = 0, b_row_first = 0, b_rmin = 1, b_rmax = 0;
-		if constexpr(PREFETCH)
-		{
-			b_span_base = lane_push(int32_t(b.span_base), dst);
-			b_row_first = lane_push(b.row_first, dst);
-			b_rmin = lane_push(int32_t(b.row_min), dst);
-			b_rmax = lane_push(int32_t(b.row_max), dst);
-			if(err & ERROR_SPAN_OVERFLOW)
-				return; // the host runs the batch again with room for every span record
-		}
-		auto load_group_spans_b = [&](uint32_t kgp, SpanRec& out) -> bool {
-			const uint32_t kq = (kgp + lane / ROWS) & 63u;
-			const int32_t y = y0 + int32_t(lane % ROWS);
-			const int32_t q_base = lane_pull(b_span_base, kq);
-			const int32_t q_first = lane_pull(b_row_first, kq);
-			const int32_t q_min = lane_pull(b_rmin, kq), q_max = lane_pull(b_rmax, kq);
-			if(lane < uint32_t(GD * ROWS) && kgp + lane / ROWS < nh && y >= q_min && y < q_max)
-			{
-				out = spans[uint32_t(q_base) + uint32_t(y - q_first)];
-				return true;
-			}
-			return false;
+		const int32_t h_span_base = lane_push(int32_t(b.span_base), dst);
+		const int32_t h_row_first = lane_push(b.row_first, dst);
+		const int32_t h_rows = lane_push(int32_t(uint32_t(uint16_t(b.row_min)) | (uint32_t(uint16_t(b.row_max)) << 16)), dst);
+		// The span records of the tile's rows for the group of draws from hit kg on, a dword per lane: the
+		// 16 lanes of a row hold two records of 8 dwords (of two row sets, or with 4-row tiles of two draws),
+		// so a record is read once and costs half a register until its values are broadcast over the row's
+		// lanes. Rows without one give 0 (an empty span).
+		auto load_group = [&](uint32_t kg, int32_t (&dwords)[DWORDS]) __attribute__((always_inline)) {
+			for_each_constant<DWORDS>([&](auto d) __attribute__((always_inline)) {
+				constexpr int g = 2 * d / RS, rs0 = 2 * d % RS;
+				uint32_t k = kg + uint32_t(g);
+				int32_t yr = y + 4 * rs0, rows, row_first, span_base;
+				if(RS == 1)
+				{
+					k += GD > 1 ? (lane >> 3) & 1u : 0u;
+					rows = lane_pull(h_rows, k & 63u);
+					row_first = lane_pull(h_row_first, k & 63u);
+					span_base = lane_pull(h_span_base, k & 63u);
+				}
+				else
+				{
+					yr += int32_t((lane >> 1) & 4u);
+					const uint32_t ku = std::min(k, nh - 1u);
+					rows = rl(h_rows, ku);
+					row_first = rl(h_row_first, ku);
+					span_base = rl(h_span_base, ku);
+				}
+				int32_t v = 0;
+				if(k < nh && yr >= int32_t(int16_t(rows)) && yr < (rows >> 16))
+					v = reinterpret_cast<const int32_t*>(spans + uint32_t(span_base))[uint32_t(yr - row_first) * 8u + (lane & 7u)];
+				dwords[d] = v;
+			});
 		};
-		if constexpr(PREFETCH)
-			next_ok = load_group_spans_b(0, next_span);
+		int32_t next_dwords[DWORDS];
+		load_group(0, next_dwords);
 		DrawRec r{};
 		if(lane < nh)
 			r = drec[h_di];
-		// per-draw parameters, one hit per lane: all in the record, except a triangle's two parts'
-		// steps
-		const int32_t h_row_first = r.row_first;
-		const int32_t h_rows = int32_t(r.rows);
-		const int32_t h_span_base = int32_t(r.span_base);
+		// per-draw parameters, one hit per lane
 		const int32_t h_rows0 = int32_t(r.rows0);
-		const int32_t h_kind = int32_t((r.stat >> DRAW_STAT_KIND_SHIFT) & 3u);
-		const int32_t h_blend = int32_t((r.stat >> DRAW_STAT_BLEND_SHIFT) & 15u);
-		const int32_t h_tw = int32_t(r.tex_w);
-		const int32_t h_th = int32_t(r.tex_h);
+		const int32_t h_stat = int32_t(r.stat);
+		const int32_t h_size = int32_t((r.tex_w - 1u) | ((r.tex_h - 1u) << 16)); // sizes are 1 .. 65536
 		const uint64_t tex = (r.stat & DRAW_STAT_TRIANGLE) ? reinterpret_cast<uint64_t>(m.lite + r.tex_offset)
 			: (r.stat & DRAW_STAT_SKYBOX)                  ? reinterpret_cast<uint64_t>(skybox + r.tex_offset)
 			: (r.stat & DRAW_STAT_PORTAL)                  ? reinterpret_cast<uint64_t>(static_cast<const C*>(m.portal) + r.tex_offset)
 														   : reinterpret_cast<uint64_t>(arena + r.tex_offset);
 		const int32_t h_tex_lo = int32_t(uint32_t(tex));
 		const int32_t h_tex_hi = int32_t(uint32_t(tex >> 32));
-		int32_t pd[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-		if(lane < nh && h_kind == 3)
-		{
-			const PartRec& p0 = parts[h_di * MAX_PARTS_PER_DRAW];
-			const PartRec& p1 = parts[h_di * MAX_PARTS_PER_DRAW + 1];
-#pragma unroll
-			for(int i = 0; i < 5; ++i)
-			{
-				pd[i] = p0.d[i];
-				pd[5 + i] = p1.d[i];
-			}
-		}
 
-		if(err & ERROR_SPAN_OVERFLOW)
-			return; // the host runs the batch again with room for every span record
-		// Lane L < GD * ROWS loads the span record of draw kg + L / ROWS at tile row L % ROWS
-		// (non-SSPAN mode). With 4-row tiles the next group's records are loaded while the current
-		// group's texels are fetched, so each group after the first waits for one memory round
-		// trip, not two (taller tiles have no registers to spare for the second set of records).
-		auto load_group_spans = [&](uint32_t kgp, SpanRec& out) -> bool {
-			const uint32_t kq = (kgp + lane / ROWS) & 63u;
-			const int32_t q_row = y0 + int32_t(lane % ROWS) - lane_pull(h_row_first, kq);
-			const int32_t q_rows = lane_pull(h_rows, kq);
-			const int32_t q_base = lane_pull(h_span_base, kq);
-			if(lane < uint32_t(GD * ROWS) && kgp + lane / ROWS < nh && q_row >= 0 && q_row < q_rows)
-			{
-				out = spans[uint32_t(q_base) + uint32_t(q_row)];
-				return true;
-			}
-			return false;
-		};
 		for(uint32_t kg = 0; kg < nh; kg += GD)
 		{
-			if constexpr(!SSPAN)
-			{
-				// Each lane tests whether its record's span meets the tile; the ballot of the tests
-				// names the active items, and only those are walked (scalar bit tests), their
-				// values read from the item's lane. Texels of the lanes outside a span are fetched
-				// at index 0 of the same texture (in bounds) and discarded by a select, so the
-				// fetches and blends change no execution mask.
-				SpanRec mine = SpanRec{0, 0, {0, 0, 0, 0, 0, 0}};
-				bool act = false;
-				if constexpr(PREFETCH)
+			int32_t dwords[DWORDS];
+			for_each_constant<DWORDS>([&](auto d) __attribute__((always_inline)) { dwords[d] = next_dwords[d]; });
+			if(kg + GD < nh)
+				load_group(kg + GD, next_dwords);
+			uint32_t tix[GD][UNITS];
+			uint64_t ok[GD][UNITS];
+			int32_t light[GD][RS][3], light_step[GD][RS][3]; // triangles: the lane's light in unit k = 0, its step per pixel
+			for_each_constant<GD * UNITS>([&](auto i) __attribute__((always_inline)) { any_value(tix[i / UNITS][i % UNITS]); });
+			for_each_constant<GD * RS * 3>([&](auto i) __attribute__((always_inline)) {
+				any_value(light[i / (RS * 3)][i / 3 % RS][i % 3]);
+				any_value(light_step[i / (RS * 3)][i / 3 % RS][i % 3]);
+			});
+			for_each_constant<GD>([&](auto g) __attribute__((always_inline)) {
+				const uint32_t k = std::min(kg + uint32_t(g), nh - 1u);
+				const uint32_t kind = (uint32_t(rl(h_stat, k)) >> DRAW_STAT_KIND_SHIFT) & 3u;
+				const uint32_t size = uint32_t(rl(h_size, k)), tw = (size & 0xFFFFu) + 1u, th = (size >> 16) + 1u;
+				int32_t d0[RS], d1[RS];
+				if(kind == 0)
+					unit_texel_indices<0, RS, NK, g * RS>(dwords, x, tw, th, d0, d1, tix[g], ok[g]);
+				else if(kind == 3)
 				{
-					if(next_ok)
-						mine = next_span;
-					act = next_ok;
-					next_ok = false;
-					if(kg + GD < nh)
-						next_ok = load_group_spans_b(kg + GD, next_span);
+					// the steps of the triangle's two parts (scalar loads: the draw is uniform)
+					const PartRec* p = parts + uint32_t(rl(int32_t(h_di), k)) * MAX_PARTS_PER_DRAW;
+					const int32_t upper0 = y - rl(h_row_first, k) - rl(h_rows0, k); // >= 0: unit row 0's pixel is in the upper part
+					for_each_constant<RS>([&](auto rs) __attribute__((always_inline)) {
+						const bool upper = upper0 + 4 * rs >= 0;
+						d0[rs] = upper ? p[1].d[0] : p[0].d[0];
+						d1[rs] = upper ? p[1].d[1] : p[0].d[1];
+						const SpanRec rec = row_span<g * RS + rs>(dwords);
+						const int32_t j = wadd(x, -rec.x0);
+						for_each_constant<3>([&](auto c) __attribute__((always_inline)) {
+							light_step[g][rs][c] = upper ? p[1].d[2 + c] : p[0].d[2 + c];
+							light[g][rs][c] = wadd(rec.v[2 + c], wmul(j, light_step[g][rs][c]));
+						});
+					});
+					unit_texel_indices<3, RS, NK, g * RS>(dwords, x, tw, th, d0, d1, tix[g], ok[g]);
 				}
 				else
-					act = load_group_spans(kg, mine);
-				act = act && mine.x0 < mine.x1 && mine.x1 > x0 && mine.x0 < x0 + 64;
-				const uint64_t amask = __ballot(act);
-				if(amask == 0)
-					continue;
-				int32_t tix[GD][ROWS];
-				C texel[GD][ROWS];
-#pragma unroll
-				for(int g = 0; g < GD; ++g)
-				{
-					const uint32_t gmask = uint32_t(amask >> (g * ROWS)) & ((1u << ROWS) - 1u);
-#pragma unroll
-					for(int rr = 0; rr < ROWS; ++rr)
+					unit_texel_indices<1, RS, NK, g * RS>(dwords, x, tw, th, d0, d1, tix[g], ok[g]);
+			});
+			// the group's fetches, in flight together
+			C texel[GD][UNITS];
+			for_each_constant<GD>([&](auto g) __attribute__((always_inline)) {
+				const uint32_t k = std::min(kg + uint32_t(g), nh - 1u);
+				const GlobalBytes ktex = (GlobalBytes)(uint64_t(uint32_t(rl(h_tex_lo, k))) | (uint64_t(uint32_t(rl(h_tex_hi, k))) << 32));
+				const bool lite = sizeof(C) != 4 && (uint32_t(rl(h_stat, k)) & DRAW_STAT_TRIANGLE) != 0;
+				for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+					any_value(texel[g][u]);
+					if(ok[g][u] != 0)
 					{
-						tix[g][rr] = -1;
-						texel[g][rr] = 0;
-					}
-					if(gmask == 0)
-						continue;
-					const uint32_t k = kg + uint32_t(g); // below nh: the draw has an active item
-					const int32_t kind = rl(h_kind, k);
-					const uint32_t tw = uint32_t(rl(h_tw, k)), th = uint32_t(rl(h_th, k));
-					// the draw's kind is tested once, the rows below are straight-line code
-					if(kind == 0)
-						span_texel_indices<0, ROWS>(tix[g], gmask, g, mine, x, tw, th, 0, 0, 0, 0, 0);
-					else if(kind == 3)
-						span_texel_indices<3, ROWS>(tix[g], gmask, g, mine, x, tw, th, y0 - rl(h_row_first, k) - rl(h_rows0, k),
-							rl(pd[5], k), rl(pd[0], k), rl(pd[6], k), rl(pd[1], k));
-					else
-						span_texel_indices<1, ROWS>(tix[g], gmask, g, mine, x, tw, th, 0, 0, 0, 0, 0);
-				}
-				// every span value is read before the fetches are issued, so all of the group's
-				// fetches are in flight together
-#pragma unroll
-				for(int g = 0; g < GD; ++g)
-				{
-					const uint32_t gmask = uint32_t(amask >> (g * ROWS)) & ((1u << ROWS) - 1u);
-					if(gmask == 0)
-						continue;
-					const uint32_t k = kg + uint32_t(g);
-					const uint64_t tex = uint64_t(uint32_t(rl(h_tex_lo, k))) | (uint64_t(uint32_t(rl(h_tex_hi, k))) << 32);
-					if(rl(h_kind, k) == 3)
-					{
-#pragma unroll
-						for(int rr = 0; rr < ROWS; ++rr)
-							if(gmask & (1u << rr))
-								texel[g][rr] = C(global_at<uint32_t>(tex, tix[g][rr] < 0 ? 0 : tix[g][rr]));
-					}
-					else
-					{
-#pragma unroll
-						for(int rr = 0; rr < ROWS; ++rr)
-							if(gmask & (1u << rr))
-								texel[g][rr] = global_at<C>(tex, tix[g][rr] < 0 ? 0 : tix[g][rr]);
-					}
-				}
-#pragma unroll
-				for(int g = 0; g < GD; ++g)
-				{
-					const uint32_t gmask = uint32_t(amask >> (g * ROWS)) & ((1u << ROWS) - 1u);
-					if(gmask == 0)
-						continue;
-					const uint32_t k = kg + uint32_t(g);
-					const uint32_t blend = uint32_t(rl(h_blend, k));
-					if(rl(h_kind, k) != 3)
-					{
-						if(blend == SW_BLEND_NONE)
-						{
-#pragma unroll
-							for(int rr = 0; rr < ROWS; ++rr)
-								if(gmask & (1u << rr))
-									acc[rr] = tix[g][rr] >= 0 ? texel[g][rr] : acc[rr];
-						}
+						// index * size < 2^32: textures hold at most 2^29 texels (the draw validation)
+						if(lite)
+							texel[g][u] = *(const __attribute__((address_space(1))) uint32_t*)(ktex + tix[g][u] * 4u);
 						else
-						{
-#pragma unroll
-							for(int rr = 0; rr < ROWS; ++rr)
-							{
-								if(!(gmask & (1u << rr)))
-									continue;
-								const C nc = write_into_framebuffer<CT>(blend, acc[rr], texel[g][rr]);
-								acc[rr] = tix[g][rr] >= 0 ? nc : acc[rr];
-							}
-						}
-						continue;
+							texel[g][u] = *(const __attribute__((address_space(1))) C*)(ktex + tix[g][u] * uint32_t(sizeof(C)));
 					}
-					const int32_t part_row0 = rl(h_row_first, k), rows0 = rl(h_rows0, k);
-					const int32_t dr_u = rl(pd[7], k), dr_l = rl(pd[2], k);
-					const int32_t dg_u = rl(pd[8], k), dg_l = rl(pd[3], k);
-					const int32_t db_u = rl(pd[9], k), db_l = rl(pd[4], k);
-#pragma unroll
-					for(int rr = 0; rr < ROWS; ++rr)
-					{
-						if(!(gmask & (1u << rr)))
-							continue;
-						const int sl = g * ROWS + rr;
-						const bool upper = y0 + rr - part_row0 >= rows0;
-						const int32_t j = x - rl(mine.x0, sl);
-						const int32_t lr = wadd(rl(mine.v[2], sl), wmul(j, upper ? dr_u : dr_l));
-						const int32_t lg = wadd(rl(mine.v[3], sl), wmul(j, upper ? dg_u : dg_l));
-						const int32_t lb = wadd(rl(mine.v[4], sl), wmul(j, upper ? db_u : db_l));
-						const uint32_t tv = uint32_t(texel[g][rr]);
-						const CI tc = Color32T::to_ci(tv);
-						const CI lit = CI{wmul(tc.b, lb) >> 16, wmul(tc.g, lg) >> 16, wmul(tc.r, lr) >> 16, 0};
-						const C dst_c = acc[rr];
-						C nc = dst_c;
-						switch(blend)
-						{
-						case SW_BLEND_NONE: nc = CT::from_ci(lit); break;
-						case SW_BLEND_AVERAGE: nc = CT::average(dst_c, CT::from_ci(lit)); break;
-						case SW_BLEND_ADDITIVE: nc = CT::saturated_sum(dst_c, CT::from_ci(lit)); break;
-						case SW_BLEND_ALPHA_TEST: nc = Color32T::test_alpha(tv) ? CT::from_ci(lit) : dst_c; break;
-						case SW_BLEND_ALPHA_BLEND: nc = alpha_blend_ci<CT>(dst_c, lit, Color32T::get_alpha(tv)); break;
-						default: break;
-						}
-						acc[rr] = tix[g][rr] >= 0 ? nc : dst_c;
-					}
-				}
-				continue;
-			}
-			// Span records of the group's 16 items. SSPAN: each item's record is loaded through the
-			// scalar unit into SGPRs when the item is processed. Otherwise lane L < GD * ROWS loads
-			// the record of draw kg + L / ROWS at tile row L % ROWS and items read them with
-			// readlane (fewer, wider loads; better where many distinct records are in flight).
-			SpanRec mine = SpanRec{0, 0, {0, 0, 0, 0, 0, 0}};
-			if constexpr(!SSPAN)
-			{
-				const uint32_t kq = (kg + lane / ROWS) & 63u;
-				const int32_t q_row = y0 + int32_t(lane % ROWS) - lane_pull(h_row_first, kq);
-				const int32_t q_rows = lane_pull(h_rows, kq);
-				const int32_t q_base = lane_pull(h_span_base, kq);
-				if(lane < uint32_t(GD * ROWS) && kg + lane / ROWS < nh && q_row >= 0 && q_row < q_rows)
-					mine = spans[uint32_t(q_base) + uint32_t(q_row)];
-			}
-			int32_t tix[GD][ROWS];
-#pragma unroll
-			for(int g = 0; g < GD; ++g)
-			{
-				const uint32_t k = kg + uint32_t(g);
-				const uint32_t kk = k < nh ? k : 0u;
-				const int32_t kind = rl(h_kind, kk);
-				const uint32_t tw = uint32_t(rl(h_tw, kk)), th = uint32_t(rl(h_th, kk));
-				const int32_t part_row0 = rl(h_row_first, kk), rows0 = rl(h_rows0, kk);
-				const int32_t nrows = rl(h_rows, kk), span_base = rl(h_span_base, kk);
-#pragma unroll
-				for(int rr = 0; rr < ROWS; ++rr)
+				});
+			});
+			for_each_constant<GD>([&](auto g) __attribute__((always_inline)) {
+				const uint32_t k = std::min(kg + uint32_t(g), nh - 1u);
+				const uint32_t stat = uint32_t(rl(h_stat, k)), blend = (stat >> DRAW_STAT_BLEND_SHIFT) & 15u;
+				if(!(stat & DRAW_STAT_TRIANGLE))
 				{
-					// every value of the item is uniform over the wave, its span record is loaded
-					// through the scalar unit straight into SGPRs, and every branch below is a
-					// scalar one; the lane's own span test only masks the result
-					const int32_t q = y0 + rr - part_row0;
-					const int sl = g * ROWS + rr;
-					int32_t ti = -1;
-					SpanRec sp = SpanRec{0, 0, {0, 0, 0, 0, 0, 0}};
-					bool row_ok;
-					if constexpr(SSPAN)
-					{
-						row_ok = k < nh && q >= 0 && q < nrows;
-						if(row_ok)
-							sp = spans[uint32_t(span_base) + uint32_t(q)];
-					}
+					if(blend == SW_BLEND_NONE)
+						for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+							if(ok[g][u] != 0)
+								acc[u] = lane_in(ok[g][u]) ? texel[g][u] : acc[u];
+						});
 					else
-					{
-						row_ok = k < nh;
-						sp.x0 = rl(mine.x0, sl);
-						sp.x1 = rl(mine.x1, sl);
-					}
-					if(row_ok)
-					{
-						const int32_t sx0 = sp.x0, sx1 = sp.x1;
-						if(sx0 < sx1 && sx1 > x0 && sx0 < x0 + 64)
-						{
-							if constexpr(!SSPAN)
+						for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+							if(ok[g][u] != 0)
 							{
-#pragma unroll
-								for(int i = 0; i < 6; ++i)
-									sp.v[i] = rl(mine.v[i], sl);
+								const C nc = write_into_framebuffer<CT>(blend, acc[u], texel[g][u]);
+								acc[u] = lane_in(ok[g][u]) ? nc : acc[u];
 							}
-							const int32_t* sv = sp.v;
-							const int32_t j = x - sx0;
-							const bool in = x >= sx0 && x < sx1;
-							if(kind == 3)
-							{
-								const bool upper = q >= rows0;
-								const int32_t d0u = rl(pd[5], kk), d0l = rl(pd[0], kk);
-								const int32_t d1u = rl(pd[6], kk), d1l = rl(pd[1], kk);
-								const int32_t d0 = upper ? d0u : d0l, d1 = upper ? d1u : d1l;
-								const uint32_t u = uint32_t(fixed16_floor_to_int(wadd(sv[0], wmul(j, d0))));
-								const uint32_t v = uint32_t(fixed16_floor_to_int(wadd(sv[1], wmul(j, d1))));
-								ti = in && u < tw && v < th ? int32_t(u + v * tw) : -1;
-							}
-							else if(kind == 0)
-							{
-								const int32_t t = polygon_texel_index<0>(sv, j, tw, th);
-								ti = in ? t : -1;
-							}
-							else
-							{
-								const int32_t t = polygon_texel_index<1>(sv, j, tw, th);
-								ti = in ? t : -1;
-							}
-						}
-					}
-					tix[g][rr] = ti;
+						});
+					return;
 				}
-			}
-
-			C texel[GD][ROWS];
-#pragma unroll
-			for(int g = 0; g < GD; ++g)
-			{
-				const uint32_t k = kg + uint32_t(g);
-				const uint32_t kk = k < nh ? k : 0u;
-				const bool tri = rl(h_kind, kk) == 3;
-				const uint64_t tex = uint64_t(uint32_t(rl(h_tex_lo, kk))) | (uint64_t(uint32_t(rl(h_tex_hi, kk))) << 32);
-#pragma unroll
-				for(int rr = 0; rr < ROWS; ++rr)
-				{
-					C tv = 0;
-					if(tix[g][rr] >= 0)
-						tv = tri ? C(global_at<uint32_t>(tex, tix[g][rr])) : global_at<C>(tex, tix[g][rr]);
-					texel[g][rr] = tv;
-				}
-			}
-
-#pragma unroll
-			for(int g = 0; g < GD; ++g)
-			{
-				const uint32_t k = kg + uint32_t(g);
-				if(k >= nh)
-					continue;
-				const uint32_t blend = uint32_t(rl(h_blend, k));
-				if(rl(h_kind, k) != 3)
-				{
-#pragma unroll
-					for(int rr = 0; rr < ROWS; ++rr)
-						if(tix[g][rr] >= 0)
-							acc[rr] = write_into_framebuffer<CT>(blend, acc[rr], texel[g][rr]);
-					continue;
-				}
-				const int32_t part_row0 = rl(h_row_first, k), rows0 = rl(h_rows0, k);
-				const int32_t nrows = rl(h_rows, k), span_base = rl(h_span_base, k);
-				const int32_t dr_u = rl(pd[7], k), dr_l = rl(pd[2], k);
-				const int32_t dg_u = rl(pd[8], k), dg_l = rl(pd[3], k);
-				const int32_t db_u = rl(pd[9], k), db_l = rl(pd[4], k);
-#pragma unroll
-				for(int rr = 0; rr < ROWS; ++rr)
-				{
-					const int32_t q = y0 + rr - part_row0;
-					if(q < 0 || q >= nrows)
-						continue; // no span in this row (so no texel either)
-					const bool upper = q >= rows0;
-					int32_t sx0, l0, l1, l2;
-					if constexpr(SSPAN)
-					{
-						const SpanRec sp = spans[uint32_t(span_base) + uint32_t(q)]; // scalar load, cached
-						sx0 = sp.x0;
-						l0 = sp.v[2];
-						l1 = sp.v[3];
-						l2 = sp.v[4];
-					}
-					else
-					{
-						const int sl = g * ROWS + rr;
-						sx0 = rl(mine.x0, sl);
-						l0 = rl(mine.v[2], sl);
-						l1 = rl(mine.v[3], sl);
-						l2 = rl(mine.v[4], sl);
-					}
-					if(tix[g][rr] < 0)
-						continue;
-					const int32_t j = x - sx0;
-					const int32_t dr = upper ? dr_u : dr_l;
-					const int32_t dg = upper ? dg_u : dg_l;
-					const int32_t db = upper ? db_u : db_l;
-					const int32_t lr = wadd(l0, wmul(j, dr));
-					const int32_t lg = wadd(l1, wmul(j, dg));
-					const int32_t lb = wadd(l2, wmul(j, db));
-					const uint32_t tv = uint32_t(texel[g][rr]);
+				for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+					if(ok[g][u] == 0)
+						return;
+					constexpr int rs = u / NK, k16 = 16 * (u % NK);
+					const int32_t lr = wadd(light[g][rs][0], wmul(light_step[g][rs][0], k16));
+					const int32_t lg = wadd(light[g][rs][1], wmul(light_step[g][rs][1], k16));
+					const int32_t lb = wadd(light[g][rs][2], wmul(light_step[g][rs][2], k16));
+					const uint32_t tv = uint32_t(texel[g][u]);
 					const CI tc = Color32T::to_ci(tv);
 					const CI lit = CI{wmul(tc.b, lb) >> 16, wmul(tc.g, lg) >> 16, wmul(tc.r, lr) >> 16, 0};
-					C& dst_c = acc[rr];
+					const C dst_c = acc[u];
+					C nc = dst_c;
 					switch(blend)
 					{
-					case SW_BLEND_NONE: dst_c = CT::from_ci(lit); break;
-					case SW_BLEND_AVERAGE: dst_c = CT::average(dst_c, CT::from_ci(lit)); break;
-					case SW_BLEND_ADDITIVE: dst_c = CT::saturated_sum(dst_c, CT::from_ci(lit)); break;
-					case SW_BLEND_ALPHA_TEST:
-						if(Color32T::test_alpha(tv))
-							dst_c = CT::from_ci(lit);
-						break;
-					case SW_BLEND_ALPHA_BLEND: dst_c = alpha_blend_ci<CT>(dst_c, lit, Color32T::get_alpha(tv)); break;
+					case SW_BLEND_NONE: nc = CT::from_ci(lit); break;
+					case SW_BLEND_AVERAGE: nc = CT::average(dst_c, CT::from_ci(lit)); break;
+					case SW_BLEND_ADDITIVE: nc = CT::saturated_sum(dst_c, CT::from_ci(lit)); break;
+					case SW_BLEND_ALPHA_TEST: nc = Color32T::test_alpha(tv) ? CT::from_ci(lit) : dst_c; break;
+					case SW_BLEND_ALPHA_BLEND: nc = alpha_blend_ci<CT>(dst_c, lit, Color32T::get_alpha(tv)); break;
 					default: break;
 					}
-				}
-			}
+					acc[u] = lane_in(ok[g][u]) ? nc : dst_c;
+				});
+			});
 		}
 	}
 
-	if(x < W)
-	{
-#pragma unroll
-		for(int r = 0; r < ROWS; ++r)
-		{
-			const int32_t y = y0 + r;
-			if(y < H) // non-temporal: the finished tile is not read again by this kernel
-				__builtin_nontemporal_store(acc[r], &vfb[uint64_t(y) * uint32_t(W) + uint32_t(x)]);
-		}
-	}
+	for_each_constant<UNITS>([&](auto u) __attribute__((always_inline)) {
+		const int32_t px = x + 16 * (u % NK), py = y + 4 * (u / NK);
+		if(px < W && py < H) // non-temporal: the finished tile is not read again by this kernel
+			__builtin_nontemporal_store(acc[u], &vfb[uint64_t(uint32_t(py)) * uint32_t(W) + uint32_t(px)]);
+	});
 }
 
 // =============================================================================================
@@ -3163,48 +2970,40 @@ void launch_build_surfaces(hipStream_t st, uint32_t color_bits, const MapPtrs& m
 	}
 }
 
-template <class CT, bool SSPAN>
-static void launch_raster_ct(hipStream_t st, uint32_t tile_rows, const MapPtrs& m, const DrawBounds* bounds, const DrawRec* drec,
-	const PartRec* parts, const SpanRec* spans, const ViewsArg& views, const void* arena, const void* skybox,
+// The tile sizes of raster_tile_width (sw_runtime.hip): at most 512 pixels.
+template <class CT>
+static void launch_raster_ct(hipStream_t st, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m, const DrawBounds* bounds,
+	const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views, const void* arena, const void* skybox,
 	void* fb, uint32_t total_tiles, const uint32_t* counters)
 {
 	typedef typename CT::T C;
 	const uint32_t blocks = (total_tiles + 3) / 4;
 	if(blocks == 0)
 		return;
-	const C* a = static_cast<const C*>(arena);
-	const C* sky = static_cast<const C*>(skybox);
-	C* out = static_cast<C*>(fb);
+	auto launch = [&](auto kernel) {
+		timed_launch(kernel, dim3(blocks), dim3(256), 0, st, m, bounds, drec, parts, spans, views, static_cast<const C*>(arena),
+			static_cast<const C*>(skybox), static_cast<C*>(fb), total_tiles, counters);
+	};
 	if(tile_rows == 4)
-		timed_launch(k_raster_tiles<CT, 4, SSPAN>, dim3(blocks), dim3(256), 0, st, m, bounds, drec, parts, spans, views,
-			a, sky, out, total_tiles, counters);
+		tile_width == 64   ? launch(k_raster_tiles<CT, 4, 4>)
+		: tile_width == 32 ? launch(k_raster_tiles<CT, 4, 2>)
+						   : launch(k_raster_tiles<CT, 4, 1>);
 	else if(tile_rows == 8)
-		timed_launch(k_raster_tiles<CT, 8, SSPAN>, dim3(blocks), dim3(256), 0, st, m, bounds, drec, parts, spans, views,
-			a, sky, out, total_tiles, counters);
+		tile_width == 64   ? launch(k_raster_tiles<CT, 8, 4>)
+		: tile_width == 32 ? launch(k_raster_tiles<CT, 8, 2>)
+						   : launch(k_raster_tiles<CT, 8, 1>);
 	else
-		timed_launch(k_raster_tiles<CT, 16, SSPAN>, dim3(blocks), dim3(256), 0, st, m, bounds, drec, parts, spans, views,
-			a, sky, out, total_tiles, counters);
+		tile_width == 32 ? launch(k_raster_tiles<CT, 16, 2>) : launch(k_raster_tiles<CT, 16, 1>);
 }
 
-void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, bool scalar_spans, const MapPtrs& m,
+void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
 	const DrawBounds* bounds, const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views,
 	const void* arena, const void* skybox, void* fb, uint32_t total_tiles, const uint32_t* counters)
 {
 	if(color_bits == 64)
-	{
-		if(scalar_spans)
-			launch_raster_ct<Color64T, true>(st, tile_rows, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles,
-				counters);
-		else
-			launch_raster_ct<Color64T, false>(st, tile_rows, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles,
-				counters);
-	}
-	else if(scalar_spans)
-		launch_raster_ct<Color32T, true>(st, tile_rows, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles,
-			counters);
+		launch_raster_ct<Color64T>(st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
 	else
-		launch_raster_ct<Color32T, false>(st, tile_rows, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles,
-			counters);
+		launch_raster_ct<Color32T>(st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
 }
 
 void launch_finish(hipStream_t st, const DrawRec* drec, uint32_t nd, uint32_t* counters, uint32_t* result)

@@ -81,7 +81,7 @@ struct sw_ctx
 	uint32_t num_shadows = 0; // sw_set_light_shadows: entries in `shadows`
 	const float* shadow_texels = nullptr;
 	uint32_t tile_rows = 8; // raster tile height (SW_TILE_ROWS_*), set by sw_set_tile_rows / the autotuner
-	bool scalar_spans = true; // raster span records through the scalar unit (chosen by the autotuner)
+	bool scalar_spans = true; // sw_set_scalar_spans
 	uint32_t* counters_host = nullptr; // pinned, device-mapped: result block (k_finish), then the error words
 	float* noalloc_scratch = nullptr; // this device's address of `scratch`
 	const void* portal_texels = nullptr; // sw_set_portal_textures (plain path)
@@ -125,7 +125,7 @@ struct sw_ctx
 		uint64_t arena_texels = 0;
 		void* arena = nullptr;
 		void* fb = nullptr;
-		uint32_t total_tiles = 0;
+		uint32_t total_tiles = 0, tile_width = 64; // of the raster (raster_tile_width)
 		uint32_t max_view_height = 0;
 		const void* portal = nullptr; // textures of SW_TEXSRC_PORTAL draws
 		uint64_t num_portal = 0;
@@ -334,13 +334,36 @@ void collect_timings(sw_ctx* ctx)
 	ctx->pending.clear();
 }
 
+// Raster tile width for views of this size: a wave takes 256 pixels, 512 once that still makes 128 waves per
+// SIMD (binning costs a wave the same for either), and fewer while the chip gets less than four waves per
+// SIMD, since a tile then waits alone for its loads. Measured raster times (us) at 64 / 32 / 16 pixels of
+// width: 640 x 400 in 4 rows (1,000 tiles at 64) 8.7 / 6.8 / 6.5; 1920 x 1080 in 4 rows (8,100) 11.1 / 15.2 / -,
+// in 8 rows 13.5 / 11.6 / 15.7; 2560 x 1440 Color64 in 8 rows 53.8 / 39.7 / -; 13 views in 8 rows (62,000 tiles
+// of 256 pixels) 29.2 / 25.3 / -; 256 views in 8 rows (421,000) 273 / 341 / -.
+uint32_t raster_tile_width(const sw_view* views, uint32_t n, uint32_t tile_rows)
+{
+	auto tiles = [&](uint32_t width) {
+		uint64_t t = 0;
+		for(uint32_t i = 0; i < n; ++i)
+			t += uint64_t((views[i].width + width - 1) / width) * ((views[i].height + tile_rows - 1) / tile_rows);
+		return t;
+	};
+	uint32_t width = std::min(512u / tile_rows, 64u);
+	if(width * tile_rows > 256u && tiles(width / 2) < 128u * NUM_SIMDS)
+		width /= 2;
+	while(width > 16u && tiles(width) < 4u * NUM_SIMDS)
+		width /= 2;
+	return width;
+}
+
 // Per-view tiling of a batch (views are always host memory).
 int build_view_ext(sw_ctx* ctx, const sw_view* views, uint32_t n, uint64_t arena_texels, std::vector<ViewExt>& out,
-	uint32_t& total_tiles, uint32_t* max_height = nullptr)
+	uint32_t& total_tiles, uint32_t& tile_width, uint32_t* max_height = nullptr)
 {
 	if(max_height)
 		*max_height = 0;
 	const uint32_t tile_rows = ctx->tile_rows;
+	tile_width = raster_tile_width(views, n, tile_rows);
 	out.resize(n);
 	uint64_t tiles = 0;
 	uint32_t next_surface = 0, next_draw = 0;
@@ -359,7 +382,7 @@ int build_view_ext(sw_ctx* ctx, const sw_view* views, uint32_t n, uint64_t arena
 		if(max_height)
 			*max_height = std::max(*max_height, v.height);
 		e.num_bands = (v.height + tile_rows - 1) / tile_rows;
-		e.cols = (v.width + 63) / 64;
+		e.cols = (v.width + tile_width - 1) / tile_width;
 		e.first_tile = uint32_t(tiles);
 		e.pad = 0;
 		// a view's surfaces, and the arena texels its draws read, lie in [its offset, the next
@@ -531,7 +554,7 @@ int launch_stages(sw_ctx* ctx, const sw_ctx::Launch& L, bool surfaces, bool rast
 	{
 		{
 			StageTimer t(ctx, STAGE_RASTER);
-			swk::launch_raster_tiles(ctx->stream, L.color_bits, ctx->tile_rows, ctx->scalar_spans, mp,
+			swk::launch_raster_tiles(ctx->stream, L.color_bits, ctx->tile_rows, L.tile_width, mp,
 				static_cast<DrawBounds*>(ctx->dbounds.p),
 				static_cast<DrawRec*>(ctx->drec.p), static_cast<PartRec*>(ctx->parts.p), static_cast<SpanRec*>(ctx->spans.p),
 				ctx->views_arg, L.arena, L.color_bits == 64 ? map->sky64.p : map->sky32.p, L.fb, L.total_tiles, counters);
@@ -750,7 +773,7 @@ int launch_frame(sw_ctx* ctx, uint32_t num_draws, uint64_t num_vertex_ints, bool
 	std::vector<ViewExt> ve;
 	sw_ctx::Launch& L = ctx->last;
 	L = sw_ctx::Launch{};
-	if((r = build_view_ext(ctx, &v, 1, ctx->frame_arena_texels, ve, L.total_tiles, &L.max_view_height)))
+	if((r = build_view_ext(ctx, &v, 1, ctx->frame_arena_texels, ve, L.total_tiles, L.tile_width, &L.max_view_height)))
 		return r;
 	L.surface_mode = SURF_SEARCH;
 	if((r = set_views(ctx, ve, true)))
@@ -2109,7 +2132,7 @@ static int prepare_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_
 	if(b->color_bits != 32 && b->color_bits != 64)
 		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "color_bits must be 32 or 64");
 	int r;
-	if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, L.total_tiles, &L.max_view_height)))
+	if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, L.total_tiles, L.tile_width, &L.max_view_height)))
 		return r;
 	if((r = validate_views_fit(ctx, ve, b->framebuffer_texels, b->num_surfaces, b->num_draws)))
 		return r;
@@ -2256,7 +2279,6 @@ int sw_render_batch_graph(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out
 	mix(uint64_t(uintptr_t(b->portal_texels)));
 	mix(b->num_portal_texels);
 	mix(ctx->tile_rows);
-	mix(ctx->scalar_spans ? 1 : 0);
 	for(uint32_t i = 0; i < b->num_views; ++i)
 	{
 		mix(b->views[i].width);
@@ -2327,8 +2349,8 @@ int sw_render_batch_graph(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out
 		// the captured kernels read the views from the device array: refresh it (camera
 		// positions, framebuffer offsets and clear flags may change between replays)
 		std::vector<ViewExt> ve;
-		uint32_t tiles = 0;
-		if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, tiles)) ||
+		uint32_t tiles = 0, tile_width = 0;
+		if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, tiles, tile_width)) ||
 			(r = validate_views_fit(ctx, ve, b->framebuffer_texels, b->num_surfaces, b->num_draws)) ||
 			(r = set_views(ctx, ve, false)))
 			return r;
@@ -2359,11 +2381,7 @@ int sw_set_scalar_spans(sw_ctx* ctx, uint32_t enable)
 {
 	if(!ctx)
 		return SW_ERR_INVALID_ARGUMENT;
-	if((enable != 0) != ctx->scalar_spans)
-	{
-		ctx->scalar_spans = enable != 0;
-		ctx->graph_key = 0;
-	}
+	ctx->scalar_spans = enable != 0;
 	return SW_OK;
 }
 
@@ -2385,17 +2403,14 @@ int sw_autotune_batches(sw_ctx* ctx, sw_map* map, const sw_batch* batches, uint3
 		r = hip_check(ctx, hipEventCreate(&e1), "hipEventCreate");
 	double best_ms = 0.0;
 	uint32_t best = ctx->tile_rows;
-	bool best_scalar = ctx->scalar_spans;
 	const bool profiling = ctx->profiling;
 	ctx->profiling = false;
-	// every tile height with both ways of loading span records, each timed over all the batches
-	// (median of five rounds); out_ms keeps each height's better mode, per batch
-	for(uint32_t c = 0; c < 2 * SW_TILE_ROWS_COUNT && !r; ++c)
+	// every tile height timed over all the batches (median of five rounds)
+	for(uint32_t c = 0; c < SW_TILE_ROWS_COUNT && !r; ++c)
 	{
-		const uint32_t rows = candidates[c / 2];
+		const uint32_t rows = candidates[c];
 		if((r = sw_set_tile_rows(ctx, rows)))
 			break;
-		ctx->scalar_spans = (c & 1) != 0;
 		// one untimed pass sizes the buffers
 		for(uint32_t i = 0; i < num_batches && !r; ++i)
 			r = sw_render_batch(ctx, map, &batches[i], out_fb);
@@ -2416,13 +2431,12 @@ int sw_autotune_batches(sw_ctx* ctx, sw_map* map, const sw_batch* batches, uint3
 			break;
 		std::sort(t, t + ROUNDS);
 		const double ms = double(t[ROUNDS / 2]) / num_batches;
-		if(out_ms && ((c & 1) == 0 || ms < out_ms[c / 2]))
-			out_ms[c / 2] = ms;
+		if(out_ms)
+			out_ms[c] = ms;
 		if(c == 0 || ms < best_ms)
 		{
 			best_ms = ms;
 			best = rows;
-			best_scalar = ctx->scalar_spans;
 		}
 	}
 	ctx->profiling = profiling;
@@ -2431,11 +2445,6 @@ int sw_autotune_batches(sw_ctx* ctx, sw_map* map, const sw_batch* batches, uint3
 	if(e1)
 		(void)hipEventDestroy(e1);
 	const int r2 = sw_set_tile_rows(ctx, best);
-	if(ctx->scalar_spans != best_scalar)
-	{
-		ctx->scalar_spans = best_scalar;
-		ctx->graph_key = 0;
-	}
 	if(out_rows)
 		*out_rows = best;
 	return r ? r : r2;

@@ -34,6 +34,8 @@ def lib():
     lib.sweep_z.argtypes = [C.c_uint32, C.c_uint32]
     lib.sweep_z_rcp_perturbed.restype = u64
     lib.sweep_z_rcp_perturbed.argtypes = [C.c_uint32, C.c_uint32, C.c_int32]
+    lib.sweep_z_near_perturbed.restype = u64
+    lib.sweep_z_near_perturbed.argtypes = [C.c_uint32, C.c_uint32, C.c_int32]
     for n in ("check_fixed16_div", "check_div_rcp", "check_mod_rcp", "check_z_from_inv_z"):
         getattr(lib, n).restype = None
     return lib
@@ -107,3 +109,9 @@ def test_z_fast_branch_tolerates_an_inexact_reciprocal(lib):
     v_rcp_f32, within 1 ulp); with the reciprocal off by up to 2 ulp either way its one correction
     step still lands on 2^31 / div for every divisor."""
     assert lib.sweep_z_rcp_perturbed(1024, (1 << 24) - 1, 2) == 0
+
+
+def test_z_of_near_spans_tolerates_an_inexact_reciprocal(lib):
+    """The raster kernel's form (2048 <= div < 2^22): one upward step from a start half a unit low, exact with
+    the reciprocal off by up to 3 ulp either way."""
+    assert lib.sweep_z_near_perturbed(2048, (1 << 22) - 1, 3) == 0
