@@ -218,9 +218,10 @@ struct BloomArgs
 	uint32_t w, h;
 	uint32_t bw, bh, scale_log2; // bloom buffer size, scale 2^scale_log2 (1..3)
 	int32_t radius; // blur radius (0: no blur)
-	uint64_t* buf0; // bloom buffer (downscaled, then blurred)
-	uint64_t* buf1; // horizontal pass output
-	int32_t* line_sums; // 4 per bloom row: the row's sum of averages, lanes B, G, R, A (16-byte aligned)
+	uint64_t* buf0; // bloom buffer, downscaled
+	uint64_t* buf1; // bloom buffer, blurred (radius > 0)
+	int32_t* line_sums; // 4 per part of a bloom row: its sum of averages, lanes B, G, R, A (16-byte aligned)
+	uint32_t line_parts; // parts of a bloom row, 512 source pixels each
 	float* average; // 4 floats: the average colour, lanes B, G, R, A (host memory)
 	int32_t k1[BLOOM_KERNEL], k2[BLOOM_KERNEL]; // integer weights of the two passes (scale 2^14)
 	float inv_scale[3]; // tonemap 1 / (exposure * modulate), lanes B, G, R

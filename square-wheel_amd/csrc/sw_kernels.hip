@@ -2529,54 +2529,64 @@ SW_DEV CI ci_add(CI a, CI b) { return CI{wadd(a.b, b.b), wadd(a.g, b.g), wadd(a.
 SW_DEV CI ci_mul(CI a, int32_t s) { return CI{wmul(a.b, s), wmul(a.g, s), wmul(a.r, s), wmul(a.a, s)}; }
 SW_DEV CI ci_shr(CI a, int k) { return CI{a.b >> k, a.g >> k, a.r >> k, a.a >> k}; }
 
-// downscale_hdr_buffer (:805-853): one block per bloom row. Each bloom texel is the integer average
-// of its scale x scale source pixels ((sum * (256 / scale^2)) >> 8, packed with unsigned
-// saturation); the block also sums the row's averages (integers, so any order is exact).
+// Two pixels of 8 bytes (rows of odd width start at multiples of 8 bytes, which the 16-byte loads allow).
+typedef uint64_t PixelPair __attribute__((ext_vector_type(2), aligned(8)));
+typedef uint32_t ColorPair __attribute__((ext_vector_type(2), aligned(4)));
+
+// downscale_hdr_buffer (:805-853). Each bloom texel is the integer average of its S x S source pixels
+// ((sum * (256 / S^2)) >> 8, packed with unsigned saturation); a block leaves the sum of its texels' averages
+// for its part of the row (integers, so any order is exact).
+// A lane takes two pixels of each of the S rows in one load and the S / 2 lanes of a texel add up by DPP, so
+// every load is 16 bytes next to its neighbours'. Bound by memory: 2557 x 1439 to 1278 x 719 (36.8 MB) 9.9 us
+// with a thread per texel -> 8.5 (4.3 TB/s).
 template <uint32_t S>
 __global__ __launch_bounds__(256) void k_bloom_downscale(BloomArgs a)
 {
-	const uint32_t dy = blockIdx.x;
-	const int32_t scaler = (1 << 8) / int32_t(S * S);
-	const uint64_t* __restrict__ src = a.hdr + uint64_t(dy * S) * a.w;
-	uint64_t* __restrict__ dst = a.buf0 + uint64_t(dy) * a.bw;
-	CI line = CI{0, 0, 0, 0};
-#pragma unroll 2
-	for(uint32_t dx = threadIdx.x; dx < a.bw; dx += blockDim.x)
-	{
-		CI sum = CI{0, 0, 0, 0};
+	const uint32_t i = blockIdx.x * 256u + threadIdx.x, dx = i / (S / 2), dy = blockIdx.y;
+	const bool in = dx < a.bw;
+	const uint64_t* __restrict__ src = a.hdr + uint64_t(dy * S) * a.w + (in ? 2u * i : 0u);
+	PixelPair v[S];
 #pragma unroll
-		for(uint32_t y = 0; y < S; ++y)
+	for(uint32_t y = 0; y < S; ++y)
+		v[y] = *reinterpret_cast<const PixelPair*>(src + uint64_t(y) * a.w);
+	CI sum = CI{0, 0, 0, 0};
 #pragma unroll
-			for(uint32_t x = 0; x < S; ++x)
-				sum = ci_add(sum, Color64T::to_ci(src[uint64_t(y) * a.w + dx * S + x]));
-		const CI average = ci_shr(ci_mul(sum, scaler), 8);
-		dst[dx] = Color64T::from_ci(average);
-		line = ci_add(line, average);
-	}
-	__shared__ int32_t red[4][4];
-	int32_t v[4] = {line.b, line.g, line.r, line.a};
+	for(uint32_t y = 0; y < S; ++y)
+		sum = ci_add(sum, ci_add(Color64T::to_ci(v[y].x), Color64T::to_ci(v[y].y)));
+	int32_t line[4] = {sum.b, sum.g, sum.r, sum.a};
 #pragma unroll
 	for(int k = 0; k < 4; ++k)
-		for(int off = 32; off > 0; off >>= 1)
-			v[k] = wadd(v[k], __shfl_xor(v[k], off));
+	{
+		if(S >= 4)
+			line[k] += __builtin_amdgcn_update_dpp(0, line[k], 0xB1, 0xF, 0xF, false); // quad_perm 1 0 3 2
+		if(S >= 8)
+			line[k] += __builtin_amdgcn_update_dpp(0, line[k], 0x4E, 0xF, 0xF, false); // quad_perm 2 3 0 1
+		line[k] = wmul(line[k], (1 << 8) / int32_t(S * S)) >> 8;
+	}
+	const bool texel = in && i % (S / 2) == 0;
+	if(texel)
+		a.buf0[uint64_t(dy) * a.bw + dx] = Color64T::from_ci(CI{line[0], line[1], line[2], line[3]});
+	__shared__ int32_t red[4][4];
 	const uint32_t wave = threadIdx.x >> 6;
-	if((threadIdx.x & 63) == 0)
-		for(int k = 0; k < 4; ++k)
-			red[wave][k] = v[k];
+#pragma unroll
+	for(int k = 0; k < 4; ++k)
+	{
+		line[k] = texel ? line[k] : 0;
+		for(int off = 32; off > 0; off >>= 1)
+			line[k] = wadd(line[k], __shfl_xor(line[k], off));
+		if((threadIdx.x & 63) == 0)
+			red[wave][k] = line[k];
+	}
 	__syncthreads();
 	if(threadIdx.x < 4)
-	{
-		int32_t t = 0;
-		for(uint32_t w = 0; w < (blockDim.x + 63) / 64; ++w)
-			t = wadd(t, red[w][threadIdx.x]);
-		a.line_sums[dy * 4 + threadIdx.x] = t;
-	}
+		a.line_sums[(dy * gridDim.x + blockIdx.x) * 4 + threadIdx.x] =
+			wadd(wadd(red[0][threadIdx.x], red[1][threadIdx.x]), wadd(red[2][threadIdx.x], red[3][threadIdx.x]));
 }
 
 // The average colour (:838-852): the rows' integer sums converted and added in row order, then
 // scaled by 1 / (bloom texels). Float addition is not associative, so each lane is one sequential
-// sum, like the reference's; the block converts chunks of rows into LDS in parallel (one 16-byte
-// load per row) and four threads (one per lane) add them up in order. `a.average` is host memory.
+// sum, like the reference's; the block adds up and converts chunks of rows into LDS in parallel and
+// four threads (one per lane) add them up in order. `a.average` is host memory.
 #define BLOOM_AVG_CHUNK 512u
 SW_DEV void bloom_average_block(const BloomArgs& a)
 {
@@ -2589,7 +2599,13 @@ SW_DEV void bloom_average_block(const BloomArgs& a)
 		const uint32_t n = min(BLOOM_AVG_CHUNK, a.bh - y0);
 		for(uint32_t i = threadIdx.x; i < n; i += blockDim.x)
 		{
-			const int4 l = line_sums[y0 + i];
+			int4 l = make_int4(0, 0, 0, 0);
+#pragma unroll 4
+			for(uint32_t p = 0; p < a.line_parts; ++p)
+			{
+				const int4 v = line_sums[uint64_t(y0 + i) * a.line_parts + p];
+				l = make_int4(wadd(l.x, v.x), wadd(l.y, v.y), wadd(l.z, v.z), wadd(l.w, v.w));
+			}
 			rows[i] = make_float4(float(l.x), float(l.y), float(l.z), float(l.w));
 		}
 		__syncthreads();
@@ -2606,136 +2622,249 @@ SW_DEV void bloom_average_block(const BloomArgs& a)
 		a.average[lane] = sum * (1.0f / float(a.bw * a.bh));
 }
 
-__global__ __launch_bounds__(256) void k_bloom_average(BloomArgs a) { bloom_average_block(a); }
-
-// perform_blur_impl (:855-937), one pass: pass 0 horizontal (buf0 -> buf1, weights k1), pass 1
-// vertical (buf1 -> buf0, weights k2 = k1 scaled by bloom_scale); edge texels repeat (clamped
-// coordinates); integer weights at scale 2^14, arithmetic shift, unsigned-saturating pack.
-// Grid: x over the row in blocks of BLUR_PX * 256 texels (BLUR_PX per thread, their taps loaded
-// together), y = bloom row. with_average: block (0, 0), dispatched first, also computes the
-// average colour (pass 0 only; it reads the line sums the downscale left).
-#define BLUR_PX 2
-__global__ __launch_bounds__(256) void k_bloom_blur(BloomArgs a, uint32_t pass, uint32_t with_average)
+// perform_blur_impl (:855-937), both passes: horizontal (weights k1), then vertical (k2 = k1 scaled by
+// bloom_scale); edge texels repeat (clamped coordinates); integer weights at scale 2^14, arithmetic shift,
+// unsigned-saturating pack to 16 bits after each.
+// A block blurs 32 x 32 texels: their surroundings (RP >= radius texels to each side) are staged in LDS by
+// channel, two neighbours to a dword, so that a tap pair is one dot product of 16-bit pairs (weights and
+// texels are below 2^16, their sums below 2^30: the weights add up to 2^14 at most). An output at an odd
+// position takes the same dwords as its even neighbour with the weights shifted by one. The horizontal pass
+// writes its results as vertical pairs over the staged texels, for the vertical pass to read alike.
+// Two kernels with a thread per texel, four shift / add / multiply chains to a tap pair, took at 2560 x 1440
+// 2 x 20.7 us with radius 12 of 1278 x 719 texels, 2 x 8.3 with radius 1 of 1280 x 720; now 13.5 and 7.2
+// (a block's loads, dot products and stores follow each other and all blocks are on the chip at once).
+struct BlurWeights
 {
-	if(with_average && blockIdx.x == 0 && blockIdx.y == 0)
-		bloom_average_block(a);
-	const uint32_t y = blockIdx.y;
-	const int32_t R = a.radius;
-	const int32_t* k = pass == 0 ? a.k1 : a.k2;
-	const uint64_t* __restrict__ src = pass == 0 ? a.buf0 : a.buf1;
-	uint64_t* __restrict__ dst = pass == 0 ? a.buf1 : a.buf0;
-	const int32_t last = pass == 0 ? int32_t(a.bw) - 1 : int32_t(a.bh) - 1;
-	CI sum[BLUR_PX];
-	uint32_t xs[BLUR_PX];
+	uint32_t even[2][BLOOM_MAX_RADIUS + 1], odd[2][BLOOM_MAX_RADIUS + 1]; // [pass][pair]
+};
+constexpr uint32_t BLUR_TILE = 32;
+
+SW_DEV uint32_t dot2_u16(uint32_t a, uint32_t b, uint32_t c)
+{
+	typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
+	return __builtin_amdgcn_udot2(__builtin_bit_cast(U16x2, a), __builtin_bit_cast(U16x2, b), c, false);
+}
+
+SW_DEV uint32_t blur_pack(uint32_t lo, uint32_t hi) { return min(lo >> 14, 65535u) | (min(hi >> 14, 65535u) << 16); }
+
+template <int RP>
+__global__ __launch_bounds__(256) void k_bloom_blur(BloomArgs a, const BlurWeights w)
+{
+	constexpr uint32_t T = BLUR_TILE, ROWS = T + 2 * RP, PAIRS = T / 2 + RP;
+	// dwords to a row: two rows are 16 banks apart (of 32), four lanes of a row read 16 bytes each
+	constexpr uint32_t PITCH = RP > 8 ? 40 : 24, PLANE = ROWS * PITCH, MID_PITCH = T, MID_PLANE = ROWS / 2 * MID_PITCH;
+	static_assert(PITCH >= PAIRS && MID_PLANE <= PLANE);
+	__shared__ __align__(16) uint32_t lds[4 * PLANE];
+	const int32_t x0 = int32_t(blockIdx.x * T) - RP, y0 = int32_t(blockIdx.y * T) - RP;
+	const int32_t last_x = int32_t(a.bw) - 1, last_y = int32_t(a.bh) - 1;
+	constexpr uint32_t STAGE = (ROWS * PAIRS + 255) / 256;
+	PixelPair t[STAGE];
 #pragma unroll
-	for(int j = 0; j < BLUR_PX; ++j)
+	for(uint32_t s = 0; s < STAGE; ++s)
 	{
-		// out-of-row threads work on the row's last texel and store nothing
-		xs[j] = min(blockIdx.x * (256u * BLUR_PX) + uint32_t(j) * 256u + threadIdx.x, a.bw - 1);
-		const int32_t c = pass == 0 ? int32_t(xs[j]) : int32_t(y);
-		const uint64_t v = pass == 0 ? src[uint64_t(y) * a.bw + uint32_t(c)] : src[uint64_t(c) * a.bw + xs[j]];
-		sum[j] = ci_mul(Color64T::to_ci(v), k[R]);
+		const uint32_t i = min(s * 256u + threadIdx.x, ROWS * PAIRS - 1), r = i / PAIRS, p = i - r * PAIRS;
+		const uint64_t* row = a.buf0 + uint64_t(uint32_t(imin32(imax32(y0 + int32_t(r), 0), last_y))) * a.bw;
+		const int32_t x = x0 + 2 * int32_t(p);
+		if(x >= 0 && x < last_x)
+			t[s] = *reinterpret_cast<const PixelPair*>(row + x);
+		else
+			t[s] = row[x < 0 ? 0 : last_x]; // the edge texel, or the last column of an odd width and its repetition
 	}
-	for(int32_t d = 1; d <= R; ++d)
-	{
-		const int32_t w = k[d + R];
 #pragma unroll
-		for(int j = 0; j < BLUR_PX; ++j)
+	for(uint32_t s = 0; s < STAGE; ++s)
+	{
+		const uint32_t i = s * 256u + threadIdx.x, r = i / PAIRS, p = i - r * PAIRS;
+		if(i >= ROWS * PAIRS)
+			break;
+		uint32_t* d = lds + r * PITCH + p;
+		const uint32_t bg0 = uint32_t(t[s].x), bg1 = uint32_t(t[s].y), ra0 = uint32_t(t[s].x >> 32), ra1 = uint32_t(t[s].y >> 32);
+		d[0 * PLANE] = (bg0 & 0xFFFFu) | (bg1 << 16);
+		d[1 * PLANE] = (bg0 >> 16) | (bg1 & 0xFFFF0000u);
+		d[2 * PLANE] = (ra0 & 0xFFFFu) | (ra1 << 16);
+		d[3 * PLANE] = (ra0 >> 16) | (ra1 & 0xFFFF0000u);
+	}
+	__syncthreads();
+	// horizontal: an item is 8 texels of two rows of a channel
+	constexpr uint32_t ITEMS = ROWS / 2 * (T / 8) * 4, H = (ITEMS + 255) / 256;
+	uint32_t mid[H][8];
+#pragma unroll
+	for(uint32_t s = 0; s < H; ++s)
+	{
+		const uint32_t i = s * 256u + threadIdx.x, xg = i % (T / 8), rp = i / (T / 8) % (ROWS / 2), ch = i / (T / 8) / (ROWS / 2);
+		if(i >= ITEMS)
+			break;
+		uint32_t acc[2][8];
+#pragma unroll
+		for(uint32_t k = 0; k < 2; ++k)
 		{
-			const int32_t c = pass == 0 ? int32_t(xs[j]) : int32_t(y);
-			const int32_t p0 = imax32(c - d, 0), p1 = imin32(c + d, last);
-			uint64_t v0, v1;
-			if(pass == 0)
-			{
-				v0 = src[uint64_t(y) * a.bw + uint32_t(p0)];
-				v1 = src[uint64_t(y) * a.bw + uint32_t(p1)];
-			}
-			else
-			{
-				v0 = src[uint64_t(p0) * a.bw + xs[j]];
-				v1 = src[uint64_t(p1) * a.bw + xs[j]];
-			}
-			sum[j] = ci_add(sum[j], ci_mul(ci_add(Color64T::to_ci(v0), Color64T::to_ci(v1)), w));
-		}
-	}
+			const uint4* d4 = reinterpret_cast<const uint4*>(lds + ch * PLANE + (2 * rp + k) * PITCH + 4 * xg);
+			constexpr uint32_t N4 = (RP + 4 + 3) / 4;
+			uint32_t d[4 * N4];
 #pragma unroll
-	for(int j = 0; j < BLUR_PX; ++j)
+			for(uint32_t q = 0; q < N4; ++q)
+			{
+				const uint4 v = d4[q];
+				d[4 * q] = v.x;
+				d[4 * q + 1] = v.y;
+				d[4 * q + 2] = v.z;
+				d[4 * q + 3] = v.w;
+			}
+#pragma unroll
+			for(uint32_t m = 0; m < 4; ++m)
+			{
+				uint32_t e = 0, o = 0;
+#pragma unroll
+				for(uint32_t j = 0; j <= RP; ++j)
+				{
+					e = dot2_u16(d[m + j], w.even[0][j], e);
+					o = dot2_u16(d[m + j], w.odd[0][j], o);
+				}
+				acc[k][2 * m] = e;
+				acc[k][2 * m + 1] = o;
+			}
+		}
+#pragma unroll
+		for(uint32_t m = 0; m < 8; ++m)
+			mid[s][m] = blur_pack(acc[0][m], acc[1][m]);
+	}
+	__syncthreads();
+#pragma unroll
+	for(uint32_t s = 0; s < H; ++s)
 	{
-		const uint32_t x = blockIdx.x * (256u * BLUR_PX) + uint32_t(j) * 256u + threadIdx.x;
-		if(x < a.bw)
-			dst[uint64_t(y) * a.bw + x] = Color64T::from_ci(ci_shr(sum[j], 14));
+		const uint32_t i = s * 256u + threadIdx.x, xg = i % (T / 8), rp = i / (T / 8) % (ROWS / 2), ch = i / (T / 8) / (ROWS / 2);
+		if(i >= ITEMS)
+			break;
+		uint4* d4 = reinterpret_cast<uint4*>(lds + ch * MID_PLANE + rp * MID_PITCH + 8 * xg);
+		d4[0] = make_uint4(mid[s][0], mid[s][1], mid[s][2], mid[s][3]);
+		d4[1] = make_uint4(mid[s][4], mid[s][5], mid[s][6], mid[s][7]);
+	}
+	__syncthreads();
+	// vertical: a thread takes four rows of a column, all channels
+	const uint32_t x = threadIdx.x % T, yg = threadIdx.x / T;
+	uint32_t out[4][4]; // [row][channel]
+#pragma unroll
+	for(uint32_t ch = 0; ch < 4; ++ch)
+	{
+		const uint32_t* c = lds + ch * MID_PLANE + 2 * yg * MID_PITCH + x;
+		uint32_t acc[4] = {0, 0, 0, 0};
+#pragma unroll
+		for(uint32_t j = 0; j < RP + 2; ++j)
+		{
+			const uint32_t d = c[j * MID_PITCH];
+#pragma unroll
+			for(uint32_t m = 0; m < 2; ++m)
+				if(j >= m && j - m <= RP)
+				{
+					acc[2 * m] = dot2_u16(d, w.even[1][j - m], acc[2 * m]);
+					acc[2 * m + 1] = dot2_u16(d, w.odd[1][j - m], acc[2 * m + 1]);
+				}
+		}
+#pragma unroll
+		for(uint32_t m = 0; m < 4; ++m)
+			out[m][ch] = acc[m];
+	}
+	const uint32_t ox = blockIdx.x * T + x;
+#pragma unroll
+	for(uint32_t m = 0; m < 4; ++m)
+	{
+		const uint32_t oy = blockIdx.y * T + 4 * yg + m;
+		if(ox < a.bw && oy < a.bh)
+			a.buf1[uint64_t(oy) * a.bw + ox] =
+				uint64_t(blur_pack(out[m][0], out[m][1])) | (uint64_t(blur_pack(out[m][2], out[m][3])) << 32);
 	}
 }
 
-// perform_tonemapping_with_bloom_{nearest,linear} (:346-726), one thread per pixel: the bloom value
-// of the pixel's region (block, border or corner of the reference's loops), added to the pixel,
-// tonemapped.
-// Grid: x over the row in blocks of TM_PX * 256 pixels (TM_PX per thread, their frame loads issued
-// together), y = frame row.
-#define TM_PX 4
+// perform_tonemapping_with_bloom_{nearest,linear} (:346-726): the bloom value of the pixel added to it,
+// tonemapped. The reference's regions (block, borders, corners) are one formula: the bilinear mix with a
+// weight of 0 for what a border or corner leaves out (x * 0 + c and x * 1 + c are exact here: the lanes are
+// finite and not negative).
+// A thread takes 2 x 2 pixels of one bloom cell (cells start at odd coordinates with scale 2 and bilinear
+// upsampling), so the cell's texels, their conversion and the vertical mix are shared; the frame's two pairs
+// of pixels are 16-byte loads. With a thread per pixel, which divided by the scale for its mix, 2557 x 1439
+// took 17.7 us bilinear and 2560 x 1440 11.0 nearest; now 14.5 and 11.3 (bound by the divisions).
+// with_average: the first row of blocks computes the average colour (dispatched first, it ends long before
+// the frame does).
 template <bool LINEAR>
-SW_DEV uint32_t bloom_pixel(const BloomArgs& a, uint32_t x, uint32_t y, CV c)
+__global__ __launch_bounds__(256) void k_bloom_tonemap(BloomArgs a, const uint64_t* __restrict__ bloom, uint32_t with_average)
 {
-	const uint32_t sl = a.scale_log2, S = 1u << sl;
-	auto bl = [&](uint32_t bx, uint32_t by) { return cv_from_color64(a.buf0[uint64_t(by) * a.bw + bx]); };
-	CV sum;
+	if(with_average && blockIdx.y == 0)
+	{
+		if(blockIdx.x == 0)
+			bloom_average_block(a);
+		return;
+	}
+	const uint32_t sl = a.scale_log2, half = 1u << (sl - 1), off = LINEAR && sl == 1 ? 1u : 0u;
+	// the group's first pixel (at -1 with off: that pixel is not stored)
+	const int32_t x0 = int32_t(2u * (blockIdx.x * 256u + threadIdx.x) - off), y0 = int32_t(2u * (blockIdx.y - with_average) - off);
+	if(x0 >= int32_t(a.w))
+		return;
+	const bool in_x[2] = {x0 >= 0, x0 + 1 < int32_t(a.w)};
+	const bool in_y[2] = {y0 >= 0, y0 + 1 < int32_t(a.h)};
+	CV c[2][2];
+#pragma unroll
+	for(int j = 0; j < 2; ++j)
+	{
+		const uint64_t* row = a.hdr + uint64_t(uint32_t(in_y[j] ? y0 + j : y0 + 1 - j)) * a.w;
+		PixelPair v;
+		if(in_x[0] && in_x[1])
+			v = *reinterpret_cast<const PixelPair*>(row + x0);
+		else
+			v = row[in_x[0] ? x0 : x0 + 1];
+		c[j][0] = cv_from_color64(v.x);
+		c[j][1] = cv_from_color64(v.y);
+	}
+	CV sum[2][2];
 	if(!LINEAR)
-		sum = cv_add(bl(std::min(x >> sl, a.bw - 1), std::min(y >> sl, a.bh - 1)), c);
+	{
+		const CV b = cv_from_color64(bloom[uint64_t(std::min(uint32_t(y0) >> sl, a.bh - 1)) * a.bw + std::min(uint32_t(x0) >> sl, a.bw - 1)]);
+#pragma unroll
+		for(int j = 0; j < 2; ++j)
+#pragma unroll
+			for(int i = 0; i < 2; ++i)
+				sum[j][i] = cv_add(b, c[j][i]);
+	}
 	else
 	{
-		const uint32_t half = S / 2;
-		const float sf = float(S);
-		auto mix = [&](uint32_t k) { return float((S + 1) & 1) / (2.0f * sf) + float(k) / sf; };
-		const uint32_t right_x = (a.bw - 1) * S + half, upper_y = (a.bh - 1) * S + half;
-		const bool lower = y < half, upper = y >= upper_y, left = x < half, right = x >= right_x;
-		if((lower || upper) && (left || right))
-			sum = cv_add(bl(left ? 0 : a.bw - 1, lower ? 0 : a.bh - 1), c); // corners
-		else if(lower || upper)
+		// the cell's first texel, and the weights of the second (0 in the borders, which keep to one texel)
+		const float inv_s = __builtin_bit_cast(float, (127u - sl) << 23); // 1 / S
+		auto axis = [&](int32_t p, uint32_t n, uint32_t& t0, uint32_t& t1, float (&m)[2]) {
+			const uint32_t q = uint32_t(p) - half; // huge before the first cell
+			const bool before = int32_t(p + int32_t(off)) < int32_t(half), after = !before && (q >> sl) >= n - 1;
+			t0 = before ? 0u : after ? n - 1 : q >> sl;
+			t1 = before || after ? t0 : t0 + 1;
+#pragma unroll
+			for(uint32_t k = 0; k < 2; ++k)
+				m[k] = before || after ? 0.0f : 0.5f * inv_s + float((q + k) & ((1u << sl) - 1u)) * inv_s;
+		};
+		uint32_t sx0, sx1, sy0, sy1;
+		float mx[2], my[2];
+		axis(x0, a.bw, sx0, sx1, mx);
+		axis(y0, a.bh, sy0, sy1, my);
+		const uint64_t* r0 = bloom + uint64_t(sy0) * a.bw;
+		const uint64_t* r1 = bloom + uint64_t(sy1) * a.bw;
+		const CV b00 = cv_from_color64(r0[sx0]), b10 = cv_from_color64(r0[sx1]);
+		const CV b01 = cv_from_color64(r1[sx0]), b11 = cv_from_color64(r1[sx1]);
+#pragma unroll
+		for(int j = 0; j < 2; ++j)
 		{
-			// lower / upper border: horizontal mix of the first / last bloom row
-			const uint32_t by = lower ? 0 : a.bh - 1;
-			const uint32_t sx = (x - half) >> sl, dx = (x - half) & (S - 1);
-			const float mx = mix(dx);
-			sum = cv_mul_scalar_add(bl(sx, by), 1.0f - mx, cv_mul_scalar_add(bl(sx + 1, by), mx, c));
-		}
-		else
-		{
-			const uint32_t sy = (y - half) >> sl, dy = (y - half) & (S - 1);
-			const float my = mix(dy), omy = 1.0f - my;
-			if(left || right)
-			{
-				const uint32_t bx = left ? 0 : a.bw - 1;
-				sum = cv_add(cv_mul_scalar_add(bl(bx, sy), omy, cv_scalar_mul(bl(bx, sy + 1), my)), c);
-			}
-			else
-			{
-				const uint32_t sx = (x - half) >> sl, dx = (x - half) & (S - 1);
-				const float mx = mix(dx);
-				const CV l = cv_mul_scalar_add(bl(sx, sy), omy, cv_scalar_mul(bl(sx, sy + 1), my));
-				const CV r = cv_mul_scalar_add(bl(sx + 1, sy), omy, cv_scalar_mul(bl(sx + 1, sy + 1), my));
-				sum = cv_mul_scalar_add(l, 1.0f - mx, cv_mul_scalar_add(r, mx, c));
-			}
+			const CV l = cv_mul_scalar_add(b00, 1.0f - my[j], cv_scalar_mul(b01, my[j]));
+			const CV r = cv_mul_scalar_add(b10, 1.0f - my[j], cv_scalar_mul(b11, my[j]));
+#pragma unroll
+			for(int i = 0; i < 2; ++i)
+				sum[j][i] = cv_mul_scalar_add(l, 1.0f - mx[i], cv_mul_scalar_add(r, mx[i], c[j][i]));
 		}
 	}
-	return tonemap_cv(sum, a.inv_scale);
-}
-
-template <bool LINEAR>
-__global__ __launch_bounds__(256) void k_bloom_tonemap(BloomArgs a)
-{
-	const uint32_t y = blockIdx.y;
-	const uint32_t x0 = blockIdx.x * (256u * TM_PX) + threadIdx.x;
-	const uint64_t* __restrict__ src = a.hdr + uint64_t(y) * a.w;
-	uint64_t v[TM_PX];
 #pragma unroll
-	for(int j = 0; j < TM_PX; ++j)
-		v[j] = src[min(x0 + uint32_t(j) * 256u, a.w - 1)];
-#pragma unroll
-	for(int j = 0; j < TM_PX; ++j)
+	for(int j = 0; j < 2; ++j)
 	{
-		const uint32_t x = x0 + uint32_t(j) * 256u;
-		if(x < a.w)
-			__builtin_nontemporal_store(bloom_pixel<LINEAR>(a, x, y, cv_from_color64(v[j])), &a.dst[uint64_t(y) * a.dst_pitch + x]);
+		if(!in_y[j])
+			continue;
+		uint32_t* out = a.dst + uint64_t(uint32_t(y0 + j)) * a.dst_pitch;
+		const ColorPair t = {tonemap_cv(sum[j][0], a.inv_scale), tonemap_cv(sum[j][1], a.inv_scale)};
+		if(in_x[0] && in_x[1])
+			__builtin_nontemporal_store(t, reinterpret_cast<ColorPair*>(out + x0));
+		else
+			out[in_x[0] ? x0 : x0 + 1] = in_x[0] ? t.x : t.y;
 	}
 }
 
@@ -2744,7 +2873,8 @@ __global__ __launch_bounds__(256) void k_bloom_tonemap(BloomArgs a)
 // =============================================================================================
 // Tonemap blocks walk the frame's rows (block b: rows b, b + grid, ...; the threads over the row);
 // each block leaves the partial colour sums of its pixels (no atomics on three shared addresses),
-// k_tonemap_sums adds them up.
+// k_tonemap_sums adds them up. A thread's TM_PX pixels are loaded together.
+#define TM_PX 4
 
 __global__ __launch_bounds__(256) void k_tonemap(const uint64_t* __restrict__ hdr, uint32_t width, uint32_t height,
 	float inv_scale_r, float inv_scale_g, float inv_scale_b, uint32_t* __restrict__ dst, uint32_t dst_pitch,
@@ -3013,25 +3143,46 @@ void launch_finish(hipStream_t st, const DrawRec* drec, uint32_t nd, uint32_t* c
 
 void launch_bloom(hipStream_t st, const BloomArgs& a, bool average)
 {
+	const dim3 down_grid(a.line_parts, a.bh);
 	switch(a.scale_log2)
 	{
-	case 1: hipLaunchKernelGGL(k_bloom_downscale<2>, dim3(a.bh), dim3(256), 0, st, a); break;
-	case 2: hipLaunchKernelGGL(k_bloom_downscale<4>, dim3(a.bh), dim3(256), 0, st, a); break;
-	default: hipLaunchKernelGGL(k_bloom_downscale<8>, dim3(a.bh), dim3(256), 0, st, a); break;
+	case 1: hipLaunchKernelGGL(k_bloom_downscale<2>, down_grid, dim3(256), 0, st, a); break;
+	case 2: hipLaunchKernelGGL(k_bloom_downscale<4>, down_grid, dim3(256), 0, st, a); break;
+	default: hipLaunchKernelGGL(k_bloom_downscale<8>, down_grid, dim3(256), 0, st, a); break;
 	}
 	if(a.radius > 0)
 	{
-		const dim3 blur_grid((a.bw + 256 * BLUR_PX - 1) / (256 * BLUR_PX), a.bh);
-		hipLaunchKernelGGL(k_bloom_blur, blur_grid, dim3(256), 0, st, a, 0u, average ? 1u : 0u);
-		hipLaunchKernelGGL(k_bloom_blur, blur_grid, dim3(256), 0, st, a, 1u, 0u);
+		// the smallest reach that holds the radius; the weights beyond the radius are 0 (radius 12: 13.5 us with
+		// a reach of 12, 14.6 with 16)
+		const int rp = a.radius <= 2 ? 2 : a.radius <= 4 ? 4 : a.radius <= 8 ? 8 : a.radius <= 12 ? 12 : 16;
+		BlurWeights w{};
+		for(int pass = 0; pass < 2; ++pass)
+		{
+			const int32_t* k = pass == 0 ? a.k1 : a.k2;
+			auto tap = [&](int i) { return std::abs(i - rp) <= a.radius ? uint32_t(k[a.radius + std::abs(i - rp)]) : 0u; };
+			for(int j = 0; j <= rp; ++j)
+			{
+				w.even[pass][j] = tap(2 * j) | (tap(2 * j + 1) << 16);
+				w.odd[pass][j] = tap(2 * j - 1) | (tap(2 * j) << 16);
+			}
+		}
+		const dim3 grid((a.bw + BLUR_TILE - 1) / BLUR_TILE, (a.bh + BLUR_TILE - 1) / BLUR_TILE);
+		switch(rp)
+		{
+		case 2: hipLaunchKernelGGL(k_bloom_blur<2>, grid, dim3(256), 0, st, a, w); break;
+		case 4: hipLaunchKernelGGL(k_bloom_blur<4>, grid, dim3(256), 0, st, a, w); break;
+		case 8: hipLaunchKernelGGL(k_bloom_blur<8>, grid, dim3(256), 0, st, a, w); break;
+		case 12: hipLaunchKernelGGL(k_bloom_blur<12>, grid, dim3(256), 0, st, a, w); break;
+		default: hipLaunchKernelGGL(k_bloom_blur<16>, grid, dim3(256), 0, st, a, w); break;
+		}
 	}
-	else if(average)
-		hipLaunchKernelGGL(k_bloom_average, dim3(1), dim3(256), 0, st, a);
-	const dim3 grid((a.w + 256 * TM_PX - 1) / (256 * TM_PX), a.h);
+	const uint64_t* bloom = a.radius > 0 ? a.buf1 : a.buf0;
+	const uint32_t off = a.linear && a.scale_log2 == 1 ? 1u : 0u, with_average = average ? 1u : 0u;
+	const dim3 grid((a.w + off + 511) / 512, (a.h + off + 1) / 2 + with_average);
 	if(a.linear)
-		hipLaunchKernelGGL(k_bloom_tonemap<true>, grid, dim3(256), 0, st, a);
+		hipLaunchKernelGGL(k_bloom_tonemap<true>, grid, dim3(256), 0, st, a, bloom, with_average);
 	else
-		hipLaunchKernelGGL(k_bloom_tonemap<false>, grid, dim3(256), 0, st, a);
+		hipLaunchKernelGGL(k_bloom_tonemap<false>, grid, dim3(256), 0, st, a, bloom, with_average);
 }
 
 void launch_portal_mix(hipStream_t st, uint32_t color_bits, const uint32_t* lite, const PortalMixRec* recs, uint32_t num,

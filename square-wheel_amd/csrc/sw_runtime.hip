@@ -1330,9 +1330,10 @@ int sw_postprocess_device(sw_ctx* ctx, const void* hdr_device, uint32_t width, u
 	a.dst = static_cast<uint32_t*>(dst32_device);
 	a.dst_pitch = uint32_t(dst_pitch_bytes / 4);
 	const uint64_t texels = uint64_t(a.bw) * a.bh;
+	a.line_parts = (a.bw * S + 511) / 512;
 	int r;
 	if((r = ensure(ctx, ctx->bloom0, texels * 8)) || (r = ensure(ctx, ctx->bloom1, texels * 8)) ||
-		(r = ensure(ctx, ctx->bloom_lines, uint64_t(a.bh) * 16)))
+		(r = ensure(ctx, ctx->bloom_lines, uint64_t(a.bh) * a.line_parts * 16)))
 		return r;
 	a.buf0 = static_cast<uint64_t*>(ctx->bloom0.p);
 	a.buf1 = static_cast<uint64_t*>(ctx->bloom1.p);
