@@ -63,6 +63,7 @@ enum
 // besides the draw blocks): a second round of blocks would add a whole block's latency.
 #define SURF_BLOCK 256
 #define SURF_MAX_TEXELS_PER_THREAD 8
+#define SURF_LINES_MIN_TEXELS 1024 // blocks of at least this many texels stage lightmap lines
 __host__ __device__ inline uint32_t surf_block_texels(uint64_t arena_texels)
 {
 	const uint64_t per_thread = (arena_texels + uint64_t(SURF_BLOCK) * 1024u - 1) / (uint64_t(SURF_BLOCK) * 1024u);
