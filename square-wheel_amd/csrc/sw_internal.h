@@ -272,12 +272,16 @@ void launch_tonemap(hipStream_t st, const uint64_t* hdr, uint32_t w, uint32_t h,
 // vertex int, first fan-count byte), device copies of runs and bases; the host checked every range.
 void launch_expand_mesh_runs(hipStream_t st, const sw_mesh_run* runs, uint32_t num_runs, uint32_t max_triangles, const uint64_t* bases,
 	const sw_model_vertex* vertices, const uint16_t* triangles, const uint32_t* counts, int32_t* out_ints, uint8_t* out_fans);
-// Triangle-model preparation: one block per instance. meshes / instances / sort_offsets are device
-// copies; scratch holds the sort keys of instances above model_sort_lds_limit() triangles
-// (sort_offsets[i] entries into it, a power of two of them each).
-void launch_prepare_models(hipStream_t st, uint32_t num_instances, const sw_model_mesh* meshes, const sw_model_instance* instances,
-	const uint64_t* sort_offsets, uint64_t* scratch, sw_model_vertex* out_vertices, uint16_t* out_triangles, uint32_t* out_counts,
-	uint32_t* host_err);
+// Triangle-model preparation: one block per instance. recs is device-visible; scratch holds the sort keys of
+// instances above model_sort_lds_limit() triangles (a power of two of them from sort_offset on).
+struct ModelRec
+{
+	sw_model_mesh mesh;
+	uint64_t sort_offset;
+	sw_model_instance instance;
+};
+void launch_prepare_models(hipStream_t st, uint32_t num_instances, const ModelRec* recs, uint64_t* scratch,
+	sw_model_vertex* out_vertices, uint16_t* out_triangles, uint32_t* out_counts, uint32_t* host_err);
 uint32_t model_sort_lds_limit();
 
 // Texture operations: pack_texture_ops validates them against the level table and packs the

@@ -2,9 +2,17 @@
 // light.rs:296-340): one block per model instance animates, transforms and lights the mesh's
 // vertices, then rejects back faces and sorts the front-facing triangles back to front.
 //
+// A block's phases follow each other and each is a few loads long, so latency bounds it: the instance's
+// record comes from pinned host memory into LDS in one round trip (a copy to the device, then chains of
+// dependent loads, before), positions stay in LDS for the back-face test, the sort's keys in registers.
+// 64 instances of 642 vertices and 1280 triangles: 32 us after a copy of
+// 5.8 us before, now 15.1.
+//
 // Float operations keep the reference's order and fusion (cgmath 0.18 f32 arithmetic: matrix x
 // vector is the column sum c0*x + c1*y + c2*z (+ c3*w), left to right, unfused; the file is built
 // with -ffp-contract=off), so the results are bit-exact to the oracle's restatement.
+#include <type_traits>
+
 #include "sw_internal.h"
 #include "sw_device.h"
 
@@ -14,7 +22,8 @@ namespace
 {
 
 #define MODEL_BLOCK 1024u
-#define MODEL_SORT_LDS 4096u // sort keys kept in LDS up to this many (power of two) triangles
+#define MODEL_SORT_LDS 4096u // up to this many triangles the block sorts in registers and LDS
+#define MODEL_LDS_VERTICES 4000u // positions kept in LDS up to this many vertices
 
 struct F3
 {
@@ -61,25 +70,29 @@ SW_DEV void m3_mul_m3(const float* a, const float* b, float* out)
 
 // get_normals_matrix (triangle_models_rendering.rs:722-731): the 3x3 axes of the model matrix,
 // transposed and inverted (cgmath 0.18 Matrix3::invert: cofactor columns c1 x c2, c2 x c0, c0 x c1
-// divided by the determinant, transposed; identity when the determinant is 0).
+// divided by the determinant, transposed; identity when the determinant is 0). c(i, n) is component n of
+// column i of the transposed axes; element (j, k), the product's column j and row k, is component j of
+// cofactor column k.
+SW_DEV float normals_determinant(const float* m4)
+{
+	auto c = [&](int i, int n) { return m4[4 * n + i]; };
+	return c(0, 0) * (c(1, 1) * c(2, 2) - c(2, 1) * c(1, 2)) - c(1, 0) * (c(0, 1) * c(2, 2) - c(2, 1) * c(0, 2)) +
+		c(2, 0) * (c(0, 1) * c(1, 2) - c(1, 1) * c(0, 2));
+}
+SW_DEV float normals_element(const float* m4, float det, int j, int k)
+{
+	auto c = [&](int i, int n) { return m4[4 * n + i]; };
+	if(det == 0.0f)
+		return j == k ? 1.0f : 0.0f;
+	const int a = (k + 1) % 3, b = (k + 2) % 3, n = (j + 1) % 3, o = (j + 2) % 3;
+	return (c(a, n) * c(b, o) - c(a, o) * c(b, n)) / det;
+}
 SW_DEV void normals_matrix(const float* m4, float* out)
 {
-	// A = transpose(axes): column k of A is row k of the axes, A[k][j] = m4 column j, component k
-	const F3 c0 = f3(m4[0], m4[4], m4[8]), c1 = f3(m4[1], m4[5], m4[9]), c2 = f3(m4[2], m4[6], m4[10]);
-	const float det = c0.x * (c1.y * c2.z - c2.y * c1.z) - c1.x * (c0.y * c2.z - c2.y * c0.z) + c2.x * (c0.y * c1.z - c1.y * c0.z);
-	if(det == 0.0f)
-	{
-		for(int i = 0; i < 9; ++i)
-			out[i] = (i % 4 == 0) ? 1.0f : 0.0f;
-		return;
-	}
-	const F3 r0 = cross(c1, c2), r1 = cross(c2, c0), r2 = cross(c0, c1);
-	const F3 r[3] = {f3(r0.x / det, r0.y / det, r0.z / det), f3(r1.x / det, r1.y / det, r1.z / det),
-		f3(r2.x / det, r2.y / det, r2.z / det)};
-	// transpose of from_cols(r0, r1, r2): column j = (r0[j], r1[j], r2[j])
+	const float det = normals_determinant(m4);
 	for(int j = 0; j < 3; ++j)
 		for(int k = 0; k < 3; ++k)
-			out[j * 3 + k] = (&r[k].x)[j];
+			out[j * 3 + k] = normals_element(m4, det, j, k);
 }
 
 // get_vertex_light (triangle_models_rendering.rs:702-720) with get_light_cube_light (light.rs:296-340).
@@ -129,9 +142,7 @@ SW_DEV uint64_t sort_key(float z, uint32_t t)
 
 struct ModelLaunch
 {
-	const sw_model_mesh* meshes;
-	const sw_model_instance* instances;
-	const uint64_t* sort_offsets; // per instance: its region of `scratch` (sorts above MODEL_SORT_LDS)
+	const swk::ModelRec* recs; // pinned host memory, one per instance
 	uint64_t* scratch;
 	sw_model_vertex* out_vertices;
 	uint16_t* out_triangles;
@@ -139,26 +150,101 @@ struct ModelLaunch
 	uint32_t* host_err; // pinned word set on an out-of-range vertex or bone index
 };
 
+// Bitonic sort of n_pad <= E * MODEL_BLOCK keys, ascending; the thread holds elements e * MODEL_BLOCK + tid.
+// A partner is a lane of the wave (most steps), a thread of another wave (through LDS, two buffers in turn, so
+// one barrier a step; b0 may still be read when the sort starts) or another of the thread's own elements.
+template <int E>
+SW_DEV void sort_keys(uint64_t (&key)[E], uint32_t n_pad, uint64_t* b0, uint64_t* b1)
+{
+	const uint32_t tid = threadIdx.x;
+	uint64_t *next = b1, *other_buffer = b0;
+#pragma unroll 1
+	for(uint32_t k = 2; k <= n_pad; k <<= 1)
+#pragma unroll 1
+		for(uint32_t j = k >> 1; j > 0; j >>= 1)
+		{
+			if(j >= MODEL_BLOCK)
+			{
+#pragma unroll
+				for(uint32_t step = 1; step < E; step <<= 1)
+					if(j == step * MODEL_BLOCK)
+#pragma unroll
+						for(uint32_t e = 0; e < E; ++e)
+							if((e & step) == 0)
+							{
+								const bool up = (e * MODEL_BLOCK & k) == 0; // k > j >= MODEL_BLOCK: the thread's bits are below
+								const uint64_t x = key[e], y = key[e | step];
+								if(up == (x > y))
+								{
+									key[e] = y;
+									key[e | step] = x;
+								}
+							}
+				continue;
+			}
+			uint64_t other[E];
+			if(j >= 64)
+			{
+#pragma unroll
+				for(uint32_t e = 0; e < E; ++e)
+					next[e * MODEL_BLOCK + tid] = key[e];
+				__syncthreads();
+#pragma unroll
+				for(uint32_t e = 0; e < E; ++e)
+					other[e] = next[e * MODEL_BLOCK + (tid ^ j)];
+				uint64_t* const t = next;
+				next = other_buffer;
+				other_buffer = t;
+			}
+			else
+#pragma unroll
+				for(uint32_t e = 0; e < E; ++e)
+					other[e] = __shfl_xor(key[e], int(j));
+#pragma unroll
+			for(uint32_t e = 0; e < E; ++e)
+			{
+				const uint32_t i = e * MODEL_BLOCK + tid;
+				const bool keep_less = ((i & j) == 0) == ((i & k) == 0);
+				key[e] = (other[e] < key[e]) == keep_less ? other[e] : key[e];
+			}
+		}
+}
+
 __global__ __launch_bounds__(MODEL_BLOCK) void k_prepare_models(ModelLaunch L)
 {
-	__shared__ float bone_m[SW_MODEL_MAX_BONES * 16]; // model-view * bone matrix, / 255
-	__shared__ float bone_n[SW_MODEL_MAX_BONES * 9]; // normals matrix * bone normals matrix, / 255
-	__shared__ uint8_t bone_done[SW_MODEL_MAX_BONES];
+	__shared__ __align__(16) swk::ModelRec rec;
+	__shared__ float nm[9];
 	__shared__ uint64_t keys_lds[MODEL_SORT_LDS];
+	// the vertices' positions, then the sort's second buffer
+	__shared__ __align__(8) float positions[MODEL_LDS_VERTICES * 3];
 	__shared__ uint32_t visible;
+	static_assert(sizeof(positions) >= sizeof(keys_lds));
+	// the skeleton's matrices, until the vertices are done
+	float* bone_m = reinterpret_cast<float*>(keys_lds); // model-view * bone matrix, / 255
+	float* bone_n = bone_m + SW_MODEL_MAX_BONES * 16; // normals matrix * bone normals matrix, / 255
+	uint8_t* bone_done = reinterpret_cast<uint8_t*>(bone_n + SW_MODEL_MAX_BONES * 9);
+	static_assert(sizeof(keys_lds) >= SW_MODEL_MAX_BONES * (16 + 9) * 4 + SW_MODEL_MAX_BONES);
 
-	const sw_model_instance& in = L.instances[blockIdx.x];
-	const sw_model_mesh M = L.meshes[in.mesh];
 	const uint32_t tid = threadIdx.x;
+	static_assert(sizeof(rec) % 4 == 0 && sizeof(rec) / 4 <= MODEL_BLOCK);
+	if(tid < sizeof(rec) / 4)
+		reinterpret_cast<uint32_t*>(&rec)[tid] = reinterpret_cast<const uint32_t*>(L.recs + blockIdx.x)[tid];
+	if(tid == 0)
+		visible = 0;
+	__syncthreads();
+	const sw_model_instance& in = rec.instance;
+	const sw_model_mesh M = rec.mesh;
+	if(tid < 9)
+		nm[tid] = normals_element(in.model_matrix, normals_determinant(in.model_matrix), int(tid / 3), int(tid % 3));
+	__syncthreads();
 	bool bad = false;
 
 	const float lerp0 = fmin_r(fmax_r(in.lerp, 0.0f), 1.0f);
 	const float lerp1 = 1.0f - lerp0;
 	const bool perform_lerp = lerp0 > 0.01f && lerp0 < 0.99f;
 	const uint32_t frame_single = lerp0 > lerp1 ? in.frames[0] : in.frames[1];
-	float nm[9];
-	normals_matrix(in.model_matrix, nm);
 	sw_model_vertex* out_v = L.out_vertices + in.first_vertex;
+	const bool keep_positions = M.num_vertices <= MODEL_LDS_VERTICES;
 
 	const bool skeleton = M.kind == SW_MODEL_SKELETON_ANIMATED && M.num_bones > 0;
 	if(skeleton)
@@ -339,73 +425,112 @@ __global__ __launch_bounds__(MODEL_BLOCK) void k_prepare_models(ModelLaunch L)
 		}
 		// tc: tex_coord * tc_scale + tc_shift (:37)
 		store_vertex(out_v + v, pos, tc0 * in.tc_scale[0] + in.tc_shift[0], tc1 * in.tc_scale[1] + in.tc_shift[1], light);
+		if(keep_positions)
+		{
+			positions[v * 3] = pos.x;
+			positions[v * 3 + 1] = pos.y;
+			positions[v * 3 + 2] = pos.z;
+		}
 	}
-	if(tid == 0)
-		visible = 0;
 	__syncthreads();
 
 	// back faces (:324-341): the front faces' sort keys (:343-391) are compacted to the front of
 	// `keys` (in any order: the keys hold the triangle index, so the sort fixes the order)
-	uint32_t n_cap = 1;
-	while(n_cap < M.num_triangles)
-		n_cap <<= 1;
-	uint64_t* keys = n_cap <= MODEL_SORT_LDS ? keys_lds : L.scratch + L.sort_offsets[blockIdx.x];
-	for(uint32_t t = tid; t < M.num_triangles; t += MODEL_BLOCK)
+	const bool lds_sort = M.num_triangles <= MODEL_SORT_LDS;
+	uint64_t* keys = lds_sort ? keys_lds : L.scratch + rec.sort_offset;
+	for(uint32_t t0 = 0; t0 < M.num_triangles; t0 += MODEL_BLOCK)
 	{
-		uint32_t idx[3];
-		for(int k = 0; k < 3; ++k)
+		const uint32_t t = t0 + tid;
+		bool front = false;
+		float z = 0.0f;
+		if(t < M.num_triangles)
 		{
-			idx[k] = M.triangles[uint64_t(t) * 3 + k];
-			if(idx[k] >= M.num_vertices)
+			uint32_t idx[3];
+			for(int k = 0; k < 3; ++k)
 			{
-				bad = true;
-				idx[k] = M.num_vertices - 1;
+				idx[k] = M.triangles[uint64_t(t) * 3 + k];
+				if(idx[k] >= M.num_vertices)
+				{
+					bad = true;
+					idx[k] = M.num_vertices - 1;
+				}
 			}
+			F3 p[3];
+			for(int k = 0; k < 3; ++k)
+				p[k] = keep_positions ? load_f3(positions + idx[k] * 3) : load_f3(&out_v[idx[k]].pos[0]);
+			// get_triangle_plane (:393-401): (v1 - v0) x (v2 - v1), dist = vec . v0
+			const F3 vec = cross(sub(p[1], p[0]), sub(p[2], p[1]));
+			front = dot(vec, p[0]) > 0.0f;
+			z = fmax_r(fmax_r(p[0].z, p[1].z), p[2].z);
 		}
-		const F3 p0 = load_f3(&out_v[idx[0]].pos[0]), p1 = load_f3(&out_v[idx[1]].pos[0]), p2 = load_f3(&out_v[idx[2]].pos[0]);
-		// get_triangle_plane (:393-401): (v1 - v0) x (v2 - v1), dist = vec . v0
-		const F3 vec = cross(sub(p1, p0), sub(p2, p1));
-		if(dot(vec, p0) > 0.0f)
-			keys[atomicAdd(&visible, 1u)] = sort_key(fmax_r(fmax_r(p0.z, p1.z), p2.z), t);
+		const uint64_t mask = __ballot(front);
+		uint32_t first = 0;
+		if((tid & 63) == 0 && mask)
+			first = atomicAdd(&visible, uint32_t(__popcll(mask)));
+		first = __builtin_amdgcn_readfirstlane(first);
+		if(front)
+			keys[first + uint32_t(__popcll(mask & ((1ull << (tid & 63)) - 1ull)))] = sort_key(z, t);
 	}
 	__syncthreads();
 	const uint32_t count = visible;
 	uint32_t n_pad = 1;
 	while(n_pad < count)
 		n_pad <<= 1;
-	for(uint32_t t = count + tid; t < n_pad; t += MODEL_BLOCK)
-		keys[t] = ~0ull;
-	__syncthreads();
-
-	// bitonic sort, ascending
-	for(uint32_t k = 2; k <= n_pad; k <<= 1)
-		for(uint32_t j = k >> 1; j > 0; j >>= 1)
-		{
-			for(uint32_t i = tid; i < n_pad; i += MODEL_BLOCK)
-			{
-				const uint32_t l = i ^ j;
-				if(l > i)
-				{
-					const uint64_t a = keys[i], b = keys[l];
-					if(((i & k) == 0) == (a > b))
-					{
-						keys[i] = b;
-						keys[l] = a;
-					}
-				}
-			}
-			__syncthreads();
-		}
-
 	uint16_t* out_t = L.out_triangles + uint64_t(in.first_triangle) * 3;
-	for(uint32_t i = tid; i < count; i += MODEL_BLOCK)
-	{
-		const uint32_t t = uint32_t(keys[i]);
+	auto store_triangle = [&](uint32_t i, uint32_t t) {
 		for(int k = 0; k < 3; ++k)
 		{
 			const uint32_t idx = M.triangles[uint64_t(t) * 3 + k];
 			out_t[uint64_t(i) * 3 + k] = uint16_t(idx < M.num_vertices ? idx : M.num_vertices - 1);
 		}
+	};
+	if(lds_sort)
+	{
+		auto sort = [&](auto elements) __attribute__((always_inline)) {
+			constexpr int E = elements;
+			uint64_t key[E];
+#pragma unroll
+			for(uint32_t e = 0; e < E; ++e)
+				key[e] = e * MODEL_BLOCK + tid < count ? keys_lds[e * MODEL_BLOCK + tid] : ~0ull;
+			sort_keys<E>(key, n_pad, keys_lds, reinterpret_cast<uint64_t*>(positions));
+#pragma unroll
+			for(uint32_t e = 0; e < E; ++e)
+				if(e * MODEL_BLOCK + tid < count)
+					store_triangle(e * MODEL_BLOCK + tid, uint32_t(key[e]));
+		};
+		if(n_pad <= MODEL_BLOCK)
+			sort(std::integral_constant<int, 1>{});
+		else if(n_pad <= 2 * MODEL_BLOCK)
+			sort(std::integral_constant<int, 2>{});
+		else
+			sort(std::integral_constant<int, 4>{});
+		static_assert(MODEL_SORT_LDS == 4 * MODEL_BLOCK);
+	}
+	else
+	{
+		for(uint32_t t = count + tid; t < n_pad; t += MODEL_BLOCK)
+			keys[t] = ~0ull;
+		__syncthreads();
+		for(uint32_t k = 2; k <= n_pad; k <<= 1)
+			for(uint32_t j = k >> 1; j > 0; j >>= 1)
+			{
+				for(uint32_t i = tid; i < n_pad; i += MODEL_BLOCK)
+				{
+					const uint32_t l = i ^ j;
+					if(l > i)
+					{
+						const uint64_t a = keys[i], b = keys[l];
+						if(((i & k) == 0) == (a > b))
+						{
+							keys[i] = b;
+							keys[l] = a;
+						}
+					}
+				}
+				__syncthreads();
+			}
+		for(uint32_t i = tid; i < count; i += MODEL_BLOCK)
+			store_triangle(i, uint32_t(keys[i]));
 	}
 	if(tid == 0)
 		L.out_counts[blockIdx.x] = count;
@@ -588,11 +713,10 @@ void launch_expand_mesh_runs(hipStream_t st, const sw_mesh_run* runs, uint32_t n
 	ExpandLaunch a{runs, bases, vertices, triangles, counts, out_ints, out_fans};
 	hipLaunchKernelGGL(k_expand_mesh_runs, dim3((max_triangles + 255u) / 256u, num_runs), dim3(256), 0, st, a);
 }
-void launch_prepare_models(hipStream_t st, uint32_t num_instances, const sw_model_mesh* meshes, const sw_model_instance* instances,
-	const uint64_t* sort_offsets, uint64_t* scratch, sw_model_vertex* out_vertices, uint16_t* out_triangles, uint32_t* out_counts,
-	uint32_t* host_err)
+void launch_prepare_models(hipStream_t st, uint32_t num_instances, const ModelRec* recs, uint64_t* scratch,
+	sw_model_vertex* out_vertices, uint16_t* out_triangles, uint32_t* out_counts, uint32_t* host_err)
 {
-	ModelLaunch L{meshes, instances, sort_offsets, scratch, out_vertices, out_triangles, out_counts, host_err};
+	ModelLaunch L{recs, scratch, out_vertices, out_triangles, out_counts, host_err};
 	hipLaunchKernelGGL(k_prepare_models, dim3(num_instances), dim3(MODEL_BLOCK), 0, st, L);
 }
 

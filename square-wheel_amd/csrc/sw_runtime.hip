@@ -76,7 +76,7 @@ struct sw_ctx
 
 	// command buffers / work buffers
 	DevBuf views, surfaces, lights, light_indices, draws, vdata, surf_ext, blk_surf, parts, spans, drec, dbounds, counters, arena, fb,
-		tonemap_out, tonemap_sums, bloom0, bloom1, bloom_lines, model_args, model_scratch, texop_args, shadows, depth_args,
+		tonemap_out, tonemap_sums, bloom0, bloom1, bloom_lines, model_scratch, texop_args, shadows, depth_args,
 		depth_rows, water_points, fire_args, portal_mix, mesh_args, mesh_fans;
 	uint32_t num_shadows = 0; // sw_set_light_shadows: entries in `shadows`
 	const float* shadow_texels = nullptr;
@@ -894,7 +894,7 @@ void sw_ctx_destroy(sw_ctx* ctx)
 		(void)hipGraphDestroy(ctx->graph);
 	DevBuf* bufs[] = {&ctx->views, &ctx->surfaces, &ctx->lights, &ctx->light_indices, &ctx->draws, &ctx->vdata, &ctx->surf_ext, &ctx->blk_surf,
 		&ctx->parts, &ctx->spans, &ctx->drec, &ctx->dbounds, &ctx->counters, &ctx->arena, &ctx->fb, &ctx->tonemap_out, &ctx->tonemap_sums,
-		&ctx->bloom0, &ctx->bloom1, &ctx->bloom_lines, &ctx->model_args, &ctx->model_scratch, &ctx->texop_args, &ctx->shadows, &ctx->depth_args,
+		&ctx->bloom0, &ctx->bloom1, &ctx->bloom_lines, &ctx->model_scratch, &ctx->texop_args, &ctx->shadows, &ctx->depth_args,
 		&ctx->depth_rows, &ctx->water_points, &ctx->fire_args};
 	for(DevBuf* b : bufs)
 		release(ctx, *b);
@@ -1560,18 +1560,20 @@ int sw_prepare_models(sw_ctx* ctx, const sw_model_mesh* meshes, uint32_t num_mes
 	for(uint32_t i = 0; i < num_meshes; ++i)
 	{
 		const sw_model_mesh& m = meshes[i];
-		const std::string which = "model mesh " + std::to_string(i) + ": ";
+		auto error = [&](const char* what) {
+			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "model mesh " + std::to_string(i) + ": " + what);
+		};
 		if(m.kind > SW_MODEL_SKELETON_ANIMATED)
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "unknown kind");
+			return error("unknown kind");
 		if(m.num_triangles > SW_MODEL_MAX_TRIANGLES || m.num_vertices > 65536)
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "more than 65536 triangles or vertices");
+			return error("more than 65536 triangles or vertices");
 		if((m.num_triangles && (!m.triangles || m.num_vertices == 0)) || (m.num_vertices && !m.vertices))
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "missing vertex or triangle data");
+			return error("missing vertex or triangle data");
 		if(m.kind == SW_MODEL_VERTEX_ANIMATED && m.num_vertices && (m.num_frames == 0 || !m.frame_vertices))
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "vertex animation without frames");
+			return error("vertex animation without frames");
 		if(m.kind == SW_MODEL_SKELETON_ANIMATED &&
 			(m.num_bones > SW_MODEL_MAX_BONES || (m.num_bones && (m.num_frames == 0 || !m.frame_bones || !m.bone_parents))))
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "bad skeleton (more than 255 bones, or no frames)");
+			return error("bad skeleton (more than 255 bones, or no frames)");
 	}
 	// per-instance checks, output ranges, and the scratch regions of sorts too large for LDS
 	const uint32_t lds_limit = swk::model_sort_lds_limit();
@@ -1580,16 +1582,18 @@ int sw_prepare_models(sw_ctx* ctx, const sw_model_mesh* meshes, uint32_t num_mes
 	for(uint32_t i = 0; i < num_instances; ++i)
 	{
 		const sw_model_instance& in = instances[i];
-		const std::string which = "model instance " + std::to_string(i) + ": ";
+		auto error = [&](const char* what) {
+			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "model instance " + std::to_string(i) + ": " + what);
+		};
 		if(in.mesh >= num_meshes)
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "mesh index out of range");
+			return error("mesh index out of range");
 		const sw_model_mesh& m = meshes[in.mesh];
 		const bool animated = m.kind == SW_MODEL_VERTEX_ANIMATED || (m.kind == SW_MODEL_SKELETON_ANIMATED && m.num_bones);
 		if(animated && m.num_vertices && (in.frames[0] >= m.num_frames || in.frames[1] >= m.num_frames))
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "animation frame out of range");
+			return error("animation frame out of range");
 		if(uint64_t(in.first_vertex) + m.num_vertices > vertex_capacity ||
 			uint64_t(in.first_triangle) + m.num_triangles > triangle_capacity)
-			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, which + "output range beyond the buffers' capacity");
+			return error("output range beyond the buffers' capacity");
 		uint64_t n_pad = 1;
 		while(n_pad < m.num_triangles)
 			n_pad <<= 1;
@@ -1600,29 +1604,24 @@ int sw_prepare_models(sw_ctx* ctx, const sw_model_mesh* meshes, uint32_t num_mes
 		}
 	}
 	(void)hipSetDevice(ctx->device);
-	const size_t mesh_bytes = sizeof(sw_model_mesh) * num_meshes, inst_bytes = sizeof(sw_model_instance) * num_instances,
-				 off_bytes = sizeof(uint64_t) * num_instances;
-	const size_t inst_at = (mesh_bytes + 255) & ~size_t(255), off_at = (inst_at + inst_bytes + 255) & ~size_t(255);
 	int r;
-	if((r = ensure(ctx, ctx->model_args, off_at + off_bytes)) ||
-		(scratch_entries && (r = ensure(ctx, ctx->model_scratch, scratch_entries * sizeof(uint64_t)))))
+	if(scratch_entries && (r = ensure(ctx, ctx->model_scratch, scratch_entries * sizeof(uint64_t))))
 		return r;
-	char* args = static_cast<char*>(ctx->model_args.p);
+	// each instance's block reads its record straight from the staging memory
 	char* staging = nullptr;
-	if((r = stage_begin(ctx, off_at + off_bytes, &staging)))
+	const char* recs = nullptr;
+	if((r = stage_begin(ctx, sizeof(swk::ModelRec) * num_instances, &staging, &recs)))
 		return r;
-	std::memcpy(staging, meshes, mesh_bytes);
-	std::memcpy(staging + inst_at, instances, inst_bytes);
-	std::memcpy(staging + off_at, sort_offsets.data(), off_bytes);
-	if((r = stage_copy(ctx, args, off_at + off_bytes)))
-		return r;
+	for(uint32_t i = 0; i < num_instances; ++i)
+		reinterpret_cast<swk::ModelRec*>(staging)[i] = swk::ModelRec{meshes[instances[i].mesh], sort_offsets[i], instances[i]};
 	{
 		StageTimer t(ctx, STAGE_MODELS);
-		swk::launch_prepare_models(ctx->stream, num_instances, reinterpret_cast<const sw_model_mesh*>(args),
-			reinterpret_cast<const sw_model_instance*>(args + inst_at), reinterpret_cast<const uint64_t*>(args + off_at),
+		swk::launch_prepare_models(ctx->stream, num_instances, reinterpret_cast<const swk::ModelRec*>(recs),
 			static_cast<uint64_t*>(ctx->model_scratch.p), out_vertices, out_triangles, out_counts,
 			ctx->counters_host_dev + HOST_MODEL_ERR_OFFSET);
 	}
+	if((r = stage_used(ctx)))
+		return r;
 	return hip_check(ctx, hipGetLastError(), "model preparation launch");
 }
 
