@@ -16,6 +16,7 @@
 
 #include "sw_internal.h"
 #include "sw_device.h"
+#include "sw_divide.h"
 
 using namespace swd;
 
@@ -53,20 +54,34 @@ SW_DEV CI ci_blend(CI src, CI dst, int32_t alpha)
 		wadd(wmul(src.r, alpha), wmul(dst.r, ia)) >> 8, wadd(wmul(src.a, alpha), wmul(dst.a, ia)) >> 8};
 }
 
+enum : uint32_t
+{
+	RUN_LITE = 1, // destination (and sources) are TextureLite levels
+	RUN_OVERWRITES = 2, // the first operation leaves nothing of what the destination holds
+};
+
 struct TexOpRun
 {
 	uint32_t first_op, num_ops;
 	uint32_t first_block;
-	uint32_t lite; // destination (and sources) are TextureLite levels
+	uint32_t flags;
 	TexLevel dst;
+};
+
+enum : uint32_t
+{
+	OP_TURB = 1,
+	OP_MODULATE = 2, // layers: a light component outside [0.98, 1.02] (impl_1, :231-242)
+	OP_OVERFLOWS = 4, // layers: shift + row can overflow (and the height is no power of two), which the rem_euclid sees
+	OP_BLEND_SHIFT = 8,
 };
 
 struct DevTexOp
 {
-	uint32_t kind, blend;
-	uint32_t modulate; // layers: a light component outside [0.98, 1.02] (impl_1, :231-242)
+	uint32_t flags;
 	uint32_t turb_shifts; // TURB: first shift of the level
-	int32_t shift[2];
+	uint32_t add[2]; // layers: the source texel is (destination + add) mod size
+	int32_t shift_v;
 	int32_t light_vec[3]; // lanes B, G, R
 	TexLevel src;
 };
@@ -84,10 +99,10 @@ struct TexOpLaunch
 // apply_texture_layer_impl_2 (generative_texture_effect_layered.rs:255-381), one texel
 SW_DEV sw_texel layer_texel(const DevTexOp& op, sw_texel dst, sw_texel src)
 {
-	if(op.modulate)
+	if(op.flags & OP_MODULATE)
 	{
 		const CI m = modulate(src.diffuse, op.light_vec);
-		switch(op.blend)
+		switch(op.flags >> OP_BLEND_SHIFT)
 		{
 		case SW_BLEND_NONE: return sw_texel{Color32T::from_ci(m), src.packed_normal_roughness};
 		case SW_BLEND_AVERAGE:
@@ -101,7 +116,7 @@ SW_DEV sw_texel layer_texel(const DevTexOp& op, sw_texel dst, sw_texel src)
 		default: return dst;
 		}
 	}
-	switch(op.blend)
+	switch(op.flags >> OP_BLEND_SHIFT)
 	{
 	case SW_BLEND_NONE: return src;
 	case SW_BLEND_AVERAGE: dst.diffuse = Color32T::average(dst.diffuse, src.diffuse); return dst;
@@ -121,7 +136,7 @@ SW_DEV sw_texel layer_texel(const DevTexOp& op, sw_texel dst, sw_texel src)
 SW_DEV uint32_t lite_layer_texel(const DevTexOp& op, uint32_t dst, uint32_t src)
 {
 	const CI m = modulate(src, op.light_vec);
-	switch(op.blend)
+	switch(op.flags >> OP_BLEND_SHIFT)
 	{
 	case SW_BLEND_NONE: return Color32T::from_ci(m);
 	case SW_BLEND_AVERAGE: return Color32T::from_ci(ci_shr2(ci_add2(m, Color32T::to_ci(dst)), 1));
@@ -132,73 +147,140 @@ SW_DEV uint32_t lite_layer_texel(const DevTexOp& op, uint32_t dst, uint32_t src)
 	}
 }
 
-// make_turb_distortion (generative_texture_effect_turb.rs:89-138): the source texel at
-// (x + shift[y], y + shift[x]), wrapped by the power-of-two masks
-SW_DEV uint64_t turb_index(const TexOpLaunch& L, const DevTexOp& op, uint32_t x, uint32_t y, uint32_t w, uint32_t h)
+SW_DEV sw_texel blend_layer(const DevTexOp& op, sw_texel dst, sw_texel src) { return layer_texel(op, dst, src); }
+SW_DEV uint32_t blend_layer(const DevTexOp& op, uint32_t dst, uint32_t src) { return lite_layer_texel(op, dst, src); }
+
+// (destination + add) mod size for the texels of a thread; one division for all where size is no power of two.
+template <uint32_t N>
+SW_DEV void wrap_all(const uint32_t (&at)[N], uint32_t add, uint32_t size, uint32_t (&out)[N])
 {
-	const int32_t row_shift = L.turb_shifts[op.turb_shifts + y];
-	const int32_t column_shift = L.turb_shifts[op.turb_shifts + x];
-	const uint32_t u = uint32_t(int32_t(x) + row_shift) & (w - 1), v = uint32_t(int32_t(y) + column_shift) & (h - 1);
-	return op.src.offset + uint64_t(v) * w + u;
+	if((size & (size - 1)) == 0)
+	{
+#pragma unroll
+		for(uint32_t k = 0; k < N; ++k)
+			out[k] = (at[k] + add) & (size - 1);
+	}
+	else
+	{
+		const double inv = 1.0 / double(size);
+#pragma unroll
+		for(uint32_t k = 0; k < N; ++k)
+			out[k] = swdiv::mod_rcp(at[k] + add, size, swdiv::NO_MASK, inv);
+	}
 }
 
-__global__ __launch_bounds__(TEXOP_BLOCK) void k_texture_ops(TexOpLaunch L)
+// The operation's source texels of a thread's destination texels.
+template <class T, uint32_t N>
+SW_DEV void load_sources(const TexOpLaunch& L, const TexOpRun& run, const DevTexOp& op, const T* texels, const uint32_t (&x)[N],
+	const uint32_t (&y)[N], T (&out)[N])
 {
-	// the block's run: the last run starting at or before this block
-	uint32_t lo = 0, hi = L.num_runs;
-	while(hi - lo > 1)
+	uint32_t su[N], sv[N];
+	if(op.flags & OP_TURB)
 	{
-		const uint32_t mid = (lo + hi) >> 1;
-		if(L.runs[mid].first_block <= blockIdx.x)
-			lo = mid;
-		else
-			hi = mid;
+		// make_turb_distortion (generative_texture_effect_turb.rs:89-138): the source texel at
+		// (x + shift[y], y + shift[x]), wrapped by the power-of-two masks
+		const int32_t* shifts = L.turb_shifts + op.turb_shifts;
+#pragma unroll
+		for(uint32_t k = 0; k < N; ++k)
+		{
+			su[k] = (x[k] + uint32_t(shifts[y[k]])) & (op.src.w - 1);
+			sv[k] = (y[k] + uint32_t(shifts[x[k]])) & (op.src.h - 1);
+		}
 	}
-	const TexOpRun run = L.runs[lo];
+	else
+	{
+		// u steps from rem_euclid(shift) with a wrap at the width, v is the rem_euclid of each row's sum
+		wrap_all(x, op.add[0], op.src.w, su);
+		if(op.flags & OP_OVERFLOWS)
+#pragma unroll
+			for(uint32_t k = 0; k < N; ++k)
+				sv[k] = wrap(op.shift_v + int32_t(y[k]), op.src.h);
+		else
+			wrap_all(y, op.add[1], op.src.h, sv);
+	}
+	const T* src = texels + op.src.offset;
+#pragma unroll
+	for(uint32_t k = 0; k < N; ++k)
+		out[k] = src[uint64_t(sv[k]) * op.src.w + su[k]];
+}
+
+// A block's texels of a run: all operations in turn on TEXOP_PER_THREAD texels of a thread together; an
+// operation's sources are requested before the previous one is blended.
+template <class T>
+SW_DEV void texture_run(const TexOpLaunch& L, const TexOpRun& run, T* texels)
+{
+	constexpr uint32_t N = TEXOP_PER_THREAD;
 	const uint32_t w = run.dst.w, h = run.dst.h;
 	const uint64_t n = uint64_t(w) * h;
-	const uint64_t base = uint64_t(blockIdx.x - run.first_block) * (TEXOP_BLOCK * TEXOP_PER_THREAD);
-	for(uint32_t k = 0; k < TEXOP_PER_THREAD; ++k)
+	const uint64_t base = uint64_t(blockIdx.x - run.first_block) * (TEXOP_BLOCK * N) + threadIdx.x;
+	T* dst = texels + run.dst.offset;
+	uint32_t at[N], x[N], y[N]; // threads past the end work on the last texel and store nothing
+	const bool pow2 = (w & (w - 1)) == 0;
+	const double inv_w = pow2 ? 0.0 : 1.0 / double(w);
+#pragma unroll
+	for(uint32_t k = 0; k < N; ++k)
 	{
-		const uint64_t i = base + k * TEXOP_BLOCK + threadIdx.x;
-		if(i >= n)
-			break;
-		const uint32_t y = uint32_t(i / w), x = uint32_t(i - uint64_t(y) * w);
-		if(run.lite)
+		at[k] = uint32_t(std::min<uint64_t>(base + k * TEXOP_BLOCK, n - 1)); // n <= 2^32
+		if(pow2)
 		{
-			uint32_t* d = L.lite + run.dst.offset + i;
-			uint32_t v = *d;
-			for(uint32_t o = 0; o < run.num_ops; ++o)
-			{
-				const DevTexOp& op = L.ops[run.first_op + o];
-				if(op.kind == SW_TEXOP_TURB)
-					v = L.lite[turb_index(L, op, x, y, w, h)];
-				else
-				{
-					const uint32_t su = wrap(op.shift[0] + int32_t(x), op.src.w), sv = wrap(op.shift[1] + int32_t(y), op.src.h);
-					v = lite_layer_texel(op, v, L.lite[op.src.offset + uint64_t(sv) * op.src.w + su]);
-				}
-			}
-			*d = v;
+			x[k] = at[k] & (w - 1);
+			y[k] = at[k] >> __builtin_ctz(w);
 		}
 		else
-		{
-			sw_texel* d = L.texels + run.dst.offset + i;
-			sw_texel v = *d;
-			for(uint32_t o = 0; o < run.num_ops; ++o)
-			{
-				const DevTexOp& op = L.ops[run.first_op + o];
-				if(op.kind == SW_TEXOP_TURB)
-					v = L.texels[turb_index(L, op, x, y, w, h)];
-				else
-				{
-					const uint32_t su = wrap(op.shift[0] + int32_t(x), op.src.w), sv = wrap(op.shift[1] + int32_t(y), op.src.h);
-					v = layer_texel(op, v, L.texels[op.src.offset + uint64_t(sv) * op.src.w + su]);
-				}
-			}
-			*d = v;
-		}
+			y[k] = swdiv::div_rcp(at[k], w, inv_w, x[k]);
 	}
+	T v[N], s[N];
+	const DevTexOp* ops = L.ops + run.first_op;
+	DevTexOp op = ops[0];
+	load_sources(L, run, op, texels, x, y, s);
+	if(!(run.flags & RUN_OVERWRITES))
+#pragma unroll
+		for(uint32_t k = 0; k < N; ++k)
+			v[k] = dst[at[k]];
+#pragma unroll 1
+	for(uint32_t o = 0; o < run.num_ops; ++o)
+	{
+		const DevTexOp next = ops[std::min(o + 1, run.num_ops - 1)];
+		T next_s[N];
+		if(o + 1 < run.num_ops)
+			load_sources(L, run, next, texels, x, y, next_s);
+#pragma unroll
+		for(uint32_t k = 0; k < N; ++k)
+		{
+			v[k] = op.flags & OP_TURB ? s[k] : blend_layer(op, v[k], s[k]);
+			s[k] = next_s[k];
+		}
+		op = next;
+	}
+#pragma unroll
+	for(uint32_t k = 0; k < N; ++k)
+		if(base + k * TEXOP_BLOCK < n)
+			dst[at[k]] = v[k];
+}
+
+// Bound by latency: a few hundred blocks, each a chain of run, operation and texel loads. 8 textures of
+// 256 x 256 texels and their mips, 80 operations: 15.3 us with a binary search for the run and a texel after
+// another, its row and wrapped coordinates by integer division; now 8.4 (an
+// argument record of 40 bytes rather than 96: the arguments of a call then stay below the 16 KiB from which a copy
+// costs 10 us more).
+__global__ __launch_bounds__(TEXOP_BLOCK) void k_texture_ops(TexOpLaunch L)
+{
+	// the block's run: the last run starting at or before this block, a probe per lane and level
+	const uint32_t lane = threadIdx.x & 63;
+	uint32_t lo = 0;
+	for(uint32_t n = L.num_runs; n > 1;)
+	{
+		const uint32_t step = (n + 63u) / 64u, probe = lo + lane * step;
+		const uint64_t le = __ballot(lane * step < n && L.runs[probe].first_block <= blockIdx.x);
+		const uint32_t last = 63u - uint32_t(__builtin_clzll(le)); // lane 0's run starts at or before the block
+		lo += last * step;
+		n = std::min(step, n - last * step);
+	}
+	const TexOpRun& run = L.runs[lo];
+	if(run.flags & RUN_LITE)
+		texture_run(L, run, L.lite);
+	else
+		texture_run(L, run, L.texels);
 }
 
 // make_skybox_side_texture / make_skybox_side_texture64 (textures.rs:183-229): the top-left
@@ -267,36 +349,33 @@ int pack_texture_ops(const sw_texture_op* ops, uint32_t num_ops, const sw_textur
 	for(uint32_t i = 0; i < num_ops; ++i)
 	{
 		const sw_texture_op& op = ops[i];
-		const std::string which = "texture op " + std::to_string(i) + ": ";
+		auto fail = [&](const char* what) { return (error = "texture op " + std::to_string(i) + ": " + what), -1; };
 		if(op.kind > SW_TEXOP_LAYER_LITE)
-			return (error = which + "unknown kind"), -1;
+			return fail("unknown kind");
 		if(op.dst_level >= num_levels || op.src_level >= num_levels)
-			return (error = which + "level out of range"), -1;
+			return fail("level out of range");
 		const sw_texture_level& dl = levels[op.dst_level];
 		const sw_texture_level& sl = levels[op.src_level];
 		const bool dlite = (dl.flags & SW_TEX_LITE_LEVEL) != 0, slite = (sl.flags & SW_TEX_LITE_LEVEL) != 0;
 		if(dlite != slite || (op.kind == SW_TEXOP_LAYER && dlite) || (op.kind == SW_TEXOP_LAYER_LITE && !dlite))
-			return (error = which + "level kinds do not fit the operation"), -1;
+			return fail("level kinds do not fit the operation");
 		if(op.dst_level == op.src_level)
-			return (error = which + "source and destination are the same level"), -1;
+			return fail("source and destination are the same level");
 		if(op.kind == SW_TEXOP_TURB)
 		{
 			if(sl.width != dl.width || sl.height != dl.height || (dl.width & (dl.width - 1)) || (dl.height & (dl.height - 1)))
-				return (error = which + "turbulence needs equal power-of-two sizes"), -1;
+				return fail("turbulence needs equal power-of-two sizes");
 			if(uint64_t(op.turb_shifts) + std::max(dl.width, dl.height) > num_turb_shifts)
-				return (error = which + "turbulence shifts out of range"), -1;
+				return fail("turbulence shifts out of range");
 		}
 		else if(op.blend > SW_BLEND_ALPHA_BLEND)
-			return (error = which + "unknown blending mode"), -1;
+			return fail("unknown blending mode");
 		DevTexOp& d = dops[i];
-		d.kind = op.kind;
-		d.blend = op.blend;
-		d.modulate = 0;
+		d.flags = op.kind == SW_TEXOP_TURB ? OP_TURB : op.blend << OP_BLEND_SHIFT;
 		for(int c = 0; c < 3; ++c)
-			d.modulate |= (op.light[c] < 0.98f || op.light[c] > 1.02f) ? 1u : 0u;
+			d.flags |= (op.light[c] < 0.98f || op.light[c] > 1.02f) ? OP_MODULATE : 0u;
 		d.turb_shifts = op.turb_shifts;
-		d.shift[0] = op.shift[0];
-		d.shift[1] = op.shift[1];
+		d.shift_v = op.shift[1];
 		// ColorVecI::from_color_f32x3(light * 256): cvtps2dq (round half even, "integer indefinite"
 		// out of range), lanes B, G, R
 		for(int c = 0; c < 3; ++c)
@@ -305,17 +384,27 @@ int pack_texture_ops(const sw_texture_op* ops, uint32_t num_ops, const sw_textur
 			d.light_vec[c] = (v >= -2147483648.0f && v < 2147483648.0f) ? int32_t(std::nearbyint(v)) : INT32_MIN;
 		}
 		d.src = TexLevel{sl.offset, sl.width, sl.height};
+		const uint32_t src_size[2] = {sl.width, sl.height};
+		for(int c = 0; c < 2; ++c)
+		{
+			const int64_t size = src_size[c];
+			const bool pow2 = (size & (size - 1)) == 0;
+			d.add[c] = pow2 ? uint32_t(op.shift[c]) : uint32_t((op.shift[c] % size + size) % size);
+			if(c == 1 && !pow2 && int64_t(op.shift[1]) + dl.height > INT32_MAX)
+				d.flags |= OP_OVERFLOWS;
+		}
 		if(runs.empty() || ops[runs.back().first_op].dst_level != op.dst_level)
 		{
 			for(const TexOpRun& r : runs)
 				if(ops[r.first_op].dst_level == op.dst_level)
-					return (error = which + "a destination's operations must be consecutive"), -1;
+					return fail("a destination's operations must be consecutive");
 			TexOpRun r{};
 			r.first_op = i;
 			r.num_ops = 0;
 			r.first_block = blocks;
-			r.lite = dlite ? 1u : 0u;
 			r.dst = TexLevel{dl.offset, dl.width, dl.height};
+			// SW_BLEND_NONE: as layer_texel and lite_layer_texel do
+			r.flags = (dlite ? RUN_LITE : 0u) | (op.kind == SW_TEXOP_TURB || op.blend == SW_BLEND_NONE ? RUN_OVERWRITES : 0u);
 			const uint64_t nb = (uint64_t(dl.width) * dl.height + TEXOP_BLOCK * TEXOP_PER_THREAD - 1) / (TEXOP_BLOCK * TEXOP_PER_THREAD);
 			if(blocks + nb > 0x7FFFFFFFull)
 				return (error = "texture ops: too many texels"), -1;
