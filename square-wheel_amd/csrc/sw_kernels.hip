@@ -2997,6 +2997,23 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t value)
 		p[i] = value;
 }
 
+// A block takes COPY_BLOCK_BYTES of a range, a lane 16 bytes: reads over the bus are bound by their latency, so all
+// of them are in flight at once: the five arrays of a 320 x 200 frame 3.2 us, of 13 views 6.5.
+__global__ __launch_bounds__(256) void k_copy_pieces(const swk::CopyPieces p)
+{
+	uint32_t i = 0;
+	while(i + 1 < p.count && blockIdx.x >= p.first_block[i + 1])
+		++i;
+	const uint64_t bytes = p.piece[i].bytes, at = uint64_t(blockIdx.x - p.first_block[i]) * swk::COPY_BLOCK_BYTES + threadIdx.x * 16u;
+	const char* src = static_cast<const char*>(p.piece[i].src) + at;
+	char* dst = static_cast<char*>(p.piece[i].dst) + at;
+	if(at + 16 <= bytes)
+		*reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
+	else
+		for(uint32_t b = 0; at + b < bytes; b += 4)
+			*reinterpret_cast<uint32_t*>(dst + b) = *reinterpret_cast<const uint32_t*>(src + b);
+}
+
 // =============================================================================================
 // Launch wrappers (called from the host runtime)
 // =============================================================================================
@@ -3185,6 +3202,18 @@ void launch_bloom(hipStream_t st, const BloomArgs& a, bool average)
 		hipLaunchKernelGGL(k_bloom_tonemap<true>, grid, dim3(256), 0, st, a, bloom, with_average);
 	else
 		hipLaunchKernelGGL(k_bloom_tonemap<false>, grid, dim3(256), 0, st, a, bloom, with_average);
+}
+
+void launch_copy_pieces(hipStream_t st, CopyPieces p)
+{
+	uint32_t blocks = 0;
+	for(uint32_t i = 0; i < p.count; ++i)
+	{
+		p.first_block[i] = blocks;
+		blocks += uint32_t((p.piece[i].bytes + COPY_BLOCK_BYTES - 1) / COPY_BLOCK_BYTES);
+	}
+	if(blocks)
+		hipLaunchKernelGGL(k_copy_pieces, dim3(blocks), dim3(256), 0, st, p);
 }
 
 void launch_portal_mix(hipStream_t st, uint32_t color_bits, const uint32_t* lite, const PortalMixRec* recs, uint32_t num,

@@ -139,6 +139,13 @@ struct sw_ctx
 	char* arg_staging[ARG_STAGING_SLOTS] = {};
 	void* arg_staging_dev[ARG_STAGING_SLOTS] = {}; // their device addresses
 	size_t arg_staging_cap[ARG_STAGING_SLOTS] = {};
+	struct
+	{
+		char* host = nullptr; // the slot being filled while pieces.count > 0, and its device address
+		const char* dev = nullptr;
+		size_t used = 0, cap = 0, want = 256 << 10;
+		swk::CopyPieces pieces{};
+	} uploads; // queue_upload
 	hipEvent_t arg_staging_event[ARG_STAGING_SLOTS] = {}; // recorded after the last copy out of the slot
 	uint32_t arg_staging_slot = 0; // the slot of the current stage_begin
 	std::vector<char> texop_packed;
@@ -239,6 +246,106 @@ int upload(sw_ctx* ctx, DevBuf& b, const void* src, size_t bytes)
 	if(bytes == 0)
 		return SW_OK;
 	return hip_check(ctx, hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync H2D");
+}
+
+// Small launch arguments travel from pinned staging memory. stage_begin takes the next slot of the
+// ring, waits until the copies out of it (ARG_STAGING_SLOTS calls ago) have completed (its event),
+// grows it if needed and returns it (and its device address); stage_copy queues a copy out of the slot
+// (at src_offset) and records the slot's event after it; a launch that reads the slot itself is followed by
+// stage_used.
+int stage_used(sw_ctx* ctx)
+{
+	return hip_check(ctx, hipEventRecord(ctx->arg_staging_event[ctx->arg_staging_slot], ctx->stream), "argument staging event");
+}
+
+// Starts the copies of the queued uploads (queue_upload); before the first launch that reads them.
+int flush_uploads(sw_ctx* ctx)
+{
+	swk::CopyPieces& p = ctx->uploads.pieces;
+	if(p.count == 0)
+		return SW_OK;
+	swk::launch_copy_pieces(ctx->stream, p);
+	p.count = 0;
+	const int r = hip_check(ctx, hipGetLastError(), "upload launch");
+	return r ? r : stage_used(ctx);
+}
+
+int stage_begin(sw_ctx* ctx, size_t bytes, char** out, const char** out_device = nullptr)
+{
+	int r;
+	if((r = flush_uploads(ctx))) // the queue holds a slot until then
+		return r;
+	const uint32_t k = (ctx->arg_staging_slot + 1) % ARG_STAGING_SLOTS;
+	ctx->arg_staging_slot = k;
+	if(ctx->arg_staging_event[k] && (r = hip_check(ctx, hipEventSynchronize(ctx->arg_staging_event[k]), "argument staging wait")))
+		return r;
+	if(bytes > ctx->arg_staging_cap[k])
+	{
+		if(ctx->arg_staging[k])
+			(void)hipHostFree(ctx->arg_staging[k]);
+		ctx->arg_staging[k] = nullptr;
+		ctx->arg_staging_cap[k] = 0;
+		const size_t cap = std::max<size_t>(bytes * 2, 64 << 10);
+		if((r = hip_check(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->arg_staging[k]), cap, hipHostMallocMapped),
+				"argument staging allocation")) ||
+			(r = hip_check(ctx, hipHostGetDevicePointer(&ctx->arg_staging_dev[k], ctx->arg_staging[k], 0), "argument staging address")))
+			return r;
+		ctx->arg_staging_cap[k] = cap;
+	}
+	if(!ctx->arg_staging_event[k] &&
+		(r = hip_check(ctx, hipEventCreateWithFlags(&ctx->arg_staging_event[k], hipEventDisableTiming), "argument staging event")))
+		return r;
+	*out = ctx->arg_staging[k];
+	if(out_device)
+		*out_device = static_cast<const char*>(ctx->arg_staging_dev[k]);
+	return SW_OK;
+}
+
+int stage_copy(sw_ctx* ctx, void* dst_device, size_t bytes, size_t src_offset = 0)
+{
+	int r;
+	const uint32_t k = ctx->arg_staging_slot;
+	if((r = hip_check(ctx, hipMemcpyAsync(dst_device, ctx->arg_staging[k] + src_offset, bytes, hipMemcpyHostToDevice, ctx->stream),
+			"argument copy")))
+		return r;
+	return stage_used(ctx);
+}
+
+// A host array of a frame or batch for device buffer b: copied into pinned memory here, from there to the device
+// by one launch for all of a call's arrays (flush_uploads). A copy of its own costs each array 4 to 8 us and
+// from 16 KiB on 10 more (the DMA engine's), most of a small frame's time.
+const size_t UPLOAD_PIECE_MAX = 1 << 20, UPLOAD_SLOT_MAX = 4 << 20;
+int queue_upload(sw_ctx* ctx, DevBuf& b, const void* src, size_t bytes)
+{
+	auto& q = ctx->uploads;
+	swk::CopyPieces& p = q.pieces;
+	int r;
+	for(uint32_t i = 0; i < p.count; ++i)
+		if(p.piece[i].dst == b.p && (r = flush_uploads(ctx)))
+			return r;
+	if(bytes > UPLOAD_PIECE_MAX)
+		return upload(ctx, b, src, bytes);
+	if((r = ensure(ctx, b, bytes)) || bytes == 0)
+		return r;
+	size_t at = (q.used + 15) & ~size_t(15);
+	if(p.count && (p.count == swk::COPY_PIECES_MAX || at + bytes > q.cap))
+	{
+		if(at + bytes > q.cap)
+			q.want = std::min(2 * (q.cap + bytes), UPLOAD_SLOT_MAX);
+		if((r = flush_uploads(ctx)))
+			return r;
+	}
+	if(p.count == 0)
+	{
+		if((r = stage_begin(ctx, std::max(bytes, q.want), &q.host, &q.dev)))
+			return r;
+		q.cap = ctx->arg_staging_cap[ctx->arg_staging_slot];
+		at = 0;
+	}
+	std::memcpy(q.host + at, src, bytes);
+	p.piece[p.count++] = swk::CopyPiece{q.dev + at, b.p, bytes};
+	q.used = at + bytes;
+	return SW_OK;
 }
 
 uint64_t color_bytes(uint32_t bits) { return bits == 64 ? 8 : 4; }
@@ -428,7 +535,7 @@ int set_views(sw_ctx* ctx, const std::vector<ViewExt>& ve, bool allow_inline)
 		va.ptr = nullptr;
 		return SW_OK;
 	}
-	int r = upload(ctx, ctx->views, ve.data(), sizeof(ViewExt) * ve.size());
+	int r = queue_upload(ctx, ctx->views, ve.data(), sizeof(ViewExt) * ve.size());
 	if(r)
 		return r;
 	va.inline_one = 0;
@@ -621,8 +728,8 @@ int host_prepare_surfaces(sw_ctx* ctx, const sw_map* map, const std::vector<View
 			blk[b] = i;
 		prev_end = end;
 	}
-	int r = upload(ctx, ctx->surf_ext, ext.data(), sizeof(SurfExt) * ext.size());
-	return r ? r : upload(ctx, ctx->blk_surf, blk.data(), sizeof(uint32_t) * blk.size());
+	int r = queue_upload(ctx, ctx->surf_ext, ext.data(), sizeof(SurfExt) * ext.size());
+	return r ? r : queue_upload(ctx, ctx->blk_surf, blk.data(), sizeof(uint32_t) * blk.size());
 }
 
 // The result block k_finish wrote into host memory -> the pixel statistics.
@@ -796,6 +903,8 @@ int launch_frame(sw_ctx* ctx, uint32_t num_draws, uint64_t num_vertex_ints, bool
 	L.fb = ctx->fb.p;
 	L.portal = ctx->portal_texels;
 	L.num_portal = ctx->portal_texels ? ctx->num_portal_texels : 0;
+	if((r = flush_uploads(ctx)))
+		return r;
 	const bool surfaces = ctx->frame_surfaces_pending;
 	ctx->frame_surfaces_pending = false;
 	if(!raster && !surfaces)
@@ -1073,11 +1182,11 @@ int sw_build_surfaces(sw_ctx* ctx, const sw_surface_desc* surfaces, uint32_t num
 	int r;
 	if((r = ensure(ctx, ctx->arena, std::max<uint64_t>(arena, 1) * color_bytes(ctx->frame_color_bits))))
 		return r;
-	if((r = upload(ctx, ctx->surfaces, surfaces, sizeof(sw_surface_desc) * num_surfaces)))
+	if((r = queue_upload(ctx, ctx->surfaces, surfaces, sizeof(sw_surface_desc) * num_surfaces)))
 		return r;
-	if((r = upload(ctx, ctx->lights, lights, sizeof(sw_light) * (lights ? num_lights : 0))))
+	if((r = queue_upload(ctx, ctx->lights, lights, sizeof(sw_light) * (lights ? num_lights : 0))))
 		return r;
-	if((r = upload(ctx, ctx->light_indices, light_indices, sizeof(uint32_t) * (light_indices ? num_light_indices : 0))))
+	if((r = queue_upload(ctx, ctx->light_indices, light_indices, sizeof(uint32_t) * (light_indices ? num_light_indices : 0))))
 		return r;
 	ctx->frame_arena_texels = arena;
 	ctx->last_color_bits = ctx->frame_color_bits;
@@ -1110,9 +1219,9 @@ int sw_raster_draws(sw_ctx* ctx, const sw_draw* draws, uint32_t num_draws, const
 		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "null draws / vertex data");
 	(void)hipSetDevice(ctx->device);
 	int r;
-	if((r = upload(ctx, ctx->draws, draws, sizeof(sw_draw) * num_draws)))
+	if((r = queue_upload(ctx, ctx->draws, draws, sizeof(sw_draw) * num_draws)))
 		return r;
-	if((r = upload(ctx, ctx->vdata, vertex_data, sizeof(int32_t) * num_vertex_ints)))
+	if((r = queue_upload(ctx, ctx->vdata, vertex_data, sizeof(int32_t) * num_vertex_ints)))
 		return r;
 	if((r = launch_frame(ctx, num_draws, num_vertex_ints, true)))
 		return r;
@@ -1357,55 +1466,6 @@ int sw_postprocess_device(sw_ctx* ctx, const void* hdr_device, uint32_t width, u
 		out_average_rgb[2] = avg[0];
 	}
 	return SW_OK;
-}
-
-// Small launch arguments travel from pinned staging memory. stage_begin takes the next slot of the
-// ring, waits until the copies out of it (ARG_STAGING_SLOTS calls ago) have completed (its event),
-// grows it if needed and returns it (and its device address); stage_copy queues a copy out of the slot
-// (at src_offset) and records the slot's event after it; a launch that reads the slot itself is followed by
-// stage_used.
-static int stage_used(sw_ctx* ctx)
-{
-	return hip_check(ctx, hipEventRecord(ctx->arg_staging_event[ctx->arg_staging_slot], ctx->stream), "argument staging event");
-}
-
-static int stage_begin(sw_ctx* ctx, size_t bytes, char** out, const char** out_device = nullptr)
-{
-	int r;
-	const uint32_t k = (ctx->arg_staging_slot + 1) % ARG_STAGING_SLOTS;
-	ctx->arg_staging_slot = k;
-	if(ctx->arg_staging_event[k] && (r = hip_check(ctx, hipEventSynchronize(ctx->arg_staging_event[k]), "argument staging wait")))
-		return r;
-	if(bytes > ctx->arg_staging_cap[k])
-	{
-		if(ctx->arg_staging[k])
-			(void)hipHostFree(ctx->arg_staging[k]);
-		ctx->arg_staging[k] = nullptr;
-		ctx->arg_staging_cap[k] = 0;
-		const size_t cap = std::max<size_t>(bytes * 2, 64 << 10);
-		if((r = hip_check(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->arg_staging[k]), cap, hipHostMallocMapped),
-				"argument staging allocation")) ||
-			(r = hip_check(ctx, hipHostGetDevicePointer(&ctx->arg_staging_dev[k], ctx->arg_staging[k], 0), "argument staging address")))
-			return r;
-		ctx->arg_staging_cap[k] = cap;
-	}
-	if(!ctx->arg_staging_event[k] &&
-		(r = hip_check(ctx, hipEventCreateWithFlags(&ctx->arg_staging_event[k], hipEventDisableTiming), "argument staging event")))
-		return r;
-	*out = ctx->arg_staging[k];
-	if(out_device)
-		*out_device = static_cast<const char*>(ctx->arg_staging_dev[k]);
-	return SW_OK;
-}
-
-static int stage_copy(sw_ctx* ctx, void* dst_device, size_t bytes, size_t src_offset = 0)
-{
-	int r;
-	const uint32_t k = ctx->arg_staging_slot;
-	if((r = hip_check(ctx, hipMemcpyAsync(dst_device, ctx->arg_staging[k] + src_offset, bytes, hipMemcpyHostToDevice, ctx->stream),
-			"argument copy")))
-		return r;
-	return stage_used(ctx);
 }
 
 int sw_mix_portal_textures(sw_ctx* ctx, sw_map* map, uint32_t color_bits, const sw_portal_mix* mixes, uint32_t num_mixes,
@@ -2163,15 +2223,15 @@ static int prepare_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_
 	}
 	else
 	{
-		if((r = upload(ctx, ctx->surfaces, b->surfaces, sizeof(sw_surface_desc) * b->num_surfaces)))
+		if((r = queue_upload(ctx, ctx->surfaces, b->surfaces, sizeof(sw_surface_desc) * b->num_surfaces)))
 			return r;
-		if((r = upload(ctx, ctx->lights, b->lights, sizeof(sw_light) * L.num_lights)))
+		if((r = queue_upload(ctx, ctx->lights, b->lights, sizeof(sw_light) * L.num_lights)))
 			return r;
-		if((r = upload(ctx, ctx->light_indices, b->light_indices, sizeof(uint32_t) * L.num_light_indices)))
+		if((r = queue_upload(ctx, ctx->light_indices, b->light_indices, sizeof(uint32_t) * L.num_light_indices)))
 			return r;
-		if((r = upload(ctx, ctx->draws, b->draws, sizeof(sw_draw) * b->num_draws)))
+		if((r = queue_upload(ctx, ctx->draws, b->draws, sizeof(sw_draw) * b->num_draws)))
 			return r;
-		if((r = upload(ctx, ctx->vdata, b->vertex_data, sizeof(int32_t) * b->num_vertex_ints)))
+		if((r = queue_upload(ctx, ctx->vdata, b->vertex_data, sizeof(int32_t) * b->num_vertex_ints)))
 			return r;
 		L.surfaces = static_cast<const sw_surface_desc*>(ctx->surfaces.p);
 		L.lights = static_cast<const sw_light*>(ctx->lights.p);
@@ -2188,7 +2248,7 @@ static int prepare_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_
 	}
 	if(b->num_views == 1)
 		L.surface_mode = SURF_SEARCH;
-	return SW_OK;
+	return flush_uploads(ctx);
 }
 
 int sw_render_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_fb)
@@ -2352,7 +2412,7 @@ int sw_render_batch_graph(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out
 		uint32_t tiles = 0, tile_width = 0;
 		if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, tiles, tile_width)) ||
 			(r = validate_views_fit(ctx, ve, b->framebuffer_texels, b->num_surfaces, b->num_draws)) ||
-			(r = set_views(ctx, ve, false)))
+			(r = set_views(ctx, ve, false)) || (r = flush_uploads(ctx)))
 			return r;
 		ctx->graph_views_hash = views_hash;
 	}
