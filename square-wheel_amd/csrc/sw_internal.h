@@ -272,8 +272,8 @@ void launch_tonemap(hipStream_t st, const uint64_t* hdr, uint32_t w, uint32_t h,
 // vertex int, first fan-count byte), device copies of runs and bases; the host checked every range.
 void launch_expand_mesh_runs(hipStream_t st, const sw_mesh_run* runs, uint32_t num_runs, uint32_t max_triangles, const uint64_t* bases,
 	const sw_model_vertex* vertices, const uint16_t* triangles, const uint32_t* counts, int32_t* out_ints, uint8_t* out_fans);
-// Copies of up to COPY_PIECES_MAX ranges (16-byte aligned, multiples of 4 bytes) in one launch: device-visible host
-// memory to the device.
+// Copies of up to COPY_PIECES_MAX ranges (16-byte aligned, multiples of 4 bytes) in one launch, between the device
+// and host memory it can address; none if *skip (may be null) is set.
 const uint32_t COPY_PIECES_MAX = 8, COPY_BLOCK_BYTES = 4096;
 struct CopyPiece
 {
@@ -286,6 +286,7 @@ struct CopyPieces
 	CopyPiece piece[COPY_PIECES_MAX];
 	uint32_t first_block[COPY_PIECES_MAX]; // filled by the launch
 	uint32_t count;
+	const uint32_t* skip;
 };
 void launch_copy_pieces(hipStream_t st, CopyPieces p);
 // Triangle-model preparation: one block per instance. recs is device-visible; scratch holds the sort keys of

@@ -1229,6 +1229,32 @@ int sw_raster_draws(sw_ctx* ctx, const sw_draw* draws, uint32_t num_draws, const
 	return SW_OK;
 }
 
+// Queues the copy of a finished frame into dst if that is pinned memory a kernel may write (16-byte aligned, the
+// whole range in one allocation); the kernel leaves dst alone after an error. The frame's one synchronisation
+// then covers it. A copy by the DMA engine is queued after that one and waited for by a second.
+static int queue_copy_to_pinned(sw_ctx* ctx, void* dst, const void* src, size_t bytes, bool* queued)
+{
+	hipPointerAttribute_t attr;
+	hipDeviceptr_t base = nullptr;
+	size_t size = 0;
+	if(reinterpret_cast<uintptr_t>(dst) % 16 || hipPointerGetAttributes(&attr, dst) != hipSuccess || attr.type != hipMemoryTypeHost ||
+		!attr.devicePointer || hipMemGetAddressRange(&base, &size, attr.devicePointer) != hipSuccess)
+	{
+		(void)hipGetLastError();
+		return SW_OK;
+	}
+	const uintptr_t at = reinterpret_cast<uintptr_t>(attr.devicePointer), first = reinterpret_cast<uintptr_t>(base);
+	if(at % 16 || at < first || at - first > size || bytes > size - (at - first))
+		return SW_OK;
+	swk::CopyPieces p{};
+	p.count = 1;
+	p.piece[0] = swk::CopyPiece{src, attr.devicePointer, bytes};
+	p.skip = static_cast<uint32_t*>(ctx->counters.p) + COUNTER_ERROR;
+	swk::launch_copy_pieces(ctx->stream, p);
+	*queued = true;
+	return hip_check(ctx, hipGetLastError(), "frame copy launch");
+}
+
 int sw_frame_end(sw_ctx* ctx, void* dst, size_t dst_pitch_bytes, uint32_t dst_on_device)
 {
 	if(!ctx || !ctx->frame_active)
@@ -1241,11 +1267,15 @@ int sw_frame_end(sw_ctx* ctx, void* dst, size_t dst_pitch_bytes, uint32_t dst_on
 		if((r = sw_raster_draws(ctx, nullptr, 0, nullptr, 0)))
 			return r;
 	}
+	const size_t row = size_t(ctx->frame_view.width) * color_bytes(ctx->frame_color_bits);
+	bool copied = false;
+	if(dst && !dst_on_device && dst_pitch_bytes == row && !ctx->finish_launched && !ctx->surface_error)
+		if((r = queue_copy_to_pinned(ctx, dst, ctx->fb.p, row * ctx->frame_view.height, &copied)))
+			return r;
 	if((r = finish(ctx)))
 		return r;
-	if(dst)
+	if(dst && !copied)
 	{
-		const size_t row = size_t(ctx->frame_view.width) * color_bytes(ctx->frame_color_bits);
 		if(dst_pitch_bytes < row)
 			return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "dst pitch smaller than a row");
 		if((r = hip_check(ctx,
