@@ -2063,14 +2063,15 @@ __global__ __launch_bounds__(256) void k_setup_draws(SetupArgs a, const ViewsArg
 // Draw setup and surface texels in one launch (the host prepared and validated the surfaces): the
 // two are independent, so they run side by side. Held to 96 VGPRs: five waves per SIMD.
 // With shadowed lights (SH) too: a 1920 x 1080 frame with shadow maps took 10.0 us for the setup and then 15.8
-// for the surfaces, together 15.3.
-template <int LANES, class CT, bool SH>
+// for the surfaces, together 15.3. With lightmap lines (LINES) from SURF_LINES_MIN_TEXELS on: 13 views of 320 to
+// 2560 pixels of width in Color64 from host memory 44.2 us, 47.0 without them, 15.3 + 38.9 in two launches.
+template <int LANES, class CT, bool SH, bool LINES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_setup_and_surfaces(SetupArgs a, const ViewsArg views, SurfaceArgs sa, MapPtrs m)
 {
 	if(blockIdx.x < a.setup_blocks)
 		setup_draws_block<LANES>(blockIdx.x, a, views);
 	else
-		build_surfaces_block<CT, SH, false>(blockIdx.x - a.setup_blocks, m, sa, views);
+		build_surfaces_block<CT, SH, LINES>(blockIdx.x - a.setup_blocks, m, sa, views);
 }
 
 // One block after the raster kernel: sums the per-draw statistics into the result block and clears
@@ -3067,10 +3068,18 @@ static void launch_fused_lanes(hipStream_t st, uint32_t color_bits, uint32_t blo
 	const SurfaceArgs& sa, const MapPtrs& m)
 {
 	auto launch = [&](auto kernel) { timed_launch(kernel, dim3(blocks), dim3(256), 0, st, a, views, sa, m); };
+	const bool lines = surf_block_texels(sa.arena_texels) >= SURF_LINES_MIN_TEXELS;
+	auto of_color = [&](auto ct) {
+		typedef decltype(ct) CT;
+		if(sa.num_shadows)
+			lines ? launch(k_setup_and_surfaces<LANES, CT, true, true>) : launch(k_setup_and_surfaces<LANES, CT, true, false>);
+		else
+			lines ? launch(k_setup_and_surfaces<LANES, CT, false, true>) : launch(k_setup_and_surfaces<LANES, CT, false, false>);
+	};
 	if(color_bits == 64)
-		sa.num_shadows ? launch(k_setup_and_surfaces<LANES, Color64T, true>) : launch(k_setup_and_surfaces<LANES, Color64T, false>);
+		of_color(Color64T{});
 	else
-		sa.num_shadows ? launch(k_setup_and_surfaces<LANES, Color32T, true>) : launch(k_setup_and_surfaces<LANES, Color32T, false>);
+		of_color(Color32T{});
 }
 
 void launch_setup_and_surfaces(hipStream_t st, uint32_t lanes, uint32_t color_bits, SetupArgs a, const ViewsArg& views,

@@ -626,20 +626,7 @@ int launch_stages(sw_ctx* ctx, const sw_ctx::Launch& L, bool surfaces, bool rast
 	sa.shadow_texels = ctx->shadow_texels;
 	// a block per draw while the draws alone cannot fill the chip, a wave per draw beyond
 	const uint32_t lanes = nd <= 4096 ? 256u : 64u;
-	if(surfaces && L.surface_mode != SURF_TABLE_DEVICE && ctx->num_shadows && surf_bt >= SURF_LINES_MIN_TEXELS)
-	{
-		// shadowed lights and enough texels to stage lightmap lines: the surface kernel runs on its own after
-		// the setup (whose table blocks are not needed: the host prepared the table, or the surface blocks
-		// search)
-		{
-			StageTimer t(ctx, STAGE_SETUP);
-			swk::launch_setup(ctx->stream, lanes, a, ctx->views_arg, L.surfaces, 0, static_cast<SurfExt*>(ctx->surf_ext.p),
-				static_cast<uint32_t*>(ctx->blk_surf.p), mp);
-		}
-		StageTimer t(ctx, STAGE_SURF);
-		swk::launch_build_surfaces(ctx->stream, L.color_bits, mp, sa, ctx->views_arg, counters);
-	}
-	else if(surfaces && L.surface_mode != SURF_TABLE_DEVICE)
+	if(surfaces && L.surface_mode != SURF_TABLE_DEVICE)
 	{
 		StageTimer t(ctx, STAGE_SETUP_SURF);
 		swk::launch_setup_and_surfaces(ctx->stream, lanes, L.color_bits, a, ctx->views_arg, sa, mp);
