@@ -345,6 +345,7 @@ int pack_texture_ops(const sw_texture_op* ops, uint32_t num_ops, const sw_textur
 {
 	std::vector<TexOpRun> runs;
 	std::vector<DevTexOp> dops(num_ops);
+	std::vector<uint8_t> is_dst(num_levels, 0); // levels that a run writes
 	uint32_t blocks = 0;
 	for(uint32_t i = 0; i < num_ops; ++i)
 	{
@@ -395,9 +396,9 @@ int pack_texture_ops(const sw_texture_op* ops, uint32_t num_ops, const sw_textur
 		}
 		if(runs.empty() || ops[runs.back().first_op].dst_level != op.dst_level)
 		{
-			for(const TexOpRun& r : runs)
-				if(ops[r.first_op].dst_level == op.dst_level)
-					return fail("a destination's operations must be consecutive");
+			if(is_dst[op.dst_level])
+				return fail("a destination's operations must be consecutive");
+			is_dst[op.dst_level] = 1;
 			TexOpRun r{};
 			r.first_op = i;
 			r.num_ops = 0;
@@ -414,9 +415,8 @@ int pack_texture_ops(const sw_texture_op* ops, uint32_t num_ops, const sw_textur
 		runs.back().num_ops++;
 	}
 	for(uint32_t i = 0; i < num_ops; ++i)
-		for(const TexOpRun& r : runs)
-			if(ops[i].src_level == ops[r.first_op].dst_level)
-				return (error = "texture op " + std::to_string(i) + ": its source is the destination of another operation"), -1;
+		if(is_dst[ops[i].src_level])
+			return (error = "texture op " + std::to_string(i) + ": its source is the destination of another operation"), -1;
 	const size_t runs_bytes = sizeof(TexOpRun) * runs.size();
 	plan.ops_at = (runs_bytes + 255) & ~size_t(255);
 	plan.bytes = plan.ops_at + sizeof(DevTexOp) * dops.size();
