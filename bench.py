@@ -205,7 +205,7 @@ def hdr_leg(ctx, args):
 
     tris = [int(np.sum(f["draws"]["kind"] == sw_abi.DRAW_TRIANGLE)) for f in frames]
     rows, tune = ctx.autotune_many(mh, batches[::4], dev[::4], hdr)
-    log(f"autotune (hdr): {rows} rows, scalar spans {ctx.scalar_spans()}; ms per frame by rows {tune}")
+    log(f"autotune (hdr): {rows} rows; ms per frame by rows {tune}")
     for i in range(4 * len(cbs)):
         step(i)
     ctx.profile_read(reset=True)
@@ -733,7 +733,7 @@ def main():
 
     # tile height and span mode for this frame size, chosen by the autotuner on every fourth pose
     plain_rows, plain_tune = ctx.autotune_many(mh, batches[::4], dev[::4], out)
-    log(f"autotune (plain): {plain_rows} rows, scalar spans {ctx.scalar_spans()}; ms per frame by rows {plain_tune}")
+    log(f"autotune (plain): {plain_rows} rows; ms per frame by rows {plain_tune}")
     for i in range(args.warmup):
         render(i)
     # Timed region: K frames of the path, each call returns with its frame finished.
