@@ -2220,6 +2220,10 @@ static int prepare_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_
 		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "null argument");
 	if(b->color_bits != 32 && b->color_bits != 64)
 		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "color_bits must be 32 or 64");
+	// the arrays are read here, by the CPU
+	if(!b->inputs_on_device &&
+		((b->num_surfaces && !b->surfaces) || (b->num_draws && !b->draws) || (b->num_vertex_ints && !b->vertex_data)))
+		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "null surfaces, draws or vertex data");
 	int r;
 	if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, L.total_tiles, L.tile_width, &L.max_view_height)))
 		return r;

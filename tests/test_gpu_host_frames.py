@@ -9,6 +9,7 @@ import torch
 
 import oracle
 import scenes
+import sw_abi as A
 
 pytestmark = pytest.mark.gpu
 
@@ -77,5 +78,26 @@ def test_batch_arrays_past_the_queued_size(gpu_ctx):
     try:
         for _ in range(3):
             assert np.array_equal(gpu_ctx.render_batch(mh, b), ref)
+    finally:
+        gpu_ctx.release_map(mh)
+
+
+@pytest.mark.parametrize("views", [1, 2])
+@pytest.mark.parametrize("missing", ["surfaces", "draws", "vertex_data"])
+def test_missing_host_array_is_an_error(gpu_ctx, missing, views):
+    """A null array with a count is refused before any of the batch is read or queued, synchronously and not, and the
+    next batch of the context is drawn as usual."""
+    print(f"case missing {missing} views={views}", flush=True)
+    m, b = scenes.make_batch(44, view_sizes=((64, 48),) * views)
+    ref = oracle.render(m, b, mode=oracle.MODE_EXACT)[0]
+    out = torch.zeros(b.fb_texels, dtype=torch.int32, device="cuda")
+    mh = gpu_ctx.upload_map(m)
+    try:
+        cb = b.ctypes_batch()
+        setattr(cb, missing, None)
+        for render in (gpu_ctx.lib.sw_render_batch, gpu_ctx.lib.sw_render_batch_async):
+            with pytest.raises(A.SwError, match="null surfaces, draws or vertex data"):
+                gpu_ctx.check(render(gpu_ctx.h, mh, C.byref(cb), _p(out)), "render")
+        assert np.array_equal(gpu_ctx.render_batch(mh, b), ref)
     finally:
         gpu_ctx.release_map(mh)
