@@ -254,7 +254,8 @@ void launch_build_surfaces(hipStream_t st, uint32_t color_bits, const MapPtrs& m
 void launch_setup_and_surfaces(hipStream_t st, uint32_t lanes, uint32_t color_bits, SetupArgs a, const ViewsArg& views,
 	const SurfaceArgs& sa, const MapPtrs& m);
 // Kernel 3: one wave per tile_width x tile_rows tile (binning fused); widths 16, 32, 64, rows 4, 8, 16 (at most 512 pixels).
-void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
+// false for a size that has no kernel.
+bool launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
 	const DrawBounds* bounds, const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views, const void* arena,
 	const void* skybox, void* fb, uint32_t total_tiles, const uint32_t* counters);
 // Kernel 4 (one block): per-draw statistics -> result block (host-mapped), live block cleared.

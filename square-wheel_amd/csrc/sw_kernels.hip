@@ -3133,38 +3133,42 @@ void launch_build_surfaces(hipStream_t st, uint32_t color_bits, const MapPtrs& m
 
 // The tile sizes of raster_tile_width (sw_runtime.hip): at most 512 pixels.
 template <class CT>
-static void launch_raster_ct(hipStream_t st, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m, const DrawBounds* bounds,
+static bool launch_raster_ct(hipStream_t st, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m, const DrawBounds* bounds,
 	const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views, const void* arena, const void* skybox,
 	void* fb, uint32_t total_tiles, const uint32_t* counters)
 {
 	typedef typename CT::T C;
 	const uint32_t blocks = (total_tiles + 3) / 4;
 	if(blocks == 0)
-		return;
+		return true;
 	auto launch = [&](auto kernel) {
 		timed_launch(kernel, dim3(blocks), dim3(256), 0, st, m, bounds, drec, parts, spans, views, static_cast<const C*>(arena),
 			static_cast<const C*>(skybox), static_cast<C*>(fb), total_tiles, counters);
+		return true;
 	};
-	if(tile_rows == 4)
-		tile_width == 64   ? launch(k_raster_tiles<CT, 4, 4>)
-		: tile_width == 32 ? launch(k_raster_tiles<CT, 4, 2>)
-						   : launch(k_raster_tiles<CT, 4, 1>);
-	else if(tile_rows == 8)
-		tile_width == 64   ? launch(k_raster_tiles<CT, 8, 4>)
-		: tile_width == 32 ? launch(k_raster_tiles<CT, 8, 2>)
-						   : launch(k_raster_tiles<CT, 8, 1>);
-	else
-		tile_width == 32 ? launch(k_raster_tiles<CT, 16, 2>) : launch(k_raster_tiles<CT, 16, 1>);
+	switch(tile_rows * 256u + tile_width)
+	{
+	case 4 * 256 + 64: return launch(k_raster_tiles<CT, 4, 4>);
+	case 4 * 256 + 32: return launch(k_raster_tiles<CT, 4, 2>);
+	case 4 * 256 + 16: return launch(k_raster_tiles<CT, 4, 1>);
+	case 8 * 256 + 64: return launch(k_raster_tiles<CT, 8, 4>);
+	case 8 * 256 + 32: return launch(k_raster_tiles<CT, 8, 2>);
+	case 8 * 256 + 16: return launch(k_raster_tiles<CT, 8, 1>);
+	case 16 * 256 + 32: return launch(k_raster_tiles<CT, 16, 2>);
+	case 16 * 256 + 16: return launch(k_raster_tiles<CT, 16, 1>);
+	default: return false;
+	}
 }
 
-void launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
+bool launch_raster_tiles(hipStream_t st, uint32_t color_bits, uint32_t tile_rows, uint32_t tile_width, const MapPtrs& m,
 	const DrawBounds* bounds, const DrawRec* drec, const PartRec* parts, const SpanRec* spans, const ViewsArg& views,
 	const void* arena, const void* skybox, void* fb, uint32_t total_tiles, const uint32_t* counters)
 {
 	if(color_bits == 64)
-		launch_raster_ct<Color64T>(st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
-	else
-		launch_raster_ct<Color32T>(st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
+		return launch_raster_ct<Color64T>(
+			st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
+	return launch_raster_ct<Color32T>(
+		st, tile_rows, tile_width, m, bounds, drec, parts, spans, views, arena, skybox, fb, total_tiles, counters);
 }
 
 void launch_finish(hipStream_t st, const DrawRec* drec, uint32_t nd, uint32_t* counters, uint32_t* result)

@@ -125,7 +125,7 @@ struct sw_ctx
 		uint64_t arena_texels = 0;
 		void* arena = nullptr;
 		void* fb = nullptr;
-		uint32_t total_tiles = 0, tile_width = 64; // of the raster (raster_tile_width)
+		uint32_t total_tiles = 0, tile_rows = 8, tile_width = 64; // of the raster: a re-run keeps the views' tiling
 		uint32_t max_view_height = 0;
 		const void* portal = nullptr; // textures of SW_TEXSRC_PORTAL draws
 		uint64_t num_portal = 0;
@@ -660,10 +660,11 @@ int launch_stages(sw_ctx* ctx, const sw_ctx::Launch& L, bool surfaces, bool rast
 	{
 		{
 			StageTimer t(ctx, STAGE_RASTER);
-			swk::launch_raster_tiles(ctx->stream, L.color_bits, ctx->tile_rows, L.tile_width, mp,
-				static_cast<DrawBounds*>(ctx->dbounds.p),
-				static_cast<DrawRec*>(ctx->drec.p), static_cast<PartRec*>(ctx->parts.p), static_cast<SpanRec*>(ctx->spans.p),
-				ctx->views_arg, L.arena, L.color_bits == 64 ? map->sky64.p : map->sky32.p, L.fb, L.total_tiles, counters);
+			if(!swk::launch_raster_tiles(ctx->stream, L.color_bits, L.tile_rows, L.tile_width, mp,
+				   static_cast<DrawBounds*>(ctx->dbounds.p),
+				   static_cast<DrawRec*>(ctx->drec.p), static_cast<PartRec*>(ctx->parts.p), static_cast<SpanRec*>(ctx->spans.p),
+				   ctx->views_arg, L.arena, L.color_bits == 64 ? map->sky64.p : map->sky32.p, L.fb, L.total_tiles, counters))
+				return set_error(ctx, SW_ERR_DEVICE, "internal: no raster kernel for the views' tiles");
 		}
 		// With static span storage nothing in the live counters needs clearing after a sequence
 		// (errors also reach the host words), so the statistics wait until they are asked for; the
@@ -879,6 +880,7 @@ int launch_frame(sw_ctx* ctx, uint32_t num_draws, uint64_t num_vertex_ints, bool
 	std::vector<ViewExt> ve;
 	sw_ctx::Launch& L = ctx->last;
 	L = sw_ctx::Launch{};
+	L.tile_rows = ctx->tile_rows;
 	if((r = build_view_ext(ctx, &v, 1, ctx->frame_arena_texels, ve, L.total_tiles, L.tile_width, &L.max_view_height)))
 		return r;
 	L.surface_mode = SURF_SEARCH;
@@ -2225,6 +2227,7 @@ static int prepare_batch(sw_ctx* ctx, sw_map* map, const sw_batch* b, void* out_
 		((b->num_surfaces && !b->surfaces) || (b->num_draws && !b->draws) || (b->num_vertex_ints && !b->vertex_data)))
 		return set_error(ctx, SW_ERR_INVALID_ARGUMENT, "null surfaces, draws or vertex data");
 	int r;
+	L.tile_rows = ctx->tile_rows;
 	if((r = build_view_ext(ctx, b->views, b->num_views, b->surface_arena_texels, ve, L.total_tiles, L.tile_width, &L.max_view_height)))
 		return r;
 	if((r = validate_views_fit(ctx, ve, b->framebuffer_texels, b->num_surfaces, b->num_draws)))
