@@ -344,6 +344,10 @@ struct WavePoints
 	uint32_t address[N];
 	float value[N];
 };
+template <>
+struct WavePoints<0> // a step without points
+{
+};
 // neighbour n (left, right, up, down) of element a on the torus
 __host__ __device__ inline uint32_t water_neighbour(uint32_t a, uint32_t n, uint32_t log2w, uint32_t log2h)
 {

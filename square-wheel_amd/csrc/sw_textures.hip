@@ -497,7 +497,9 @@ __global__ __launch_bounds__(64) void k_water_points(float* field, float* field_
 // by the last of the blocks that read any point's element (they take tickets; nobody waits), when all of
 // them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 7 us
 // (2.9 us of copy, 4.3 us of points and 5.3 us of stencil as three operations); its 12.6 MB take 2.6 us at
-// the rate of a large copy. VEC: both buffers are 16-byte aligned.
+// the rate of a large copy. VEC: both buffers are 16-byte aligned. N = 0: a step without points, which then has
+// nothing of them in its arguments either (the runtime copies 516 bytes of them otherwise: four steps of a 256 x 256
+// field queued behind each other 17.7 us with them, 16.5 without).
 template <uint32_t N, bool VEC>
 __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, float* __restrict__ src, uint32_t log2w, uint32_t log2h,
 	float attenuation, swk::WavePoints<N> pts, uint32_t readers, uint32_t* __restrict__ ticket)
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 				o[k] = dst[i + k];
 			}
 	}
-	if(pts.n)
+	if constexpr(N > 0)
 	{
 		if(threadIdx.x == 0)
 			reads = 0;
@@ -593,31 +595,34 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 			for(uint32_t k = 0; k < 4; ++k)
 				dst[i + k] = r[k];
 	}
-	if(pts.n == 0 || !reads)
-		return; // uniform over the block
-	// Every element of the field that this block reads has been read: the sums made of them were stored
-	// before the barrier. Nothing else has to be ordered (the field is only read until the last reader
-	// writes it), so the ticket is relaxed: a fence here would write back the L2's dirty lines, most of
-	// the new field, once per reading block (the step took 10.7 us with fences).
-	__syncthreads();
-	if(threadIdx.x == 0)
-		last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
-	__syncthreads();
-	if(!last)
-		return;
-	// the last reader: an address's points lie together, its first point's thread adds them up in order
-	for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+	if constexpr(N > 0)
 	{
-		const uint32_t a = pts.address[k];
-		if(k > 0 && pts.address[k - 1u] == a)
-			continue;
-		float f = src[a];
-		for(uint32_t j = k; j < pts.n && pts.address[j] == a; ++j)
-			f += pts.value[j];
-		src[a] = f;
+		if(!reads)
+			return; // uniform over the block
+		// Every element of the field that this block reads has been read: the sums made of them were stored
+		// before the barrier. Nothing else has to be ordered (the field is only read until the last reader
+		// writes it), so the ticket is relaxed: a fence here would write back the L2's dirty lines, most of
+		// the new field, once per reading block (the step took 10.7 us with fences).
+		__syncthreads();
+		if(threadIdx.x == 0)
+			last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
+		__syncthreads();
+		if(!last)
+			return;
+		// the last reader: an address's points lie together, its first point's thread adds them up in order
+		for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+		{
+			const uint32_t a = pts.address[k];
+			if(k > 0 && pts.address[k - 1u] == a)
+				continue;
+			float f = src[a];
+			for(uint32_t j = k; j < pts.n && pts.address[j] == a; ++j)
+				f += pts.value[j];
+			src[a] = f;
+		}
+		if(threadIdx.x == 0)
+			*ticket = 0;
 	}
-	if(threadIdx.x == 0)
-		*ticket = 0;
 }
 
 // PackedNormalRoughness::pack (textures.rs:33-39, fast_math.rs:64-78): x 127 per lane, cvtps2dq,
@@ -1048,44 +1053,51 @@ static void launch_water_step_n(hipStream_t st, float* field, float* field_old, 
 	const sw_wave_point* points, uint32_t num_points, uint32_t* ticket)
 {
 	WavePoints<N> p;
-	p.n = num_points;
-	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
-	// sorted by address, an address's points in their order: only their own order matters to it
-	uint64_t order[N];
-	for(uint32_t k = 0; k < num_points; ++k)
-		order[k] = (uint64_t((points[k].x & mx) + ((points[k].y & my) << log2w)) << 32) | k;
-	std::sort(order, order + num_points);
-	// the blocks that read a point's element: those of its four neighbours
-	std::bitset<WATER_MAX_BLOCKS> readers;
-	for(uint32_t k = 0; k < num_points; ++k)
+	uint32_t num_readers = 0;
+	if constexpr(N > 0)
 	{
-		p.address[k] = uint32_t(order[k] >> 32);
-		p.value[k] = points[uint32_t(order[k])].value;
-		for(uint32_t n = 0; n < 4; ++n)
-			readers.set(water_neighbour(p.address[k], n, log2w, log2h) / WATER_BLOCK);
+		p.n = num_points;
+		const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+		// sorted by address, an address's points in their order: only their own order matters to it
+		uint64_t order[N];
+		for(uint32_t k = 0; k < num_points; ++k)
+			order[k] = (uint64_t((points[k].x & mx) + ((points[k].y & my) << log2w)) << 32) | k;
+		std::sort(order, order + num_points);
+		// the blocks that read a point's element: those of its four neighbours
+		std::bitset<WATER_MAX_BLOCKS> readers;
+		for(uint32_t k = 0; k < num_points; ++k)
+		{
+			p.address[k] = uint32_t(order[k] >> 32);
+			p.value[k] = points[uint32_t(order[k])].value;
+			for(uint32_t n = 0; n < 4; ++n)
+				readers.set(water_neighbour(p.address[k], n, log2w, log2h) / WATER_BLOCK);
+		}
+		num_readers = uint32_t(readers.count());
 	}
 	const uint32_t blocks = ((1u << (log2w + log2h)) + WATER_BLOCK - 1u) / WATER_BLOCK;
 	const bool vec = (reinterpret_cast<uintptr_t>(field) | reinterpret_cast<uintptr_t>(field_old)) % 16 == 0;
 	if(vec)
 		hipLaunchKernelGGL((k_water_step<N, true>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
-			uint32_t(readers.count()), ticket);
+			num_readers, ticket);
 	else
 		hipLaunchKernelGGL((k_water_step<N, false>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
-			uint32_t(readers.count()), ticket);
+			num_readers, ticket);
 }
 
 void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
 	const sw_wave_point* points, uint32_t num_points, const sw_wave_point* points_dev, uint32_t* ticket)
 {
-	// the smaller argument block where it holds the points: the runtime copies the whole block per launch
-	if(num_points <= WATER_ARG_POINTS_SMALL)
+	// the smallest argument block that holds the points: the runtime copies the whole block per launch
+	if(num_points == 0)
+		launch_water_step_n<0>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
+	else if(num_points <= WATER_ARG_POINTS_SMALL)
 		launch_water_step_n<WATER_ARG_POINTS_SMALL>(st, field, field_old, log2w, log2h, attenuation, points, num_points, ticket);
 	else if(num_points <= WATER_ARG_POINTS)
 		launch_water_step_n<WATER_ARG_POINTS>(st, field, field_old, log2w, log2h, attenuation, points, num_points, ticket);
 	else
 	{
 		hipLaunchKernelGGL(k_water_points, dim3(1), dim3(64), 0, st, field, field_old, points_dev, num_points, log2w, log2h);
-		launch_water_step_n<WATER_ARG_POINTS_SMALL>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
+		launch_water_step_n<0>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
 	}
 }
 

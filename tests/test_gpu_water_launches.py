@@ -46,6 +46,35 @@ def test_water_step_points(gpu_ctx, log2, points):
     assert np.array_equal(b.view(np.uint32), fo.view(np.uint32))
 
 
+@pytest.mark.parametrize("log2", [(4, 4), (5, 5), (10, 4), (4, 11), (9, 9), (10, 11)])
+@pytest.mark.parametrize("shift", [(0, 0), (1, 2)])
+def test_water_step_without_points(gpu_ctx, log2, shift):
+    """The kernel without points, between steps with one (whose ticket it leaves alone), on fields of less than a
+    block to the largest, 16-byte aligned and not."""
+    lw, lh = log2
+    n = 1 << (lw + lh)
+    rng = np.random.default_rng([lw, lh])
+    f, fo = rng.normal(size=n).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    steps = [_points(rng, lw, lh, k) for k in (0, 0, 1, 0, 257, 1)]
+    att = np.float32(0.97)
+    print(f"water steps without points {lw}x{lh} shift={shift}", flush=True)
+    bufs = [gpu_ctx.to_device(np.concatenate([np.full(s, 9, np.float32), v, np.full(4, 9, np.float32)])) for s, v in zip(shift, (f, fo))]
+    ptr = [C.c_void_p(b.ptr.value + 4 * s) for s, b in zip(shift, bufs)]
+    try:
+        for k, p in enumerate(steps):
+            gpu_ctx.check(gpu_ctx.lib.sw_water_step(gpu_ctx.h, ptr[k % 2], ptr[1 - k % 2], lw, lh, C.c_float(att),
+                                                    C.c_void_p(p.ctypes.data) if len(p) else None, len(p)), "sw_water_step")
+        got = [b.read(np.float32, n + s + 4) for s, b in zip(shift, bufs)]
+    finally:
+        for b in bufs:
+            b.free()
+    for p in steps:
+        f, fo = oracle.water_step(f, fo, lw, lh, att, p)
+    for g, s, ref in zip(got, shift, (f, fo)):
+        assert np.array_equal(g[s:s + n].view(np.uint32), ref.view(np.uint32))
+        assert np.all(g[:s] == 9) and np.all(g[s + n:] == 9)
+
+
 @pytest.mark.parametrize("shift", [(1, 0), (0, 3), (2, 2)])
 def test_water_unaligned_fields(gpu_ctx, shift):
     lw, lh = 6, 6
