@@ -506,8 +506,12 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 {
 	__shared__ uint64_t near_mask[N / 64 + 1]; // points whose element, or a neighbour of it, lies in this block
 	__shared__ uint32_t reads, last;
+	// Blocks are dealt to the eight XCDs in turn: each takes a contiguous eighth of the field, so that a row's
+	// neighbours above and below come from the same L2 (four queued steps of 1024 x 1024 without points: 23.8 us
+	// with consecutive blocks on different XCDs, 16.9 so).
+	const uint32_t block = gridDim.x % 8u ? blockIdx.x : blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u;
 	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
-	const uint32_t i = blockIdx.x * swk::WATER_BLOCK + threadIdx.x * 4u;
+	const uint32_t i = block * swk::WATER_BLOCK + threadIdx.x * 4u;
 	const bool in = (i >> (log2w + log2h)) == 0;
 	const uint32_t x = i & mx, y = i >> log2w;
 	const uint32_t row = y << log2w, up = (((y - 1u) & my) << log2w) + x, down = (((y + 1u) & my) << log2w) + x;
@@ -549,8 +553,8 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 			{
 				const uint32_t a = pts.address[k];
 				for(uint32_t n = 0; n < 4; ++n)
-					read = read || swk::water_neighbour(a, n, log2w, log2h) / swk::WATER_BLOCK == blockIdx.x;
-				near = read || a / swk::WATER_BLOCK == blockIdx.x;
+					read = read || swk::water_neighbour(a, n, log2w, log2h) / swk::WATER_BLOCK == block;
+				near = read || a / swk::WATER_BLOCK == block;
 			}
 			const uint64_t m = __ballot(near), r = __ballot(read);
 			if((threadIdx.x & 63u) == 0)
