@@ -491,9 +491,11 @@ __global__ __launch_bounds__(64) void k_water_points(float* field, float* field_
 
 // update_wave_field (:307-418), with the step's points (add_point_value, :68-76) where they travel in the
 // kernel's arguments: the field is a torus (rows and columns wrap); a block takes WATER_BLOCK consecutive
-// elements, four per thread. The stencil reads the field with the points added: the threads whose
-// neighbours hold points add them to the values they loaded, in the points' order (an address's additions
-// in the reference's order), and the owners subtract them from the old field. The field itself is updated
+// elements, four per thread. The stencil reads the field with the points added: a block that points touch
+// passes its values through LDS, where a thread per address adds that address's points in their order (the
+// reference's) wherever the value is held and subtracts them from the old field (every thread comparing each
+// point's address with those of the 18 values it held took 0.2 us a point: two queued steps of 32 x 32 with 200
+// points 82.8 us, 67 with the points in a kernel ahead of the step, now 12.9). The field itself is updated
 // by the last of the blocks that read any point's element (they take tickets; nobody waits), when all of
 // them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 7 us
 // (2.9 us of copy, 4.3 us of points and 5.3 us of stencil as three operations); its 12.6 MB take 2.6 us at
@@ -504,8 +506,11 @@ template <uint32_t N, bool VEC>
 __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, float* __restrict__ src, uint32_t log2w, uint32_t log2h,
 	float attenuation, swk::WavePoints<N> pts, uint32_t readers, uint32_t* __restrict__ ticket)
 {
-	__shared__ uint64_t near_mask[N / 64 + 1]; // points whose element, or a neighbour of it, lies in this block
-	__shared__ uint32_t reads, last;
+	// points only: the block's values by element (its own, their neighbours above and below, the old field, the
+	// neighbours left and right of its ends), and whether points touch them
+	__shared__ __align__(16) float l_own[N ? swk::WATER_BLOCK : 1], l_up[N ? swk::WATER_BLOCK : 1], l_down[N ? swk::WATER_BLOCK : 1],
+		l_old[N ? swk::WATER_BLOCK : 1], l_ends[2], l_value[N ? N : 1];
+	__shared__ uint32_t l_address[N ? N : 1], touched, reads, last;
 	// Blocks are dealt to the eight XCDs in turn: each takes a contiguous eighth of the field, so that a row's
 	// neighbours above and below come from the same L2 (four queued steps of 1024 x 1024 without points: 23.8 us
 	// with consecutive blocks on different XCDs, 16.9 so).
@@ -543,45 +548,86 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 	if constexpr(N > 0)
 	{
 		if(threadIdx.x == 0)
-			reads = 0;
+			touched = reads = 0;
 		__syncthreads();
-		for(uint32_t base = threadIdx.x & ~63u; base < pts.n; base += 256u)
+		// thread k's point: its address, whether it is the first of its address, and the elements that it is read by
+		static_assert(N <= 256u);
+		const uint32_t k = threadIdx.x, b0 = block * swk::WATER_BLOCK;
+		const bool has = k < pts.n;
+		const uint32_t a = pts.address[has ? k : 0u], before = pts.address[has && k > 0u ? k - 1u : 0u];
+		const float v0 = pts.value[has ? k : 0u];
+		const bool first = has && (k == 0u || before != a);
+		if(has)
 		{
-			const uint32_t k = base + (threadIdx.x & 63u);
-			bool near = false, read = false;
-			if(k < pts.n)
-			{
-				const uint32_t a = pts.address[k];
-				for(uint32_t n = 0; n < 4; ++n)
-					read = read || swk::water_neighbour(a, n, log2w, log2h) / swk::WATER_BLOCK == block;
-				near = read || a / swk::WATER_BLOCK == block;
-			}
-			const uint64_t m = __ballot(near), r = __ballot(read);
-			if((threadIdx.x & 63u) == 0)
-			{
-				near_mask[base / 64u] = m;
-				if(r)
-					reads = 1; // every writer writes 1
-			}
+			l_address[k] = a;
+			l_value[k] = v0;
 		}
-		__syncthreads();
-		for(uint32_t q = 0; q * 64u < pts.n; ++q)
-			for(uint64_t m = near_mask[q]; m; m &= m - 1u)
-			{
-				const uint32_t k = q * 64u + uint32_t(__builtin_ctzll(m)), a = pts.address[k];
-				const float v = pts.value[k];
-				// c[1 .. 4] are the thread's own elements: neighbours of each other
-				c[0] = a == il ? c[0] + v : c[0];
-				c[5] = a == ir ? c[5] + v : c[5];
+		uint32_t at[4]; // of the block: its right, left, lower and upper neighbour, whose left, ... neighbour it is
+		bool read = false;
 #pragma unroll
-				for(uint32_t e = 0; e < 4; ++e)
+		for(uint32_t n = 0; n < 4; ++n)
+		{
+			at[n] = swk::water_neighbour(a, n ^ 1u, log2w, log2h) - b0;
+			read = read || at[n] < swk::WATER_BLOCK;
+		}
+		const uint32_t own = a - b0;
+		if(has && read)
+			reads = 1; // every writer writes 1
+		if(has && (read || own < swk::WATER_BLOCK))
+			touched = 1;
+		__syncthreads();
+		if(touched)
+		{
+			// uniform over the block: the values go through LDS, where a thread per address adds its points in turn
+			const uint32_t t4 = threadIdx.x * 4u;
+			*reinterpret_cast<float4*>(l_own + t4) = make_float4(c[1], c[2], c[3], c[4]);
+			*reinterpret_cast<float4*>(l_up + t4) = make_float4(u[0], u[1], u[2], u[3]);
+			*reinterpret_cast<float4*>(l_down + t4) = make_float4(d[0], d[1], d[2], d[3]);
+			*reinterpret_cast<float4*>(l_old + t4) = make_float4(o[0], o[1], o[2], o[3]);
+			// the neighbour left of an element of the block is its predecessor, or lies at its row's other end: in the
+			// block if it holds whole rows, else only the first thread's is outside (right alike)
+			const bool left_in = il - b0 < swk::WATER_BLOCK, right_in = ir - b0 < swk::WATER_BLOCK;
+			if(!left_in)
+				l_ends[0] = c[0];
+			if(!right_in)
+				l_ends[1] = c[5];
+			__syncthreads();
+			if(first && (read || own < swk::WATER_BLOCK))
+			{
+				// whatever place holds the element's value, all of them hold the same
+				const bool is_own = own < swk::WATER_BLOCK, is_left = !is_own && at[0] < swk::WATER_BLOCK,
+						   is_right = !is_own && at[1] < swk::WATER_BLOCK, is_up = at[2] < swk::WATER_BLOCK, is_down = at[3] < swk::WATER_BLOCK;
+				float f = is_own ? l_own[own] : is_left ? l_ends[0] : is_right ? l_ends[1] : is_up ? l_up[at[2]] : l_down[at[3]];
+				float old = is_own ? l_old[own] : 0.0f;
+				for(uint32_t j = k; j < pts.n && l_address[j] == a; ++j)
 				{
-					c[e + 1] = a == i + e ? c[e + 1] + v : c[e + 1];
-					o[e] = a == i + e ? o[e] - v : o[e];
-					u[e] = a == up + e ? u[e] + v : u[e];
-					d[e] = a == down + e ? d[e] + v : d[e];
+					f += l_value[j];
+					old -= l_value[j];
 				}
+				if(is_own)
+				{
+					l_own[own] = f;
+					l_old[own] = old;
+				}
+				if(is_left)
+					l_ends[0] = f;
+				if(is_right)
+					l_ends[1] = f;
+				if(is_up)
+					l_up[at[2]] = f;
+				if(is_down)
+					l_down[at[3]] = f;
 			}
+			__syncthreads();
+			const float4 c4 = *reinterpret_cast<const float4*>(l_own + t4), u4 = *reinterpret_cast<const float4*>(l_up + t4),
+						 d4 = *reinterpret_cast<const float4*>(l_down + t4), o4 = *reinterpret_cast<const float4*>(l_old + t4);
+			c[0] = left_in ? l_own[il - b0] : l_ends[0];
+			c[1] = c4.x, c[2] = c4.y, c[3] = c4.z, c[4] = c4.w;
+			c[5] = right_in ? l_own[ir - b0] : l_ends[1];
+			u[0] = u4.x, u[1] = u4.y, u[2] = u4.z, u[3] = u4.w;
+			d[0] = d4.x, d[1] = d4.y, d[2] = d4.z, d[3] = d4.w;
+			o[0] = o4.x, o[1] = o4.y, o[2] = o4.z, o[3] = o4.w;
+		}
 	}
 	if(in)
 	{
@@ -614,14 +660,13 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 		if(!last)
 			return;
 		// the last reader: an address's points lie together, its first point's thread adds them up in order
-		for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+		const uint32_t k = threadIdx.x;
+		if(k < pts.n && (k == 0u || l_address[k - 1u] != l_address[k]))
 		{
-			const uint32_t a = pts.address[k];
-			if(k > 0 && pts.address[k - 1u] == a)
-				continue;
+			const uint32_t a = l_address[k];
 			float f = src[a];
-			for(uint32_t j = k; j < pts.n && pts.address[j] == a; ++j)
-				f += pts.value[j];
+			for(uint32_t j = k; j < pts.n && l_address[j] == a; ++j)
+				f += l_value[j];
 			src[a] = f;
 		}
 		if(threadIdx.x == 0)

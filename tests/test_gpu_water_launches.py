@@ -46,6 +46,29 @@ def test_water_step_points(gpu_ctx, log2, points):
     assert np.array_equal(b.view(np.uint32), fo.view(np.uint32))
 
 
+@pytest.mark.parametrize("log2", [(4, 4), (5, 4), (9, 5), (10, 5), (11, 4), (12, 6)])
+@pytest.mark.parametrize("points", [9, 64, 250])
+def test_water_step_crowded_points(gpu_ctx, log2, points):
+    """Points side by side in one corner, over the torus's seams, and many of them at one address: rows shorter than a
+    block, exactly one, and several blocks long (a row's ends then lie in other blocks)."""
+    lw, lh = log2
+    n, w, h = 1 << (lw + lh), 1 << lw, 1 << lh
+    rng = np.random.default_rng([lw, lh, points])
+    f, fo = rng.normal(size=n).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    p = np.zeros(points, A.WAVE_POINT_DTYPE)
+    p["x"], p["y"] = (w + rng.integers(-4, 4, points)) % w, (h + rng.integers(-3, 3, points)) % h
+    p["x"][1::4] = (1024 + rng.integers(-2, 2, len(p[1::4]))) % w  # both sides of a block's end inside a row
+    p["x"][2::4], p["y"][2::4] = 0, 0
+    p["value"] = rng.normal(size=points) * np.exp2(rng.integers(-20, 20, points))
+    att = np.float32(0.99)
+    print(f"water crowded points {lw}x{lh} points={points}", flush=True)
+    a, b = gpu_ctx.water_steps(f, fo, lw, lh, att, [p, p[::-1].copy()])
+    for q in (p, p[::-1].copy()):
+        f, fo = oracle.water_step(f, fo, lw, lh, att, q)
+    assert np.array_equal(a.view(np.uint32), f.view(np.uint32))
+    assert np.array_equal(b.view(np.uint32), fo.view(np.uint32))
+
+
 @pytest.mark.parametrize("log2", [(4, 4), (5, 5), (10, 4), (4, 11), (9, 9), (10, 11)])
 @pytest.mark.parametrize("shift", [(0, 0), (1, 2)])
 def test_water_step_without_points(gpu_ctx, log2, shift):
