@@ -31,7 +31,7 @@ namespace
 SW_DEV int32_t imax32(int32_t a, int32_t b) { return a > b ? a : b; }
 SW_DEV int32_t imin32(int32_t a, int32_t b) { return a < b ? a : b; }
 
-struct DepthRow
+struct alignas(8) DepthRow
 {
 	uint16_t x0, x1; // [x0, x1): the span's pixels (empty when x0 >= x1)
 	float inv_z; // 1 / z at x0
@@ -57,7 +57,7 @@ struct DepthTargetDev
 };
 
 // What the raster reads of a draw, beside its row records.
-struct DepthDrawInfo
+struct alignas(16) DepthDrawInfo
 {
 	int32_t first, end; // rows [first, end) have records
 	float dx;
@@ -242,13 +242,42 @@ SW_DEV uint32_t span_bits(int32_t x0, int32_t x1, int32_t base)
 }
 
 #define DEPTH_SEGMENTS 4u // 64-pixel segments a wave holds at once
+#define DEPTH_PASS (64u * DEPTH_SEGMENTS) // columns of a pass
+#define DEPTH_GROUP (64u * DEPTH_PASS) // columns of 64 passes
+#define DEPTH_NARROW (4u * DEPTH_PASS) // wider rows look at all their draws' spans first
+#define DEPTH_FOUND 128u // and keep that many in LDS
+
+// A draw's span of a row, packed x0 | x1 << 16 (0: none).
+struct alignas(16) RowSpan
+{
+	uint32_t span;
+	float inv_z; // 1 / z at x0
+	float dx;
+	uint32_t depth_test;
+};
+
+// the passes, a bit each, of the group of columns from base on that [x0, x1) meets
+SW_DEV uint64_t pass_bits(uint32_t x0, uint32_t x1, uint32_t base)
+{
+	if(x0 >= x1 || x1 <= base || x0 >= base + DEPTH_GROUP)
+		return 0ull;
+	const uint32_t a = x0 > base ? (x0 - base) / DEPTH_PASS : 0u;
+	return low_bits(int32_t((x1 - base + DEPTH_PASS - 1u) / DEPTH_PASS)) & ~low_bits(int32_t(a));
+}
 
 // The rows of a 256 x 256 cube side take one pass of 256 columns each. A back-to-front list overwrites
 // most pixels several times: walked backwards, a row is finished after its nearest spans, and each pixel's
 // chain is evaluated once instead of once per draw that covers it. Eight lights' 256 x 256 cube maps (3.1
-// Mtexels, 1,633 draws): 33.6 us with every span filled in draw order by 16-lane chains.
+// Mtexels, 1,633 draws): 33.6 us with every span filled in draw order by 16-lane chains, now 19.
+// WIDE (a target wider than DEPTH_NARROW): a row's draws are looked at once, which gives the passes that a span meets
+// and a list of the spans for them. Without it every pass loads every draw's record, also where none has a span:
+// 300 polygons of up to 32 x 32 pixels in a 4096 x 4096 target 76.0 us a call, 38.1 so (54.9 with every span filled in
+// draw order), in 16384 x 512 156.9, 49.7 (57.9). Rows of up to four passes go without (twelve targets of 640 x 640
+// with 40 such polygons 38.9 us a call, 40.1 with the list).
+template <bool WIDE>
 __global__ __launch_bounds__(256) void k_depth_raster(DepthLaunch L)
 {
+	__shared__ RowSpan found[WIDE ? 4 : 1][WIDE ? DEPTH_FOUND : 1]; // a wave's: the spans of a wide row
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
 	if(wave >= L.num_rows)
@@ -266,128 +295,157 @@ __global__ __launch_bounds__(256) void k_depth_raster(DepthLaunch L)
 	}
 	const DepthTargetDev t = L.targets[ti];
 	const int32_t y = int32_t(wave - t.first_row);
-	const uint32_t draws_end = t.first_draw + t.num_draws;
 	const DepthRow* rows = L.rows + t.rec_base + uint64_t(uint32_t(y)) * t.num_draws;
 	float* out = L.texels + t.offset + uint64_t(uint32_t(y)) * t.w;
-	// lane's draw di: its span of this row, packed x0 | x1 << 16 (0: none), 1 / z at x0
-	auto load_span = [&](bool ok, uint32_t di, DepthDrawInfo& info, float& inv_z) -> uint32_t {
-		inv_z = 0.0f;
-		info = DepthDrawInfo{0, 0, 0.0f, 0};
+	// the row's spans in draw order: those of all draws, or (listed) the ones found
+	uint32_t n = t.num_draws;
+	bool listed = false;
+	auto load_span = [&](bool ok, uint32_t i) -> RowSpan {
 		if(!ok)
-			return 0u;
-		const DepthRow r = rows[di - t.first_draw]; // not written outside the draw's rows: dropped below
-		info = L.infos[di];
-		inv_z = r.inv_z;
-		return y >= info.first && y < info.end && r.x0 < r.x1 ? uint32_t(r.x0) | (uint32_t(r.x1) << 16) : 0u;
+			return RowSpan{0u, 0.0f, 0.0f, 0u};
+		if(WIDE && listed)
+			return found[threadIdx.x >> 6][i];
+		// both records whole, and no condition between them: a second trip to memory otherwise
+		const uint2 r = *reinterpret_cast<const uint2*>(rows + i); // not written outside the draw's rows: dropped here
+		const uint4 info = *reinterpret_cast<const uint4*>(L.infos + t.first_draw + i);
+		const bool has = (y >= int32_t(info.x)) & (y < int32_t(info.y)) & ((r.x & 0xFFFFu) < r.x >> 16);
+		return RowSpan{has ? r.x : 0u, __builtin_bit_cast(float, r.y), __builtin_bit_cast(float, info.z), info.w};
 	};
-	for(uint32_t cx = 0; cx < t.w; cx += 64u * DEPTH_SEGMENTS)
+	const uint32_t margin = t.flags & SW_DEPTH_CIRCLE ? circle_margin(int32_t(t.w), y) : 0u;
+	for(uint32_t base_x = 0; base_x < t.w; base_x += DEPTH_GROUP)
 	{
-		uint64_t open[DEPTH_SEGMENTS]; // pixels no overwriting draw has taken yet
-		float z[DEPTH_SEGMENTS];
-		uint32_t from[DEPTH_SEGMENTS]; // the draw that took the pixel, + 1
-		uint64_t any_open = 0;
-		bool tests = false;
+		uint64_t passes = pass_bits(0u, t.w, base_x);
+		if(WIDE && t.w > DEPTH_NARROW)
+		{
+			// only the passes that a span, or what lies outside the circle, meets; the spans are listed for them
+			uint64_t met = pass_bits(0u, margin, base_x) | pass_bits(t.w - margin, t.w, base_x);
+			uint32_t count = 0;
+			for(uint32_t base = 0; base < n; base += 64u)
+			{
+				const RowSpan r = load_span(base + lane < n, base + lane);
+				met |= pass_bits(r.span & 0xFFFFu, r.span >> 16, base_x);
+				const uint64_t has = __ballot(r.span != 0u);
+				const uint32_t at = count + uint32_t(__popcll(has & ((1ull << lane) - 1ull)));
+				if(!listed && r.span != 0u && at < DEPTH_FOUND)
+					found[threadIdx.x >> 6][at] = r;
+				count += uint32_t(__popcll(has));
+			}
+			if(count <= DEPTH_FOUND)
+			{
+				__builtin_amdgcn_wave_barrier(); // the wave's own LDS operations take effect in order
+				listed = true;
+				n = count;
+			}
 #pragma unroll
-		for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
-		{
-			open[s] = low_bits(int32_t(t.w) - int32_t(cx + 64u * s));
-			any_open |= open[s];
-			z[s] = 0.0f;
-			from[s] = 0;
+			for(int off = 32; off > 0; off >>= 1)
+				met |= __shfl_xor(met, off);
+			passes &= uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int32_t(met)))) |
+				(uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int32_t(met >> 32)))) << 32);
 		}
-		// backwards, 64 draws at a time: lane k holds draw chunk_end - 1 - k
-		for(uint32_t chunk_end = draws_end; chunk_end > t.first_draw && any_open; chunk_end = chunk_end - t.first_draw > 64u ? chunk_end - 64u : t.first_draw)
+		for(; passes; passes &= passes - 1u)
 		{
-			const uint32_t left = chunk_end - t.first_draw;
-			DepthDrawInfo info;
-			float inv_z;
-			const uint32_t span = load_span(lane < left, chunk_end - 1u - lane, info, inv_z);
-			const bool meets = (span >> 16) > cx && (span & 0xFFFFu) < cx + 64u * DEPTH_SEGMENTS && span != 0u;
-			tests = tests || __ballot(meets && info.depth_test != 0u) != 0;
-			uint64_t hits = __ballot(meets && info.depth_test == 0u);
-			// every lane's span as bits of the segments, so that a hit costs two readlanes, three scalar
-			// operations and a select per segment
-			uint32_t src[DEPTH_SEGMENTS], bits[DEPTH_SEGMENTS][2];
+			const uint32_t cx = base_x + uint32_t(__builtin_ctzll(passes)) * DEPTH_PASS;
+			uint64_t open[DEPTH_SEGMENTS]; // pixels no overwriting draw has taken yet
+			float z[DEPTH_SEGMENTS];
+			uint32_t from[DEPTH_SEGMENTS]; // the place in draw order of the span that took the pixel, + 1
+			uint64_t any_open = 0;
+			bool tests = false;
 #pragma unroll
 			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 			{
-				src[s] = 64u;
-#pragma unroll
-				for(uint32_t h = 0; h < 2; ++h)
-					bits[s][h] = span_bits(int32_t(span & 0xFFFFu), int32_t(span >> 16), int32_t(cx + 64u * s + 32u * h));
+				open[s] = low_bits(int32_t(t.w) - int32_t(cx + 64u * s));
+				any_open |= open[s];
+				z[s] = 0.0f;
+				from[s] = 0;
 			}
-			while(hits && any_open)
+			// backwards, 64 spans at a time: lane k holds span end - 1 - k
+			for(uint32_t end = n; end > 0u && any_open; end = end > 64u ? end - 64u : 0u)
 			{
-				const uint32_t k = uint32_t(__builtin_ctzll(hits));
-				hits &= hits - 1u;
-				any_open = 0;
+				const RowSpan r = load_span(lane < end, end - 1u - lane);
+				const bool meets = (r.span >> 16) > cx && (r.span & 0xFFFFu) < cx + DEPTH_PASS && r.span != 0u;
+				tests = tests || __ballot(meets && r.depth_test != 0u) != 0;
+				uint64_t hits = __ballot(meets && r.depth_test == 0u);
+				// every lane's span as bits of the segments, so that a hit costs two readlanes, three scalar
+				// operations and a select per segment
+				uint32_t src[DEPTH_SEGMENTS], bits[DEPTH_SEGMENTS][2];
 #pragma unroll
 				for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 				{
-					const uint64_t take = open[s] & (uint64_t(uint32_t(rl(int32_t(bits[s][0]), k))) | (uint64_t(uint32_t(rl(int32_t(bits[s][1]), k))) << 32));
-					open[s] ^= take;
-					any_open |= open[s];
-					src[s] = __builtin_amdgcn_inverse_ballot_w64(take) ? k : src[s];
-				}
-			}
-			// the pixels taken in this chunk: their chain's end
+					src[s] = 64u;
 #pragma unroll
-			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
-			{
-				if(__ballot(src[s] < 64u) == 0)
-					continue;
-				const uint32_t k = src[s] & 63u;
-				const float start = lane_pull_f(inv_z, k), step = lane_pull_f(info.dx, k);
-				const uint32_t x0 = uint32_t(lane_pull(int32_t(span), k)) & 0xFFFFu;
-				if(src[s] < 64u)
+					for(uint32_t h = 0; h < 2; ++h)
+						bits[s][h] = span_bits(int32_t(r.span & 0xFFFFu), int32_t(r.span >> 16), int32_t(cx + 64u * s + 32u * h));
+				}
+				while(hits && any_open)
 				{
-					z[s] = swchain::chain_add(start, step, cx + 64u * s + lane - x0);
-					from[s] = chunk_end - k;
+					const uint32_t k = uint32_t(__builtin_ctzll(hits));
+					hits &= hits - 1u;
+					any_open = 0;
+#pragma unroll
+					for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+					{
+						const uint64_t take = open[s] & (uint64_t(uint32_t(rl(int32_t(bits[s][0]), k))) | (uint64_t(uint32_t(rl(int32_t(bits[s][1]), k))) << 32));
+						open[s] ^= take;
+						any_open |= open[s];
+						src[s] = __builtin_amdgcn_inverse_ballot_w64(take) ? k : src[s];
+					}
+				}
+				// the pixels taken in this chunk: their chain's end
+#pragma unroll
+				for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+				{
+					if(__ballot(src[s] < 64u) == 0)
+						continue;
+					const uint32_t k = src[s] & 63u;
+					const float start = lane_pull_f(r.inv_z, k), step = lane_pull_f(r.dx, k);
+					const uint32_t x0 = uint32_t(lane_pull(int32_t(r.span), k)) & 0xFFFFu;
+					if(src[s] < 64u)
+					{
+						z[s] = swchain::chain_add(start, step, cx + 64u * s + lane - x0);
+						from[s] = end - k;
+					}
 				}
 			}
-		}
-		if(tests)
-		{
-			// depth-tested draws over the pixels' overwriting draw (or the buffer's value), in order
+			if(tests)
+			{
+				// depth-tested draws over the pixels' overwriting draw (or the buffer's value), in order
+#pragma unroll
+				for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+				{
+					const uint32_t x = cx + 64u * s + lane;
+					if(from[s] == 0 && x < t.w)
+						z[s] = out[x];
+				}
+				for(uint32_t base = 0; base < n; base += 64u)
+				{
+					const RowSpan r = load_span(base + lane < n, base + lane);
+					uint64_t hits = __ballot((r.span >> 16) > cx && (r.span & 0xFFFFu) < cx + DEPTH_PASS && r.span != 0u && r.depth_test != 0u);
+					while(hits)
+					{
+						const uint32_t k = uint32_t(__builtin_ctzll(hits));
+						hits &= hits - 1u;
+						const uint32_t sp = uint32_t(rl(int32_t(r.span), k)), x0 = sp & 0xFFFFu, x1 = sp >> 16;
+						const float start = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, r.inv_z), k));
+						const float step = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, r.dx), k));
+#pragma unroll
+						for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
+						{
+							const uint32_t x = cx + 64u * s + lane;
+							if(x >= x0 && x < x1 && base + k + 1u > from[s])
+								z[s] = fmax_r(swchain::chain_add(start, step, x - x0), z[s]);
+						}
+					}
+				}
+			}
 #pragma unroll
 			for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
 			{
 				const uint32_t x = cx + 64u * s + lane;
-				if(from[s] == 0 && x < t.w)
-					z[s] = out[x];
+				const bool outside = (t.flags & SW_DEPTH_CIRCLE) && (x < margin || x >= t.w - margin);
+				// with depth tests every pixel is stored (one that no draw touched as it was)
+				if(x < t.w && (outside || tests || !__builtin_amdgcn_inverse_ballot_w64(open[s])))
+					out[x] = outside ? 1.0e24f : z[s];
 			}
-			for(uint32_t base = t.first_draw; base < draws_end; base += 64u)
-			{
-				DepthDrawInfo info;
-				float inv_z;
-				const uint32_t span = load_span(base + lane < draws_end, base + lane, info, inv_z);
-				uint64_t hits = __ballot((span >> 16) > cx && (span & 0xFFFFu) < cx + 64u * DEPTH_SEGMENTS && span != 0u && info.depth_test != 0u);
-				while(hits)
-				{
-					const uint32_t k = uint32_t(__builtin_ctzll(hits));
-					hits &= hits - 1u;
-					const uint32_t sp = uint32_t(rl(int32_t(span), k)), x0 = sp & 0xFFFFu, x1 = sp >> 16;
-					const float start = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, inv_z), k));
-					const float step = __builtin_bit_cast(float, rl(__builtin_bit_cast(int, info.dx), k));
-#pragma unroll
-					for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
-					{
-						const uint32_t x = cx + 64u * s + lane;
-						if(x >= x0 && x < x1 && base + k + 1u > from[s])
-							z[s] = fmax_r(swchain::chain_add(start, step, x - x0), z[s]);
-					}
-				}
-			}
-		}
-		const uint32_t margin = t.flags & SW_DEPTH_CIRCLE ? circle_margin(int32_t(t.w), y) : 0u;
-#pragma unroll
-		for(uint32_t s = 0; s < DEPTH_SEGMENTS; ++s)
-		{
-			const uint32_t x = cx + 64u * s + lane;
-			const bool outside = (t.flags & SW_DEPTH_CIRCLE) && (x < margin || x >= t.w - margin);
-			// with depth tests every pixel is stored (one that no draw touched as it was)
-			if(x < t.w && (outside || tests || !__builtin_amdgcn_inverse_ballot_w64(open[s])))
-				out[x] = outside ? 1.0e24f : z[s];
 		}
 	}
 }
@@ -402,7 +460,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 	std::vector<DepthTargetDev> tg(num_targets);
 	std::vector<DepthDrawDev> dd(num_draws);
 	uint64_t rec = 0;
-	uint32_t rows = 0, next_draw = 0;
+	uint32_t rows = 0, next_draw = 0, max_width = 0;
 	for(uint32_t i = 0; i < num_targets; ++i)
 	{
 		const sw_depth_target& t = targets[i];
@@ -422,6 +480,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 			return (error = "depth targets: too many rows"), -1;
 		tg[i] = DepthTargetDev{t.offset, rec, t.width, t.height, t.first_draw, t.num_draws, rows, t.flags};
 		rows += t.height;
+		max_width = max_width > t.width ? max_width : t.width;
 		rec += uint64_t(t.height) * t.num_draws;
 		for(uint32_t k = t.first_draw; k < t.first_draw + t.num_draws; ++k)
 		{
@@ -439,6 +498,7 @@ int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_de
 	plan.bytes = plan.targets_at + sizeof(DepthTargetDev) * tg.size();
 	plan.row_records = rec;
 	plan.rows = rows;
+	plan.max_width = max_width;
 	plan.num_draws = num_draws;
 	plan.num_targets = num_targets;
 	packed.assign(plan.bytes, 0);
@@ -466,7 +526,9 @@ void launch_depth(hipStream_t st, const char* args, const int32_t* vdata, const 
 	const uint32_t copy_blocks = (plan.num_targets * uint32_t(sizeof(DepthTargetDev) / 4u) + 255u) / 256u;
 	if(!raster)
 		hipLaunchKernelGGL(k_depth_setup, dim3(draw_blocks + copy_blocks), dim3(256), 0, st, L, draw_blocks);
+	else if(plan.max_width > DEPTH_NARROW)
+		hipLaunchKernelGGL(k_depth_raster<true>, dim3((plan.rows + 3u) / 4u), dim3(256), 0, st, L);
 	else
-		hipLaunchKernelGGL(k_depth_raster, dim3((plan.rows + 3u) / 4u), dim3(256), 0, st, L);
+		hipLaunchKernelGGL(k_depth_raster<false>, dim3((plan.rows + 3u) / 4u), dim3(256), 0, st, L);
 }
 } // namespace swk

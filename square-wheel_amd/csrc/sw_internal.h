@@ -321,7 +321,7 @@ struct DepthPlan
 {
 	size_t bytes = 0, targets_at = 0;
 	uint64_t row_records = 0;
-	uint32_t rows = 0, num_draws = 0, num_targets = 0;
+	uint32_t rows = 0, max_width = 0, num_draws = 0, num_targets = 0;
 };
 int depth_plan(const sw_depth_target* targets, uint32_t num_targets, const sw_depth_draw* draws, uint32_t num_draws,
 	uint64_t num_vertex_ints, uint64_t num_texels, std::vector<char>& packed, DepthPlan& plan, std::string& error);
