@@ -33,6 +33,16 @@ SW_HD float bits_float(uint32_t u)
 	return x;
 }
 
+// 0, infinite or NaN: one instruction of the device's (a mask of classes), which the kernels' inner loop notices.
+SW_HD bool zero_or_not_finite(float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+	return __builtin_amdgcn_classf(x, 0x267);
+#else
+	return (float_bits(x) << 1) - 1u >= 0xFEFFFFFFu;
+#endif
+}
+
 // a and b, with their signs, strictly between the same two neighbouring powers of two (or both denormal);
 // then so is every value of a monotonic chain from a to b.
 SW_HD bool inside_one_binade(float a, float b)
@@ -53,8 +63,9 @@ SW_HD float chain_add(float v, float d, uint32_t n)
 		const float end = __builtin_fmaf(float(n - 2u), step, v2);
 		if(inside_one_binade(v1, end))
 			return end;
-		if(step == 0.0f)
-			return v2; // v2 + d rounds to v2 again and again
+		// a step of 0 (v2 + d rounds to v2 again and again), or an infinite one or NaN (so is v3, and stays so)
+		if(zero_or_not_finite(step))
+			return v3;
 		v = v3;
 		n -= 3u;
 		if(inside_one_binade(v1, v3))

@@ -41,4 +41,11 @@ uint64_t check_chain_ends(const float* start, const float* step, uint32_t count,
 	}
 	return bad;
 }
+
+// The chains' ends alone.
+void chain_ends(const float* start, const float* step, uint32_t count, uint32_t n, float* out)
+{
+	for(uint32_t i = 0; i < count; ++i)
+		out[i] = swchain::chain_add(start[i], step[i], n);
+}
 }

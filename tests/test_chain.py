@@ -5,6 +5,7 @@ directions and of zero, denormals, infinities and NaN, chains as long as a row."
 import ctypes as C
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -69,3 +70,25 @@ def test_long_chains(lib):
     step = (start * rng.uniform(-1, 1, n) * np.exp2(-rng.integers(8, 26, n).astype(np.float64))).astype(np.float32)
     for length in (1000, 16384, 65535):
         assert lib.check_chain_ends(C.c_void_p(start.ctypes.data), C.c_void_p(step.ctypes.data), n, length) == 0
+
+
+def test_chains_that_are_or_become_infinite_or_nan_end_at_once(lib):
+    """A chain that reaches infinity or NaN stays there: its end is found in a few steps and not walked (walked three
+    additions at a time these chains take seconds)."""
+    f = np.float32
+    values = np.array([0.0, 1.0, -2.5, 3e38, -3e38, np.inf, -np.inf, np.nan], f)
+    steps = np.array([1.0, -1.0, 2e37, -3e38, 3.4e38, np.inf, -np.inf, np.nan], f)
+    start, step = (np.ascontiguousarray(a.ravel()) for a in np.meshgrid(values, steps))
+    with np.errstate(all="ignore"):
+        walked = start.copy()
+        for _ in range(200):
+            walked = (walked + step).astype(f)
+    lost = ~np.isfinite(walked)
+    start, step, walked = (np.ascontiguousarray(a[lost]) for a in (start, step, walked))
+    assert len(start) > 40
+    out = np.empty_like(start)
+    t = time.perf_counter()
+    lib.chain_ends(C.c_void_p(start.ctypes.data), C.c_void_p(step.ctypes.data), len(start), 2 ** 24 - 1, C.c_void_p(out.ctypes.data))
+    took = time.perf_counter() - t
+    assert np.array_equal(np.isnan(out), np.isnan(walked)) and np.array_equal(out[~np.isnan(out)], walked[~np.isnan(walked)])
+    assert took < 0.05, f"{took:.3f} s"

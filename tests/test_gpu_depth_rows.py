@@ -89,3 +89,19 @@ def test_wide_rows_of_narrow_polygons(gpu_ctx, test):
     bad = np.flatnonzero(out.view(np.uint32) != ref.view(np.uint32))
     assert bad.size == 0, f"{bad.size} texels differ, first {bad[:5].tolist()}"
     assert np.any(out != init)
+
+
+def test_infinite_and_nan_equations(gpu_ctx):
+    """Equations that are infinite or NaN from the start, or overflow along a row or down a part, beside ordinary ones."""
+    rng = np.random.default_rng(33)
+    targets, draws, vdata, n = _scene(rng, [(1500, 40), (300, 64), (64, 64)], lambda t: 40, lambda i: int(i % 4 == 1))
+    bad = np.array([[0, 0, np.inf], [0, 0, -np.inf], [1e36, 0, 3e38], [0, -2e37, -3e38], [np.inf, 0, 1], [-3e38, 3e38, 0], [np.nan, 0, 0],
+                    [0, np.nan, 1]], np.float32)
+    draws["depth_equation"][::5] = bad[np.arange(len(draws[::5])) % len(bad)]
+    init = rng.uniform(-0.01, 0.01, size=n).astype(np.float32)
+    print(f"depth of infinite equations: {len(draws)} draws, {n} texels", flush=True)
+    out = gpu_ctx.render_depth(targets, draws, vdata, init)
+    ref = oracle.render_depth(targets, draws, vdata, init)
+    assert np.count_nonzero(~np.isfinite(ref)) > n // 20
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(out), nan) and np.array_equal(out.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
