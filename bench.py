@@ -267,7 +267,7 @@ def hdr_leg(ctx, args):
            "p99_ms": round(float(np.percentile(lat, 99)) * 1e3, 4),
            "triangle_draws_per_frame": round(float(np.mean(tris)), 1),
            "kernel_us_per_launch": {k: round(v[0] / max(v[1], 1) * 1e3, 3) for k, v in prof.items() if v[1]},
-           "tile_rows": rows, "scalar_spans": ctx.scalar_spans(), "with_bloom": bloom_out}
+           "tile_rows": rows, "with_bloom": bloom_out}
     log(f"hdr + models: {out}")
     return out
 

@@ -1,6 +1,6 @@
 """Frames and batches of host-resident command buffers: the queued uploads (several calls before the raster, buffers
 that grow, arrays past the size that is queued) and the copy of the frame back (pinned and pageable destinations,
-offsets, padded rows), against the oracle."""
+offsets, padded rows; left alone after an error), against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -99,5 +99,32 @@ def test_missing_host_array_is_an_error(gpu_ctx, missing, views):
             with pytest.raises(A.SwError, match="null surfaces, draws or vertex data"):
                 gpu_ctx.check(render(gpu_ctx.h, mh, C.byref(cb), _p(out)), "render")
         assert np.array_equal(gpu_ctx.render_batch(mh, b), ref)
+    finally:
+        gpu_ctx.release_map(mh)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_pinned_destination_after_an_error(gpu_ctx, bits):
+    """The copy into pinned memory is queued before the frame's errors are known: an invalid surface (a texture level out
+    of range) is reported and leaves the destination as it was; the next frame into it is the oracle's."""
+    print(f"case pinned destination after an error bits={bits}", flush=True)
+    m, b = scenes.make_batch(45, color_bits=bits, view_sizes=((160, 120),))
+    bad = scenes.make_batch(45, color_bits=bits, view_sizes=((160, 120),))[1]
+    bad.surfaces["flags"][3] |= A.SURF_DIFFUSE_LAYER
+    bad.surfaces["texture_level"][3] = 0xFFFFFF
+    ref = oracle.render(m, b, mode=oracle.MODE_EXACT)[0]
+    row = 160 * bits // 8
+    out = torch.full((row * 120,), 0x5A, dtype=torch.uint8, pin_memory=True)
+    mh = gpu_ctx.upload_map(m)
+    try:
+        for _ in range(2):
+            _draw(gpu_ctx, mh, bad)
+            with pytest.raises(A.SwError, match="invalid surface descriptor"):
+                gpu_ctx.check(gpu_ctx.lib.sw_frame_end(gpu_ctx.h, _p(out), row, 0), "end")
+            assert np.all(out.numpy() == 0x5A)
+            _draw(gpu_ctx, mh, b)
+            gpu_ctx.check(gpu_ctx.lib.sw_frame_end(gpu_ctx.h, _p(out), row, 0), "end")
+            assert np.array_equal(out.numpy().view(ref.dtype), ref)
+            out.fill_(0x5A)
     finally:
         gpu_ctx.release_map(mh)

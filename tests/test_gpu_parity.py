@@ -132,28 +132,42 @@ def test_tonemap_bit_exact(gpu_ctx, exposure, size):
 
 @pytest.mark.parametrize("color_bits", [32, 64])
 @pytest.mark.parametrize("rows", [4, 8, 16])
-@pytest.mark.parametrize("scalar_spans", [False, True])
-def test_every_tile_height_bit_exact(gpu_ctx, rows, color_bits, scalar_spans):
-    """The raster tile height and the way span records are loaded change the launch only, never a
-    pixel."""
-    _say(f"case tile rows={rows} bits={color_bits} scalar_spans={scalar_spans}")
+def test_every_tile_height_bit_exact(gpu_ctx, rows, color_bits):
+    """The raster tile height changes the launch only, never a pixel."""
+    _say(f"case tile rows={rows} bits={color_bits}")
     m, b = scenes.make_batch(30 + rows, color_bits=color_bits, view_sizes=((160, 120), (97, 61), (64, 200)))
-    prev = gpu_ctx.tile_rows(), gpu_ctx.scalar_spans()
+    prev = gpu_ctx.tile_rows()
     mh = gpu_ctx.upload_map(m)
     try:
         gpu_ctx.set_tile_rows(rows)
-        gpu_ctx.set_scalar_spans(scalar_spans)
-        assert gpu_ctx.tile_rows() == rows and gpu_ctx.scalar_spans() == scalar_spans
+        assert gpu_ctx.tile_rows() == rows
         fb = gpu_ctx.render_batch(mh, b)
         st = gpu_ctx.stats()
     finally:
-        gpu_ctx.set_tile_rows(prev[0])
-        gpu_ctx.set_scalar_spans(prev[1])
+        gpu_ctx.set_tile_rows(prev)
         gpu_ctx.release_map(mh)
     ofb, _, ost, _ = oracle.render(m, b, mode=oracle.MODE_EXACT)
     assert np.array_equal(fb, ofb)
     for k in ("polygon_pixels", "triangle_pixels", "blend_pixels"):
         assert st[k] == ost[k], (k, st[k], ost[k])
+
+
+def test_scalar_spans_are_stored_and_change_nothing(gpu_ctx):
+    """sw_set_scalar_spans is kept for callers that set it: the value comes back, the pixels stay."""
+    _say("case scalar spans")
+    m, b = scenes.make_batch(38, view_sizes=((160, 120),))
+    prev = gpu_ctx.scalar_spans()
+    mh = gpu_ctx.upload_map(m)
+    out = []
+    try:
+        for value in (not prev, prev):
+            gpu_ctx.set_scalar_spans(value)
+            assert gpu_ctx.scalar_spans() == value
+            out.append(gpu_ctx.render_batch(mh, b))
+    finally:
+        gpu_ctx.set_scalar_spans(prev)
+        gpu_ctx.release_map(mh)
+    assert np.array_equal(out[0], out[1])
 
 
 def test_autotune_keeps_output(gpu_ctx):

@@ -1,6 +1,7 @@
 """Texture operations over sizes and shifts at the edges of their index arithmetic, against the oracle: widths
 that are and are not powers of two, levels of less than a block and of several, sources of other sizes, shifts
-of any sign up to the limits of 32 bits, destinations that the first operation overwrites or blends into."""
+of any sign up to the limits of 32 bits, destinations that the first operation overwrites or blends into, calls
+of more destinations than a wave probes at once and of arguments around the size from which a kernel copies them."""
 import numpy as np
 import pytest
 
@@ -48,5 +49,51 @@ def test_layer_sizes_and_shifts(gpu_ctx, lite, first_blend):
             assert np.array_equal(gpu_ctx.map_read(mh, 1, 0, len(rlite)), rlite)
         else:
             assert np.array_equal(gpu_ctx.map_read(mh, 0, 0, len(rtex)).view(np.uint64), rtex.view(np.uint64))
+    finally:
+        gpu_ctx.release_map(mh)
+
+
+@pytest.mark.parametrize("destinations", [64, 65, 200, 5000])
+@pytest.mark.parametrize("extra", [-4, 0, 4, 40000])
+def test_many_destinations_and_argument_sizes(gpu_ctx, destinations, extra):
+    """Small levels of both kinds in turn, some of several blocks: the block's run is searched in two levels above 64
+    runs, in three above 4096. The shift table ends `extra` bytes past 16 KiB of arguments (records of 32 bytes per
+    destination and 48 per operation, each part on 256 bytes) where they leave room for it, and its last entries are
+    used."""
+    rng = np.random.default_rng([destinations, extra + 4])
+    n = destinations
+    levels = np.zeros(2 * n + 2, dtype=A.LEVEL_DTYPE)  # destinations, sources, a source for each kind of other size
+    offset = [0, 0]
+    for i in range(2 * n + 2):
+        lite = i % 2
+        w, h = (16, 16) if i >= 2 * n else ([(8, 8), (8, 8), (40, 60), (5, 3)] if n < 1000 else [(8, 8)])[i % n // 2 % (4 if n < 1000 else 1)]
+        if n % 2 and n <= i < 2 * n:
+            lite = (i - n) % 2
+        levels[i]["offset"], levels[i]["width"], levels[i]["height"] = offset[lite], w, h
+        levels[i]["flags"] = A.TEX_LITE_LEVEL if lite else 0
+        offset[lite] += w * h
+    raw = rng.integers(0, 1 << 32, size=(offset[0], 2), dtype=np.uint32)
+    data = A.MapData(np.ascontiguousarray(raw).view(A.TEXEL_DTYPE).reshape(-1), rng.integers(0, 1 << 32, offset[1], dtype=np.uint32),
+                     np.zeros((1, 3), np.float32), np.zeros(1, A.DIRLM_DTYPE), levels)
+    per = 2 if n <= 200 else 1
+    ops = np.zeros(per * n, dtype=A.TEXTURE_OP_DTYPE)
+    up = lambda x: (x + 255) // 256 * 256
+    used = up(up(32 * n) + 48 * len(ops))
+    shifts = rng.integers(-100, 100, max((16384 + extra - used) // 4, 64)).astype(np.int32)
+    for i in range(len(ops)):
+        d = i // per
+        turb = i % per == 0 and int(levels[d]["width"]) == 8
+        lite = bool(levels[d]["flags"])
+        ops[i]["kind"] = A.TEXOP_TURB if turb else A.TEXOP_LAYER_LITE if lite else A.TEXOP_LAYER
+        ops[i]["dst_level"], ops[i]["src_level"] = d, n + d if turb or d % 3 else 2 * n + int(lite)
+        ops[i]["blend"], ops[i]["shift"] = int(rng.integers(0, 5)), rng.integers(-50, 50, 2)
+        ops[i]["light"], ops[i]["turb_shifts"] = rng.uniform(0.2, 1.5, 3), len(shifts) - 8 - int(rng.integers(0, 40))
+    print(f"case texture destinations={n} extra={extra}", flush=True)
+    mh = gpu_ctx.upload_map(data)
+    try:
+        gpu_ctx.apply_texture_ops(mh, ops, shifts)
+        rtex, rlite = oracle.apply_texture_ops(data, ops, shifts)
+        assert np.array_equal(gpu_ctx.map_read(mh, 1, 0, len(rlite)), rlite)
+        assert np.array_equal(gpu_ctx.map_read(mh, 0, 0, len(rtex)).view(np.uint64), rtex.view(np.uint64))
     finally:
         gpu_ctx.release_map(mh)
