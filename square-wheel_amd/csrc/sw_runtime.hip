@@ -325,8 +325,11 @@ int stage_copy(sw_ctx* ctx, void* dst_device, size_t bytes)
 
 // A host array of a frame or batch for device buffer b: copied into pinned memory here, from there to the device
 // by one launch for all of a call's arrays (flush_uploads). A copy of its own costs each array 4 to 8 us and
-// from 16 KiB on 10 more (the DMA engine's), most of a small frame's time.
-const size_t UPLOAD_PIECE_MAX = 1 << 20, UPLOAD_SLOT_MAX = 4 << 20;
+// from 16 KiB on 10 more (the DMA engine's), most of a small frame's time. Arrays above UPLOAD_PIECE_MAX go by
+// themselves: their copy into pinned memory by this thread then costs more (batches of 24 / 64 / 96 / 200 views of
+// host arrays, us, with a limit of 128 KiB 160 / 240 / 319 / 417, of 256 KiB 154 / 239 / 314 / 397, of 512 KiB
+// 154 / 249 / 320 / 397, of 1 and 4 MiB 153 / 249 / 328 / 412; without the queue 96 views 418).
+const size_t UPLOAD_PIECE_MAX = 256 << 10, UPLOAD_SLOT_MAX = 4 << 20;
 int queue_upload(sw_ctx* ctx, DevBuf& b, const void* src, size_t bytes)
 {
 	auto& q = ctx->uploads;
