@@ -9,9 +9,10 @@
 //
 //   k_depth_setup   one wave per draw: the edge walk into parts (identical on all lanes, comparisons
 //                   only), the parts' slopes one part per lane, then one row per lane: the span's x
-//                   range and its first pixel's 1 / z. Reads the packed draws and vertices straight
-//                   from pinned host memory (each byte once, so no copy goes ahead of the launch) and
-//                   leaves in device memory what the raster reads many times.
+//                   range and its first pixel's 1 / z. Reads the packed draws, their targets and vertices
+//                   straight from pinned host memory (each draw and vertex once, a target's 40 bytes once
+//                   per draw: no copy goes ahead of the launch) and leaves in device memory what the
+//                   raster reads many times.
 //   k_depth_raster  one wave per depth-buffer row: the row's spans of the target's draws from the last
 //                   to the first, each taking the pixels no later overwriting draw has taken (64-pixel
 //                   masks, scalar arithmetic), until all are taken; then each pixel's 1 / z once.

@@ -2269,8 +2269,8 @@ SW_DEV void unit_texel_indices(const int32_t (&dwords)[DWORDS], int32_t x, uint3
 // draw's kind and blend are tested once per draw instead of once per row, and a unit that no span meets
 // costs one compare, where polygons' edges leave most of a 64-pixel strip empty. Against those strips
 // (best span load mode of each): 1920 x 1080 11.1 us from 13.6, 2560 x 1440 Color64 with 64 models and 256
-// decals 37.4 from 48.4, 256 views of 1.08e8 pixels 273 from 384, 13 views in Color64 24.1 from 32.6. Bound
-// by instruction issue (82% of the cycles issue VALU on the 256 views); tiles with hundreds of small
+// decals 37.4 from 48.4, 256 views of 1.08e8 pixels 273 from 384, 13 views in Color64 25.3 from 32.6. Bound
+// by instruction issue on many views (256 of them: vector instructions for 231 of 310 us); tiles with hundreds of small
 // triangles wait for one texel fetch per draw. Worse: eight or sixteen units together (registers), all
 // bounds' ballots before the first draw, the next draw's texel addresses during a fetch (registers, moves).
 template <class CT, int ROWS, int NK>
@@ -2783,7 +2783,9 @@ __global__ __launch_bounds__(256) void k_bloom_blur(BloomArgs a, const BlurWeigh
 // A thread takes 2 x 2 pixels of one bloom cell (cells start at odd coordinates with scale 2 and bilinear
 // upsampling), so the cell's texels, their conversion and the vertical mix are shared; the frame's two pairs
 // of pixels are 16-byte loads. With a thread per pixel, which divided by the scale for its mix, 2557 x 1439
-// took 17.7 us bilinear and 2560 x 1440 11.0 nearest; now 14.5 and 11.3 (bound by the divisions).
+// took 17.7 us bilinear and 2560 x 1440 11.0 nearest; now 14.5 and 11.3. Its 44 MB take 9.3 us at the rate of a
+// large copy and its vector instructions 6 us; the rest is the loads' latency (quotients from reciprocals instead of
+// divisions measured no faster).
 // with_average: the first row of blocks computes the average colour (dispatched first, it ends long before
 // the frame does).
 template <bool LINEAR>
@@ -3187,8 +3189,9 @@ void launch_bloom(hipStream_t st, const BloomArgs& a, bool average)
 	}
 	if(a.radius > 0)
 	{
-		// the smallest reach that holds the radius; the weights beyond the radius are 0 (radius 12: 13.5 us with
-		// a reach of 12, 14.6 with 16)
+		// the smallest reach that holds the radius; the weights beyond the radius are 0. The postprocess of a 2560 x 1440
+		// frame: radius 2 37.6 us with a reach of 2, 38.3 with 4, 42.5 with 12; radius 4 38.2 with 4, 42.5 with 12;
+		// radius 8 40.1 with 8, 42.7 with 12; the blur alone of radius 12 13.5 us with 12, 14.6 with 16
 		const int rp = a.radius <= 2 ? 2 : a.radius <= 4 ? 4 : a.radius <= 8 ? 8 : a.radius <= 12 ? 12 : 16;
 		BlurWeights w{};
 		for(int pass = 0; pass < 2; ++pass)

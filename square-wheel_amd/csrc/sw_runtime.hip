@@ -456,9 +456,9 @@ void collect_timings(sw_ctx* ctx)
 	ctx->pending.clear();
 }
 
-// Raster tile width for views of this size: a wave takes 256 pixels, 512 once that still makes 128 waves per
+// Raster tile width for views of this size: a wave takes 256 pixels, 512 once tiles of 256 would make 128 waves per
 // SIMD (binning costs a wave the same for either), and fewer while the chip gets less than four waves per
-// SIMD, since a tile then waits alone for its loads. Measured raster times (us) at 64 / 32 / 16 pixels of
+// SIMD, since a tile then waits alone for its loads. Only the tiles are counted, not the draws. Measured raster times (us) at 64 / 32 / 16 pixels of
 // width: 640 x 400 in 4 rows (1,000 tiles at 64) 8.7 / 6.8 / 6.5; 1920 x 1080 in 4 rows (8,100) 11.1 / 15.2 / -,
 // in 8 rows 13.5 / 11.6 / 15.7; 2560 x 1440 Color64 in 8 rows 53.8 / 39.7 / -; 13 views in 8 rows (62,000 tiles
 // of 256 pixels) 29.2 / 25.3 / -; 256 views in 8 rows (421,000) 273 / 341 / -.

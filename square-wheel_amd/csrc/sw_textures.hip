@@ -514,7 +514,7 @@ SW_DEV uint32_t same_address_end(const uint32_t* address, uint32_t k, uint32_t n
 // point's address with those of the 18 values it held took 0.2 us a point: two queued steps of 32 x 32 with 200
 // points 82.8 us, 67 with the points in a kernel ahead of the step, now 12.9). The field itself is updated
 // by the last of the blocks that read any point's element (they take tickets; nobody waits), when all of
-// them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 7 us
+// them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 5.7 us
 // (2.9 us of copy, 4.3 us of points and 5.3 us of stencil as three operations); its 12.6 MB take 2.6 us at
 // the rate of a large copy. VEC: both buffers are 16-byte aligned. N = 0: a step without points, which then has
 // nothing of them in its arguments either (the runtime copies 516 bytes of them otherwise: four steps of a 256 x 256
@@ -669,9 +669,12 @@ __global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, flo
 		if(!reads)
 			return; // uniform over the block
 		// Every element of the field that this block reads has been read: the sums made of them were stored
-		// before the barrier. Nothing else has to be ordered (the field is only read until the last reader
-		// writes it), so the ticket is relaxed: a fence here would write back the L2's dirty lines, most of
-		// the new field, once per reading block (the step took 10.7 us with fences).
+		// before the barrier. That is the condition the ticket stands on, and it is the hardware's order, not the
+		// memory model's: a block must read nothing of the field after its barrier (no prefetch, no load that a
+		// later change moves behind it), for the last reader may be writing it then. Nothing else has to be ordered
+		// (the field is only read until the last reader writes it), so the ticket is relaxed: a fence here would
+		// write back the L2's dirty lines, most of the new field, once per reading block (the step took 10.7 us
+		// with fences).
 		__syncthreads();
 		if(threadIdx.x == 0)
 			last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
