@@ -34,7 +34,7 @@ enum
 	COUNTER_ERROR = 9,
 	COUNTER_COUNT = 16, // size of one block
 	COUNTER_RESULT = 16, // result block [16, 32)
-	COUNTER_WATER_TICKET = 32, // k_water_step's readers that are done (its last reader clears it)
+	COUNTER_WATER_TICKET = 32, // k_water_step_points' readers that are done (its last reader clears it)
 	COUNTER_TOTAL = 36,
 };
 
@@ -338,7 +338,7 @@ void launch_depth(hipStream_t st, const char* args, const int32_t* vdata, const 
 // 256 points are 2 KiB of arguments and a thread of a block each; 64 fill the smaller argument block (0.15 us
 // of a launch less than the larger one, whose bytes the runtime copies whole).
 const uint32_t WATER_ARG_POINTS_SMALL = 64u, WATER_ARG_POINTS = 256u;
-const uint32_t WATER_BLOCK = 1024u; // elements of a k_water_step block
+const uint32_t WATER_BLOCK = 1024u; // elements of a water step's block
 const uint32_t WATER_MAX_BLOCKS = (1u << 21) / WATER_BLOCK; // field areas are below 2^22: at most 2^21
 template <uint32_t N>
 struct WavePoints
@@ -346,10 +346,6 @@ struct WavePoints
 	uint32_t n;
 	uint32_t address[N];
 	float value[N];
-};
-template <>
-struct WavePoints<0> // a step without points
-{
 };
 // neighbour n (left, right, up, down) of element a on the torus
 __host__ __device__ inline uint32_t water_neighbour(uint32_t a, uint32_t n, uint32_t log2w, uint32_t log2h)

@@ -506,196 +506,221 @@ SW_DEV uint32_t same_address_end(const uint32_t* address, uint32_t k, uint32_t n
 	return lo;
 }
 
-// update_wave_field (:307-418), with the step's points (add_point_value, :68-76) where they travel in the
-// kernel's arguments: the field is a torus (rows and columns wrap); a block takes WATER_BLOCK consecutive
-// elements, four per thread. The stencil reads the field with the points added: a block that points touch
-// passes its values through LDS, where a thread per address adds that address's points in their order (the
+// Four consecutive elements of a thread and what the stencil reads for them.
+struct WaterQuad
+{
+	uint32_t block, i, il, ir; // the block's place in the field; the first element, the neighbours left and right of the four
+	bool in;
+	float c[6], u[4], d[4], o[4]; // the row from il to ir, the elements above and below, the old field
+};
+
+// The thread's four elements, read. VEC: both buffers are 16-byte aligned.
+// Blocks are dealt to the eight XCDs in turn: each takes a contiguous eighth of the field, so that a row's
+// neighbours above and below come from the same L2 (four queued steps of 1024 x 1024 without points: 23.8 us
+// with consecutive blocks on different XCDs, 16.9 so). The number of blocks comes from the size: read as gridDim it
+// would have the runtime fill in the kernel's hidden arguments for every launch.
+template <bool VEC>
+SW_DEV WaterQuad water_load(const float* src, const float* old, uint32_t log2w, uint32_t log2h)
+{
+	WaterQuad q;
+	const uint32_t each = (1u << (log2w + log2h)) / (8u * swk::WATER_BLOCK); // blocks of an XCD
+	q.block = each ? blockIdx.x % 8u * each + blockIdx.x / 8u : blockIdx.x;
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	q.i = q.block * swk::WATER_BLOCK + threadIdx.x * 4u;
+	q.in = (q.i >> (log2w + log2h)) == 0;
+	const uint32_t x = q.i & mx, y = q.i >> log2w;
+	const uint32_t row = y << log2w, up = (((y - 1u) & my) << log2w) + x, down = (((y + 1u) & my) << log2w) + x;
+	q.il = row + ((x - 1u) & mx);
+	q.ir = row + ((x + 4u) & mx);
+	if(q.in)
+	{
+		q.c[0] = src[q.il];
+		q.c[5] = src[q.ir];
+		if(VEC)
+		{
+			const float4 c4 = *reinterpret_cast<const float4*>(src + q.i), u4 = *reinterpret_cast<const float4*>(src + up),
+						 d4 = *reinterpret_cast<const float4*>(src + down), o4 = *reinterpret_cast<const float4*>(old + q.i);
+			q.c[1] = c4.x, q.c[2] = c4.y, q.c[3] = c4.z, q.c[4] = c4.w;
+			q.u[0] = u4.x, q.u[1] = u4.y, q.u[2] = u4.z, q.u[3] = u4.w;
+			q.d[0] = d4.x, q.d[1] = d4.y, q.d[2] = d4.z, q.d[3] = d4.w;
+			q.o[0] = o4.x, q.o[1] = o4.y, q.o[2] = o4.z, q.o[3] = o4.w;
+		}
+		else
+#pragma unroll
+			for(uint32_t k = 0; k < 4; ++k)
+			{
+				q.c[k + 1] = src[q.i + k];
+				q.u[k] = src[up + k];
+				q.d[k] = src[down + k];
+				q.o[k] = old[q.i + k];
+			}
+	}
+	return q;
+}
+
+// update_wave_field (:307-418) of the thread's elements
+template <bool VEC>
+SW_DEV void water_store(const WaterQuad& q, float* dst, float attenuation)
+{
+	if(!q.in)
+		return;
+	float r[4];
+#pragma unroll
+	for(uint32_t k = 0; k < 4; ++k)
+	{
+		const float sum = ((q.c[k] + q.c[k + 2]) + q.u[k]) + q.d[k];
+		r[k] = (sum * 0.5f - q.o[k]) * attenuation;
+	}
+	if(VEC)
+		*reinterpret_cast<float4*>(dst + q.i) = make_float4(r[0], r[1], r[2], r[3]);
+	else
+#pragma unroll
+		for(uint32_t k = 0; k < 4; ++k)
+			dst[q.i + k] = r[k];
+}
+
+// A step without points: the field is a torus (rows and columns wrap). Its own kernel, with no more arguments than it
+// needs: queued steps of a field up to 256 x 256 are bound by the host's launches, and those by the bytes of arguments
+// (4.2 us a step with the points' arguments or, without them, with gridDim's, 3.7 so).
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, const float* __restrict__ src, uint32_t log2w, uint32_t log2h,
+	float attenuation)
+{
+	const WaterQuad q = water_load<VEC>(src, dst, log2w, log2h);
+	water_store<VEC>(q, dst, attenuation);
+}
+
+// A step with its points (add_point_value, :68-76), which travel in the kernel's arguments. The stencil reads the
+// field with the points added: a block that points touch passes its values through LDS, where a thread per address adds that address's points in their order (the
 // reference's) wherever the value is held and subtracts them from the old field (every thread comparing each
 // point's address with those of the 18 values it held took 0.2 us a point: two queued steps of 32 x 32 with 200
 // points 82.8 us, 67 with the points in a kernel ahead of the step, now 12.9). The field itself is updated
 // by the last of the blocks that read any point's element (they take tickets; nobody waits), when all of
 // them have read it. One launch per step, no copy ahead of it. A 1024 x 1024 step with 16 points takes 5.7 us
 // (2.9 us of copy, 4.3 us of points and 5.3 us of stencil as three operations); its 12.6 MB take 2.6 us at
-// the rate of a large copy. VEC: both buffers are 16-byte aligned. N = 0: a step without points, which then has
-// nothing of them in its arguments either (the runtime copies 516 bytes of them otherwise: four steps of a 256 x 256
-// field queued behind each other 17.7 us with them, 16.5 without).
+// the rate of a large copy.
 template <uint32_t N, bool VEC>
-__global__ __launch_bounds__(256) void k_water_step(float* __restrict__ dst, float* __restrict__ src, uint32_t log2w, uint32_t log2h,
+__global__ __launch_bounds__(256) void k_water_step_points(float* __restrict__ dst, float* __restrict__ src, uint32_t log2w, uint32_t log2h,
 	float attenuation, swk::WavePoints<N> pts, uint32_t readers, uint32_t* __restrict__ ticket)
 {
-	// points only: the block's values by element (its own, their neighbours above and below, the old field, the
+	// the block's values by element (its own, their neighbours above and below, the old field, the
 	// neighbours left and right of its ends), and whether points touch them
-	__shared__ __align__(16) float l_own[N ? swk::WATER_BLOCK : 1], l_up[N ? swk::WATER_BLOCK : 1], l_down[N ? swk::WATER_BLOCK : 1],
-		l_old[N ? swk::WATER_BLOCK : 1], l_ends[2], l_value[N ? N : 1];
-	__shared__ uint32_t l_address[N ? N : 1], touched, reads, last;
-	// Blocks are dealt to the eight XCDs in turn: each takes a contiguous eighth of the field, so that a row's
-	// neighbours above and below come from the same L2 (four queued steps of 1024 x 1024 without points: 23.8 us
-	// with consecutive blocks on different XCDs, 16.9 so).
-	const uint32_t block = gridDim.x % 8u ? blockIdx.x : blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u;
-	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
-	const uint32_t i = block * swk::WATER_BLOCK + threadIdx.x * 4u;
-	const bool in = (i >> (log2w + log2h)) == 0;
-	const uint32_t x = i & mx, y = i >> log2w;
-	const uint32_t row = y << log2w, up = (((y - 1u) & my) << log2w) + x, down = (((y + 1u) & my) << log2w) + x;
-	const uint32_t il = row + ((x - 1u) & mx), ir = row + ((x + 4u) & mx);
-	float c[6], u[4], d[4], o[4];
-	if(in)
+	__shared__ __align__(16) float l_own[swk::WATER_BLOCK], l_up[swk::WATER_BLOCK], l_down[swk::WATER_BLOCK], l_old[swk::WATER_BLOCK],
+		l_ends[2], l_value[N];
+	__shared__ uint32_t l_address[N], touched, reads, last;
+	WaterQuad q = water_load<VEC>(src, dst, log2w, log2h);
+	if(threadIdx.x == 0)
+		touched = reads = 0;
+	__syncthreads();
+	// thread k's point: its address, whether it is the first of its address, and the elements that it is read by
+	static_assert(N <= 256u);
+	const uint32_t k = threadIdx.x, b0 = q.block * swk::WATER_BLOCK;
+	const bool has = k < pts.n;
+	const uint32_t a = pts.address[has ? k : 0u], before = pts.address[has && k > 0u ? k - 1u : 0u];
+	const float v0 = pts.value[has ? k : 0u];
+	const bool first = has && (k == 0u || before != a);
+	if(has)
 	{
-		c[0] = src[il];
-		c[5] = src[ir];
-		if(VEC)
-		{
-			const float4 c4 = *reinterpret_cast<const float4*>(src + i), u4 = *reinterpret_cast<const float4*>(src + up),
-						 d4 = *reinterpret_cast<const float4*>(src + down), o4 = *reinterpret_cast<const float4*>(dst + i);
-			c[1] = c4.x, c[2] = c4.y, c[3] = c4.z, c[4] = c4.w;
-			u[0] = u4.x, u[1] = u4.y, u[2] = u4.z, u[3] = u4.w;
-			d[0] = d4.x, d[1] = d4.y, d[2] = d4.z, d[3] = d4.w;
-			o[0] = o4.x, o[1] = o4.y, o[2] = o4.z, o[3] = o4.w;
-		}
-		else
-#pragma unroll
-			for(uint32_t k = 0; k < 4; ++k)
-			{
-				c[k + 1] = src[i + k];
-				u[k] = src[up + k];
-				d[k] = src[down + k];
-				o[k] = dst[i + k];
-			}
+		l_address[k] = a;
+		l_value[k] = v0;
 	}
-	if constexpr(N > 0)
-	{
-		if(threadIdx.x == 0)
-			touched = reads = 0;
-		__syncthreads();
-		// thread k's point: its address, whether it is the first of its address, and the elements that it is read by
-		static_assert(N <= 256u);
-		const uint32_t k = threadIdx.x, b0 = block * swk::WATER_BLOCK;
-		const bool has = k < pts.n;
-		const uint32_t a = pts.address[has ? k : 0u], before = pts.address[has && k > 0u ? k - 1u : 0u];
-		const float v0 = pts.value[has ? k : 0u];
-		const bool first = has && (k == 0u || before != a);
-		if(has)
-		{
-			l_address[k] = a;
-			l_value[k] = v0;
-		}
-		uint32_t at[4]; // of the block: its right, left, lower and upper neighbour, whose left, ... neighbour it is
-		bool read = false;
+	uint32_t at[4]; // of the block: its right, left, lower and upper neighbour, whose left, ... neighbour it is
+	bool read = false;
 #pragma unroll
-		for(uint32_t n = 0; n < 4; ++n)
-		{
-			at[n] = swk::water_neighbour(a, n ^ 1u, log2w, log2h) - b0;
-			read = read || at[n] < swk::WATER_BLOCK;
-		}
-		const uint32_t own = a - b0;
-		if(has && read)
-			reads = 1; // every writer writes 1
-		if(has && (read || own < swk::WATER_BLOCK))
-			touched = 1;
-		__syncthreads();
-		if(touched)
-		{
-			// uniform over the block: the values go through LDS, where a thread per address adds its points in turn
-			const uint32_t t4 = threadIdx.x * 4u;
-			*reinterpret_cast<float4*>(l_own + t4) = make_float4(c[1], c[2], c[3], c[4]);
-			*reinterpret_cast<float4*>(l_up + t4) = make_float4(u[0], u[1], u[2], u[3]);
-			*reinterpret_cast<float4*>(l_down + t4) = make_float4(d[0], d[1], d[2], d[3]);
-			*reinterpret_cast<float4*>(l_old + t4) = make_float4(o[0], o[1], o[2], o[3]);
-			// the neighbour left of an element of the block is its predecessor, or lies at its row's other end: in the
-			// block if it holds whole rows, else only the first thread's is outside (right alike)
-			const bool left_in = il - b0 < swk::WATER_BLOCK, right_in = ir - b0 < swk::WATER_BLOCK;
-			if(!left_in)
-				l_ends[0] = c[0];
-			if(!right_in)
-				l_ends[1] = c[5];
-			__syncthreads();
-			if(first && (read || own < swk::WATER_BLOCK))
-			{
-				// whatever place holds the element's value, all of them hold the same
-				const bool is_own = own < swk::WATER_BLOCK, is_left = !is_own && at[0] < swk::WATER_BLOCK,
-						   is_right = !is_own && at[1] < swk::WATER_BLOCK, is_up = at[2] < swk::WATER_BLOCK, is_down = at[3] < swk::WATER_BLOCK;
-				float f = is_own ? l_own[own] : is_left ? l_ends[0] : is_right ? l_ends[1] : is_up ? l_up[at[2]] : l_down[at[3]];
-				float old = is_own ? l_old[own] : 0.0f;
-				const uint32_t end = same_address_end(l_address, k, pts.n);
-#pragma unroll 8
-				for(uint32_t j = k; j < end; ++j)
-				{
-					f += l_value[j];
-					old -= l_value[j];
-				}
-				if(is_own)
-				{
-					l_own[own] = f;
-					l_old[own] = old;
-				}
-				if(is_left)
-					l_ends[0] = f;
-				if(is_right)
-					l_ends[1] = f;
-				if(is_up)
-					l_up[at[2]] = f;
-				if(is_down)
-					l_down[at[3]] = f;
-			}
-			__syncthreads();
-			const float4 c4 = *reinterpret_cast<const float4*>(l_own + t4), u4 = *reinterpret_cast<const float4*>(l_up + t4),
-						 d4 = *reinterpret_cast<const float4*>(l_down + t4), o4 = *reinterpret_cast<const float4*>(l_old + t4);
-			c[0] = left_in ? l_own[il - b0] : l_ends[0];
-			c[1] = c4.x, c[2] = c4.y, c[3] = c4.z, c[4] = c4.w;
-			c[5] = right_in ? l_own[ir - b0] : l_ends[1];
-			u[0] = u4.x, u[1] = u4.y, u[2] = u4.z, u[3] = u4.w;
-			d[0] = d4.x, d[1] = d4.y, d[2] = d4.z, d[3] = d4.w;
-			o[0] = o4.x, o[1] = o4.y, o[2] = o4.z, o[3] = o4.w;
-		}
+	for(uint32_t n = 0; n < 4; ++n)
+	{
+		at[n] = swk::water_neighbour(a, n ^ 1u, log2w, log2h) - b0;
+		read = read || at[n] < swk::WATER_BLOCK;
 	}
-	if(in)
+	const uint32_t own = a - b0;
+	if(has && read)
+		reads = 1; // every writer writes 1
+	if(has && (read || own < swk::WATER_BLOCK))
+		touched = 1;
+	__syncthreads();
+	if(touched)
 	{
-		float r[4];
-#pragma unroll
-		for(uint32_t k = 0; k < 4; ++k)
-		{
-			const float sum = ((c[k] + c[k + 2]) + u[k]) + d[k];
-			r[k] = (sum * 0.5f - o[k]) * attenuation;
-		}
-		if(VEC)
-			*reinterpret_cast<float4*>(dst + i) = make_float4(r[0], r[1], r[2], r[3]);
-		else
-#pragma unroll
-			for(uint32_t k = 0; k < 4; ++k)
-				dst[i + k] = r[k];
-	}
-	if constexpr(N > 0)
-	{
-		if(!reads)
-			return; // uniform over the block
-		// Every element of the field that this block reads has been read: the sums made of them were stored
-		// before the barrier. That is the condition the ticket stands on, and it is the hardware's order, not the
-		// memory model's: a block must read nothing of the field after its barrier (no prefetch, no load that a
-		// later change moves behind it), for the last reader may be writing it then. Nothing else has to be ordered
-		// (the field is only read until the last reader writes it), so the ticket is relaxed: a fence here would
-		// write back the L2's dirty lines, most of the new field, once per reading block (the step took 10.7 us
-		// with fences).
+		// uniform over the block: the values go through LDS, where a thread per address adds its points in turn
+		const uint32_t t4 = threadIdx.x * 4u;
+		*reinterpret_cast<float4*>(l_own + t4) = make_float4(q.c[1], q.c[2], q.c[3], q.c[4]);
+		*reinterpret_cast<float4*>(l_up + t4) = make_float4(q.u[0], q.u[1], q.u[2], q.u[3]);
+		*reinterpret_cast<float4*>(l_down + t4) = make_float4(q.d[0], q.d[1], q.d[2], q.d[3]);
+		*reinterpret_cast<float4*>(l_old + t4) = make_float4(q.o[0], q.o[1], q.o[2], q.o[3]);
+		// the neighbour left of an element of the block is its predecessor, or lies at its row's other end: in the
+		// block if it holds whole rows, else only the first thread's is outside (right alike)
+		const bool left_in = q.il - b0 < swk::WATER_BLOCK, right_in = q.ir - b0 < swk::WATER_BLOCK;
+		if(!left_in)
+			l_ends[0] = q.c[0];
+		if(!right_in)
+			l_ends[1] = q.c[5];
 		__syncthreads();
-		if(threadIdx.x == 0)
-			last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
-		__syncthreads();
-		if(!last)
-			return;
-		// the last reader: an address's points lie together, its first point's thread adds them up in order
-		const uint32_t k = threadIdx.x;
-		if(k < pts.n && (k == 0u || l_address[k - 1u] != l_address[k]))
+		if(first && (read || own < swk::WATER_BLOCK))
 		{
-			const uint32_t a = l_address[k];
+			// whatever place holds the element's value, all of them hold the same
+			const bool is_own = own < swk::WATER_BLOCK, is_left = !is_own && at[0] < swk::WATER_BLOCK,
+					   is_right = !is_own && at[1] < swk::WATER_BLOCK, is_up = at[2] < swk::WATER_BLOCK, is_down = at[3] < swk::WATER_BLOCK;
+			float f = is_own ? l_own[own] : is_left ? l_ends[0] : is_right ? l_ends[1] : is_up ? l_up[at[2]] : l_down[at[3]];
+			float old = is_own ? l_old[own] : 0.0f;
 			const uint32_t end = same_address_end(l_address, k, pts.n);
-			float f = src[a];
 #pragma unroll 8
 			for(uint32_t j = k; j < end; ++j)
+			{
 				f += l_value[j];
-			src[a] = f;
+				old -= l_value[j];
+			}
+			if(is_own)
+			{
+				l_own[own] = f;
+				l_old[own] = old;
+			}
+			if(is_left)
+				l_ends[0] = f;
+			if(is_right)
+				l_ends[1] = f;
+			if(is_up)
+				l_up[at[2]] = f;
+			if(is_down)
+				l_down[at[3]] = f;
 		}
-		if(threadIdx.x == 0)
-			*ticket = 0;
+		__syncthreads();
+		const float4 c4 = *reinterpret_cast<const float4*>(l_own + t4), u4 = *reinterpret_cast<const float4*>(l_up + t4),
+					 d4 = *reinterpret_cast<const float4*>(l_down + t4), o4 = *reinterpret_cast<const float4*>(l_old + t4);
+		q.c[0] = left_in ? l_own[q.il - b0] : l_ends[0];
+		q.c[1] = c4.x, q.c[2] = c4.y, q.c[3] = c4.z, q.c[4] = c4.w;
+		q.c[5] = right_in ? l_own[q.ir - b0] : l_ends[1];
+		q.u[0] = u4.x, q.u[1] = u4.y, q.u[2] = u4.z, q.u[3] = u4.w;
+		q.d[0] = d4.x, q.d[1] = d4.y, q.d[2] = d4.z, q.d[3] = d4.w;
+		q.o[0] = o4.x, q.o[1] = o4.y, q.o[2] = o4.z, q.o[3] = o4.w;
 	}
+	water_store<VEC>(q, dst, attenuation);
+	if(!reads)
+		return; // uniform over the block
+	// Every element of the field that this block reads has been read: the sums made of them were stored
+	// before the barrier. That is the condition the ticket stands on, and it is the hardware's order, not the
+	// memory model's: a block must read nothing of the field after its barrier (no prefetch, no load that a
+	// later change moves behind it), for the last reader may be writing it then. Nothing else has to be ordered
+	// (the field is only read until the last reader writes it), so the ticket is relaxed: a fence here would
+	// write back the L2's dirty lines, most of the new field, once per reading block (the step took 10.7 us
+	// with fences).
+	__syncthreads();
+	if(threadIdx.x == 0)
+		last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == readers - 1u ? 1u : 0u;
+	__syncthreads();
+	if(!last)
+		return;
+	// the last reader: an address's points lie together, its first point's thread adds them up in order
+	if(k < pts.n && (k == 0u || l_address[k - 1u] != l_address[k]))
+	{
+		const uint32_t a = l_address[k];
+		const uint32_t end = same_address_end(l_address, k, pts.n);
+		float f = src[a];
+#pragma unroll 8
+		for(uint32_t j = k; j < end; ++j)
+			f += l_value[j];
+		src[a] = f;
+	}
+	if(threadIdx.x == 0)
+		*ticket = 0;
 }
 
 // PackedNormalRoughness::pack (textures.rs:33-39, fast_math.rs:64-78): x 127 per lane, cvtps2dq,
@@ -1121,39 +1146,49 @@ __global__ __launch_bounds__(64) void k_fire_points(uint8_t* heat, const sw_heat
 
 namespace swk
 {
+static uint32_t water_blocks(uint32_t log2w, uint32_t log2h) { return ((1u << (log2w + log2h)) + WATER_BLOCK - 1u) / WATER_BLOCK; }
+static bool water_aligned(const float* field, const float* field_old)
+{
+	return (reinterpret_cast<uintptr_t>(field) | reinterpret_cast<uintptr_t>(field_old)) % 16 == 0;
+}
+
+static void launch_water_step_alone(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation)
+{
+	const dim3 grid(water_blocks(log2w, log2h));
+	if(water_aligned(field, field_old))
+		hipLaunchKernelGGL(k_water_step<true>, grid, dim3(256), 0, st, field_old, static_cast<const float*>(field), log2w, log2h, attenuation);
+	else
+		hipLaunchKernelGGL(k_water_step<false>, grid, dim3(256), 0, st, field_old, static_cast<const float*>(field), log2w, log2h, attenuation);
+}
+
 template <uint32_t N>
 static void launch_water_step_n(hipStream_t st, float* field, float* field_old, uint32_t log2w, uint32_t log2h, float attenuation,
 	const sw_wave_point* points, uint32_t num_points, uint32_t* ticket)
 {
 	WavePoints<N> p;
-	uint32_t num_readers = 0;
-	if constexpr(N > 0)
+	p.n = num_points;
+	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
+	// sorted by address, an address's points in their order: only their own order matters to it
+	uint64_t order[N];
+	for(uint32_t k = 0; k < num_points; ++k)
+		order[k] = (uint64_t((points[k].x & mx) + ((points[k].y & my) << log2w)) << 32) | k;
+	std::sort(order, order + num_points);
+	// the blocks that read a point's element: those of its four neighbours
+	std::bitset<WATER_MAX_BLOCKS> readers;
+	for(uint32_t k = 0; k < num_points; ++k)
 	{
-		p.n = num_points;
-		const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
-		// sorted by address, an address's points in their order: only their own order matters to it
-		uint64_t order[N];
-		for(uint32_t k = 0; k < num_points; ++k)
-			order[k] = (uint64_t((points[k].x & mx) + ((points[k].y & my) << log2w)) << 32) | k;
-		std::sort(order, order + num_points);
-		// the blocks that read a point's element: those of its four neighbours
-		std::bitset<WATER_MAX_BLOCKS> readers;
-		for(uint32_t k = 0; k < num_points; ++k)
-		{
-			p.address[k] = uint32_t(order[k] >> 32);
-			p.value[k] = points[uint32_t(order[k])].value;
-			for(uint32_t n = 0; n < 4; ++n)
-				readers.set(water_neighbour(p.address[k], n, log2w, log2h) / WATER_BLOCK);
-		}
-		num_readers = uint32_t(readers.count());
+		p.address[k] = uint32_t(order[k] >> 32);
+		p.value[k] = points[uint32_t(order[k])].value;
+		for(uint32_t n = 0; n < 4; ++n)
+			readers.set(water_neighbour(p.address[k], n, log2w, log2h) / WATER_BLOCK);
 	}
-	const uint32_t blocks = ((1u << (log2w + log2h)) + WATER_BLOCK - 1u) / WATER_BLOCK;
-	const bool vec = (reinterpret_cast<uintptr_t>(field) | reinterpret_cast<uintptr_t>(field_old)) % 16 == 0;
-	if(vec)
-		hipLaunchKernelGGL((k_water_step<N, true>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
+	const uint32_t num_readers = uint32_t(readers.count());
+	const dim3 grid(water_blocks(log2w, log2h));
+	if(water_aligned(field, field_old))
+		hipLaunchKernelGGL((k_water_step_points<N, true>), grid, dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
 			num_readers, ticket);
 	else
-		hipLaunchKernelGGL((k_water_step<N, false>), dim3(blocks), dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
+		hipLaunchKernelGGL((k_water_step_points<N, false>), grid, dim3(256), 0, st, field_old, field, log2w, log2h, attenuation, p,
 			num_readers, ticket);
 }
 
@@ -1162,7 +1197,7 @@ void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t 
 {
 	// the smallest argument block that holds the points: the runtime copies the whole block per launch
 	if(num_points == 0)
-		launch_water_step_n<0>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
+		launch_water_step_alone(st, field, field_old, log2w, log2h, attenuation);
 	else if(num_points <= WATER_ARG_POINTS_SMALL)
 		launch_water_step_n<WATER_ARG_POINTS_SMALL>(st, field, field_old, log2w, log2h, attenuation, points, num_points, ticket);
 	else if(num_points <= WATER_ARG_POINTS)
@@ -1170,7 +1205,7 @@ void launch_water_step(hipStream_t st, float* field, float* field_old, uint32_t 
 	else
 	{
 		hipLaunchKernelGGL(k_water_points, dim3(1), dim3(64), 0, st, field, field_old, points_dev, num_points, log2w, log2h);
-		launch_water_step_n<0>(st, field, field_old, log2w, log2h, attenuation, nullptr, 0, ticket);
+		launch_water_step_alone(st, field, field_old, log2w, log2h, attenuation);
 	}
 }
 

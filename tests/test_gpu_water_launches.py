@@ -132,6 +132,30 @@ def test_water_unaligned_fields(gpu_ctx, shift):
     assert np.array_equal(texels.view(np.uint64), ref.view(np.uint64))
 
 
+@pytest.mark.parametrize("log2", [(4, 4), (5, 6), (6, 7), (9, 5)])
+@pytest.mark.parametrize("shift", [(0, 0), (1, 0), (0, 3)])
+def test_water_step_alone(gpu_ctx, log2, shift):
+    """A step without points: fields of less than a block, of a block for some XCDs and of several for each, both alignments."""
+    lw, lh = log2
+    n = 1 << (lw + lh)
+    rng = np.random.default_rng([lw, lh, *shift])
+    f, fo = rng.normal(size=n).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    bufs = [gpu_ctx.to_device(np.concatenate([np.full(s, 9, np.float32), v, np.full(4, 9, np.float32)])) for s, v in zip(shift, (f, fo))]
+    ptr = [C.c_void_p(b.ptr.value + 4 * s) for s, b in zip(shift, bufs)]
+    try:
+        print(f"water step of {1 << lw} x {1 << lh} without points at float offsets {shift}", flush=True)
+        gpu_ctx.check(gpu_ctx.lib.sw_water_step(gpu_ctx.h, ptr[0], ptr[1], lw, lh, C.c_float(0.98), None, 0), "sw_water_step")
+        gpu_ctx.check(gpu_ctx.lib.sw_sync(gpu_ctx.h), "sw_sync")
+        got = [b.read(np.float32, n + s + 4) for s, b in zip(shift, bufs)]
+    finally:
+        for b in bufs:
+            b.free()
+    new, old = oracle.water_step(f, fo, lw, lh, np.float32(0.98), np.zeros(0, A.WAVE_POINT_DTYPE))
+    for g, s, ref in zip(got, shift, (old, new)):
+        assert np.array_equal(g[s:s + n].view(np.uint32), ref.view(np.uint32))
+        assert np.all(g[:s] == 9) and np.all(g[s + n:] == 9)
+
+
 def test_water_texture_level_not_on_16_bytes(gpu_ctx):
     """A level that starts on an odd texel (8 bytes past a multiple of 16)."""
     lw, lh = 5, 4
