@@ -976,9 +976,9 @@ namespace
 // with no copy ahead of it: bound by launch latency (a 64 x 64 map's step: 2.2 us of update, 9.4 us of
 // points and 2.7 us of copy as three operations, 3 us as one). WORDS: both buffers are 4-byte
 // aligned, texels move as words.
-template <uint32_t N, bool WORDS>
-__global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
-	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
+template <bool POINTS, bool WORDS>
+SW_DEV void fire_step_fast(const uint8_t* src, uint8_t* dst, uint32_t log2w, uint32_t log2h, uint32_t att, const uint32_t* points,
+	uint32_t num_points)
 {
 	__shared__ __align__(16) uint32_t cells[1024];
 	const uint32_t w = 1u << log2w, h = 1u << log2h, mx = w - 1u;
@@ -1010,13 +1010,13 @@ __global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restric
 		for(uint32_t k = 0; k < 4; ++k)
 			v[k] = ((a[k] + a[k + 1] + a[k + 2] + c[k]) * att) >> 20;
 	}
-	if(pts.n)
+	if constexpr(POINTS)
 	{
 		*reinterpret_cast<uint4*>(cells + threadIdx.x * 4u) = make_uint4(v[0], v[1], v[2], v[3]);
 		__syncthreads();
-		for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+		for(uint32_t k = threadIdx.x; k < num_points; k += 256u)
 		{
-			const uint32_t p = pts.p[k], a = (p & swk::FIRE_POINT_ADDRESS) - b0;
+			const uint32_t p = points[k], a = (p & swk::FIRE_POINT_ADDRESS) - b0;
 			if(a < 1024u)
 				atomicMax(&cells[a], p >> swk::FIRE_POINT_HEAT_SHIFT);
 		}
@@ -1036,6 +1036,21 @@ __global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restric
 			dst[i + k] = uint8_t(v[k]);
 }
 
+template <uint32_t N, bool WORDS>
+__global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
+{
+	fire_step_fast<true, WORDS>(src, dst, log2w, log2h, att, pts.p, pts.n);
+}
+// A step without points, with no more arguments than it needs: queued steps of small maps are bound by the host's
+// launches (4.3 us a step with the points' arguments, 3.6 so; the slow variant alike, at 256 x 256 13.1 us by its chain).
+template <bool WORDS>
+__global__ __launch_bounds__(256) void k_fire_update_fast(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att)
+{
+	fire_step_fast<false, WORDS>(src, dst, log2w, log2h, att, nullptr, 0);
+}
+
 // The slow variant: each row is a chain (the left neighbour is the value just written; the last
 // texel's right neighbour is the row's new first texel), from the row and the row below. A block
 // takes 16 rows, 256 columns at a time: all threads sum what a texel reads besides its left neighbour
@@ -1045,9 +1060,9 @@ __global__ __launch_bounds__(256) void k_fire_step_fast(const uint8_t* __restric
 // bytes the 64 x 64 step took 5.3 us of update beside the points' 9.4 us.
 #define FIRE_SLOW_ROWS 16u
 #define FIRE_SLOW_COLS 256u
-template <uint32_t N>
-__global__ __launch_bounds__(256) void k_fire_step_slow(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
-	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
+template <bool POINTS>
+SW_DEV void fire_step_slow(const uint8_t* src, uint8_t* dst, uint32_t log2w, uint32_t log2h, uint32_t att, const uint32_t* points,
+	uint32_t num_points)
 {
 	// a row's cells: the sums, then the chain's values (a word between rows: the chain's lanes read 16
 	// rows at one column, which then lie in 16 banks)
@@ -1085,11 +1100,11 @@ __global__ __launch_bounds__(256) void k_fire_step_slow(const uint8_t* __restric
 			}
 		}
 		__syncthreads();
-		if(pts.n)
+		if constexpr(POINTS)
 		{
-			for(uint32_t k = threadIdx.x; k < pts.n; k += 256u)
+			for(uint32_t k = threadIdx.x; k < num_points; k += 256u)
 			{
-				const uint32_t p = pts.p[k], a = p & swk::FIRE_POINT_ADDRESS;
+				const uint32_t p = points[k], a = p & swk::FIRE_POINT_ADDRESS;
 				const uint32_t px = (a & (w - 1u)) - x0, py = (a >> log2w) - y0;
 				if(px < cols && py < FIRE_SLOW_ROWS)
 					atomicMax(&cells[py][px], p >> swk::FIRE_POINT_HEAT_SHIFT);
@@ -1103,6 +1118,18 @@ __global__ __launch_bounds__(256) void k_fire_step_slow(const uint8_t* __restric
 		}
 		__syncthreads(); // the next columns rewrite the cells
 	}
+}
+
+template <uint32_t N>
+__global__ __launch_bounds__(256) void k_fire_step_slow(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att, swk::FirePoints<N> pts)
+{
+	fire_step_slow<true>(src, dst, log2w, log2h, att, pts.p, pts.n);
+}
+__global__ __launch_bounds__(256) void k_fire_update_slow(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t log2w,
+	uint32_t log2h, uint32_t att)
+{
+	fire_step_slow<false>(src, dst, log2w, log2h, att, nullptr, 0);
 }
 
 // set_heat (:80-86) for more points than a step's kernel arguments hold, 64 at a time: the first point
@@ -1218,6 +1245,24 @@ void launch_water_texture(hipStream_t st, const float* field, uint32_t log2w, ui
 	else
 		hipLaunchKernelGGL(k_water_texture<false>, grid, dim3(256), 0, st, field, log2w, log2h, tiles, w, texels);
 }
+static uint32_t fire_blocks(uint32_t log2w, uint32_t log2h) { return ((1u << (log2w + log2h)) + 1023u) / 1024u; }
+static bool fire_aligned(const uint8_t* heat, const uint8_t* heat_old)
+{
+	return (reinterpret_cast<uintptr_t>(heat) | reinterpret_cast<uintptr_t>(heat_old)) % 4 == 0;
+}
+
+static void launch_fire_update(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h,
+	uint32_t attenuation_i, bool slow)
+{
+	const dim3 grid(slow ? (1u << log2h) / FIRE_SLOW_ROWS : fire_blocks(log2w, log2h));
+	if(slow)
+		hipLaunchKernelGGL(k_fire_update_slow, grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i);
+	else if(fire_aligned(heat, heat_old))
+		hipLaunchKernelGGL(k_fire_update_fast<true>, grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i);
+	else
+		hipLaunchKernelGGL(k_fire_update_fast<false>, grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i);
+}
+
 template <uint32_t N>
 static void launch_fire_step_n(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h,
 	uint32_t attenuation_i, bool slow, const sw_heat_point* points, uint32_t num_points)
@@ -1227,27 +1272,28 @@ static void launch_fire_step_n(hipStream_t st, const uint8_t* heat, uint8_t* hea
 	const uint32_t mx = (1u << log2w) - 1u, my = (1u << log2h) - 1u;
 	for(uint32_t k = 0; k < num_points; ++k)
 		p.p[k] = ((points[k].x & mx) + ((points[k].y & my) << log2w)) | ((points[k].heat & 0xFFu) << FIRE_POINT_HEAT_SHIFT);
-	const uint32_t blocks = ((1u << (log2w + log2h)) + 1023u) / 1024u;
+	const dim3 grid(slow ? (1u << log2h) / FIRE_SLOW_ROWS : fire_blocks(log2w, log2h));
 	if(slow)
-		hipLaunchKernelGGL(k_fire_step_slow<N>, dim3((1u << log2h) / FIRE_SLOW_ROWS), dim3(256), 0, st, heat, heat_old, log2w, log2h,
-			attenuation_i, p);
-	else if((reinterpret_cast<uintptr_t>(heat) | reinterpret_cast<uintptr_t>(heat_old)) % 4 == 0)
-		hipLaunchKernelGGL((k_fire_step_fast<N, true>), dim3(blocks), dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
+		hipLaunchKernelGGL(k_fire_step_slow<N>, grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
+	else if(fire_aligned(heat, heat_old))
+		hipLaunchKernelGGL((k_fire_step_fast<N, true>), grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
 	else
-		hipLaunchKernelGGL((k_fire_step_fast<N, false>), dim3(blocks), dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
+		hipLaunchKernelGGL((k_fire_step_fast<N, false>), grid, dim3(256), 0, st, heat, heat_old, log2w, log2h, attenuation_i, p);
 }
 
 void launch_fire_step(hipStream_t st, const uint8_t* heat, uint8_t* heat_old, uint32_t log2w, uint32_t log2h, uint32_t attenuation_i,
 	bool slow, const sw_heat_point* points, uint32_t num_points, const sw_heat_point* points_dev)
 {
-	// the smaller argument block where it holds the points: the runtime copies the whole block per launch
-	if(num_points <= FIRE_ARG_POINTS_SMALL)
+	// the smallest argument block that holds the points: the runtime copies the whole block per launch
+	if(num_points == 0)
+		launch_fire_update(st, heat, heat_old, log2w, log2h, attenuation_i, slow);
+	else if(num_points <= FIRE_ARG_POINTS_SMALL)
 		launch_fire_step_n<FIRE_ARG_POINTS_SMALL>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, points, num_points);
 	else if(num_points <= FIRE_ARG_POINTS)
 		launch_fire_step_n<FIRE_ARG_POINTS>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, points, num_points);
 	else
 	{
-		launch_fire_step_n<FIRE_ARG_POINTS_SMALL>(st, heat, heat_old, log2w, log2h, attenuation_i, slow, nullptr, 0);
+		launch_fire_update(st, heat, heat_old, log2w, log2h, attenuation_i, slow);
 		hipLaunchKernelGGL(k_fire_points, dim3(1), dim3(64), 0, st, heat_old, points_dev, num_points, log2w, log2h);
 	}
 }

@@ -51,3 +51,27 @@ def test_fire_step_unaligned_buffers(gpu_ctx, shift):
         dst.free()
     assert np.array_equal(out[shift[1]:shift[1] + n], oracle.fire_step(heat, lw, lh, 0.97, False, p))
     assert np.all(out[:shift[1]] == 7) and np.all(out[shift[1] + n:] == 7)
+
+
+@pytest.mark.parametrize("slow", [False, True])
+@pytest.mark.parametrize("log2", [(4, 4), (5, 6), (9, 5)])
+@pytest.mark.parametrize("shift", [(0, 0), (0, 1), (3, 0)])
+def test_fire_update_alone(gpu_ctx, slow, log2, shift):
+    """A step without points, both alignments: maps of less than a block and of several, rows of one and of two passes."""
+    lw, lh = log2
+    n = 1 << (lw + lh)
+    heat = np.random.default_rng([lw, lh, slow, *shift]).integers(0, 256, n).astype(np.uint8)
+    src = gpu_ctx.to_device(np.concatenate([np.zeros(shift[0], np.uint8), heat]))
+    dst = gpu_ctx.to_device(np.full(n + 8, 7, np.uint8))
+    try:
+        print(f"fire step of {1 << lw} x {1 << lh} without points slow={slow} at byte offsets {shift}", flush=True)
+        gpu_ctx.check(gpu_ctx.lib.sw_fire_step(gpu_ctx.h, C.c_void_p(src.ptr.value + shift[0]), C.c_void_p(dst.ptr.value + shift[1]),
+                                               lw, lh, 0.97, int(slow), None, 0), "sw_fire_step")
+        gpu_ctx.check(gpu_ctx.lib.sw_sync(gpu_ctx.h), "sw_sync")
+        out = dst.read(np.uint8, n + 8)
+    finally:
+        src.free()
+        dst.free()
+    ref = oracle.fire_step(heat, lw, lh, 0.97, slow, np.zeros(0, A.HEAT_POINT_DTYPE))
+    assert np.array_equal(out[shift[1]:shift[1] + n], ref)
+    assert np.all(out[:shift[1]] == 7) and np.all(out[shift[1] + n:] == 7)
